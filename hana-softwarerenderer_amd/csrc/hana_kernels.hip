@@ -65,6 +65,7 @@ struct TriS {
     float uz;            // cross product z (constant over the triangle)
     float z0, z1, z2;    // screen depths
     int x0, x1, y0, y1;  // pixel loop bounds (inclusive)
+    int tx0, ty0;        // first column and row of the triangle's tiles
 };
 
 // Returns false for triangles that can produce no fragment: back-facing
@@ -104,6 +105,34 @@ __device__ __forceinline__ bool tri_setup(float4 a, float4 b, float4 c, int W, i
     if (t.x0 < 0 || t.y0 < 0) return false;
     t.x1 = (mxx >= 0.f) ? (int)floorf(mxx) : -1;
     t.y1 = (mxy >= 0.f) ? (int)floorf(mxy) : -1;
+    // The scan's first column (row) lies left of (above) the whole triangle
+    // unless a corner is exactly on it.  It is dropped where the rounding of
+    // the coverage test cannot reach that far: with M the largest edge
+    // component, u = 2^-24 and D the exact cross product of the rounded edges,
+    //  - P - A = b (s0y, s1y) + c (s0x, s1x) with b = Uy / D, c = Ux / D, and
+    //    |ux - Ux|, |uy - Uy| <= 4 u 2M (2M + 1): P is within 2M + 1 of A;
+    //  - |u.z - D| <= 2.1 u M^2 + u |u.z|;
+    //  - a covered P has uy / u.z >= 0, ux / u.z >= 0 and (ux + uy) / u.z <=
+    //    1 + u, so the negative parts of its exact weights sum to at most
+    //    N = u (145 M^2 + 64 M) / |u.z|, and P.x >= min x - u M - 2M N.
+    // So a column more than 2^-24 (300 M^3 + 128 M^2) / |u.z| left of the
+    // corners holds no covered pixel; the test below asks for 2^-15 (M^3 +
+    // M^2) / |u.z| (a triangle of 2 px: 2^-13 px).  Where u.z is so small that
+    // its sign is in doubt, that is more than a pixel.  Infinite and NaN
+    // operands keep the column.  A triangle of e x e px then scans about e^2
+    // pixels instead of (e + 1)^2, and one between two columns none: the
+    // shadow and main rasters of 20 M micro-triangles at 3840x2160 went from
+    // 1495 and 756 us to 948 and 555, those of a 1.3 M-triangle 1920x1080
+    // frame from 60 and 46 us to 50 and 40.  (Testing the coverage of the
+    // triangles with at most 1, 2 or 3 candidates left in set-up and dropping
+    // the uncovered ones as well took as much time there as it saved here.)
+    float M = fmaxf(fmaxf(fabsf(t.s0x), fabsf(t.s0y)), fmaxf(fabsf(t.s1x), fabsf(t.s1y)));
+    float reach = 0x1p-15f * (M * M) * (M + 1.0f), auz = fabsf(t.uz);
+    // binning keeps the reference's scan (workspaces are sized by its pairs)
+    t.tx0 = t.x0;
+    t.ty0 = t.y0;
+    if ((mnx - (float)t.x0) * auz > reach) t.x0++;
+    if ((mny - (float)t.y0) * auz > reach) t.y0++;
     return t.x1 >= t.x0 && t.y1 >= t.y0;
 }
 
@@ -449,8 +478,8 @@ __device__ __forceinline__ void count_tiles(const PassDesc& P, const Workspace& 
                                             uint32_t entry, uint32_t slot, uint32_t local, const SegTables* L) {
     int tx0 = 0, ty0 = 0, tx1 = 0, ty1 = 0, nx = 0, n = 0;
     if (ok) {
-        tx0 = t.x0 >> TS;
-        ty0 = t.y0 >> TS;
+        tx0 = t.tx0 >> TS;
+        ty0 = t.ty0 >> TS;
         tx1 = t.x1 >> TS;
         ty1 = t.y1 >> TS;
         nx = tx1 - tx0 + 1;
