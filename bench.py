@@ -656,8 +656,8 @@ def stage_of_kernel(name):
     m = re.match(r"k_raster<\d+, (\d)(, \d+)?>", base)
     if m:
         return "raster_g" + m.group(1)
-    for k, st in (("k_vertex", "vertex"), ("k_setup", "setup"), ("k_clip", "clip"), ("k_scan", "scan"),
-                  ("k_bin", "bin"), ("k_fill32", "fill"), ("k_present", "present")):
+    for k, st in (("k_vertex", "vertex"), ("k_setup", "setup"), ("k_front", "setup"), ("k_clip", "clip"),
+                  ("k_fill32", "fill"), ("k_present", "present")):
         if base.startswith(k):
             return st
     return base

@@ -29,6 +29,7 @@ struct hana_target {
     bool pending_clear = false;
     uint32_t clear_rgba = 0;
     float clear_depth = 0;
+    int slot = -1;                // draw slot of the last call that drew into or sampled it
 };
 
 namespace hana {
@@ -65,10 +66,17 @@ struct Arena {
     // tables: the pass descriptors, then (at Plan::uni_off) their uniforms,
     // then (at Plan::tp_off) the raster's pass lookup, uploaded by one copy
     // per call
-    DevBuf tables, vr, vs, code, pof, tile_count, tile_offset, tile_cursor, bins, tris, seg_count, scan_part;
-    DevBuf seg_tiles, seg_wide, seg_info, qstate;
-    DevBuf pool_vr, pool_vs, pool_face, pool_pass, pool_n, clip_queue, status, stats;
-    uint32_t bin_cap = 0, poly_cap = 0, clipq_cap = 0, tris_cap = 0;
+    DevBuf tables, vr, vs, code, pof, bins, chunks, over, wide;
+    DevBuf pool_vr, pool_vs, pool_face, clip_queue, status, stats;
+    // two sets of a sequence's counters (Workspace::seq): consecutive calls
+    // alternate, each zeroing the set of the call before, so that no launch
+    // has to zero them first; counters_used: words of a set not yet zeroed
+    DevBuf counters[2];
+    size_t counters_used[2] = {0, 0};
+    int counters_next = 0;
+    uint32_t bin_cap = 0, poly_cap = 0, clipq_cap = 0;
+    uint64_t chunk_slots = 0;   // descriptors the chunks buffer holds
+    uint32_t over_cap = 0, wide_cap = WIDE_MAX;
 };
 
 struct Plan {
@@ -92,6 +100,8 @@ struct Plan {
     int tile_shift = TILE_SHIFT_DEFAULT;
     int raster_waves = 4;
     int raster_wgs = 0;       // workgroups of the persistent raster (0: one per tile and group)
+    bool front = false;       // geometry in one launch (k_front)
+    bool args = false;        // ... which brings the tables as arguments (no upload, no pass lookup)
     uint32_t q_g0 = 0, q_dep_from = 0;
     Workspace ws{};
 };
@@ -126,6 +136,17 @@ constexpr size_t kMaxLoggedCalls = 1024;
 constexpr int kDrawSlots = HANA_DRAW_SLOTS;
 // launch sequences of at least this many faces use two of the slots
 constexpr size_t kLargeSequenceFaces = size_t(1) << 19;
+// launch sequences of at most this many faces run their geometry in one launch
+#ifndef HANA_FRONT_FACES
+#define HANA_FRONT_FACES (1 << 18)
+#endif
+constexpr size_t kFrontFaces = HANA_FRONT_FACES;
+// sequences of at most this many faces draw on the slot that last drew into
+// their target
+#ifndef HANA_STAY_FACES
+#define HANA_STAY_FACES (1 << 15)
+#endif
+constexpr size_t kStayFaces = HANA_STAY_FACES;
 // a draw waits for another slot once that slot has more targets pending for
 // it than this, conflicting or not, which bounds the bookkeeping
 constexpr size_t kMaxPendingTargets = 1024;

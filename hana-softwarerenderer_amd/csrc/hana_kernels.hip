@@ -7,14 +7,12 @@
 //              (is_vertex_visible and the 7 plane tests), perspective divide
 //              and 1/w                                (SR/IShader.cpp, SR/graphics.cpp:29-49, 132-134, 316-337)
 //   k_setup    FPT faces per lane: back-face cull, viewport, bbox, degenerate
-//              test of trivially accepted faces; counts their (triangle,
-//              tile) pairs and lists them for binning; drops faces that the
-//              first plane they cross removes whole; queues the rest for
+//              test of trivially accepted faces; bins them; drops faces that
+//              the first plane they cross removes whole; queues the rest for
 //              clipping
-//   k_clip     clips the queued faces (SR/graphics.cpp:136-161) into polygons,
-//              counts and lists their fan triangles
-//   k_scan_*   exclusive scan of the per-tile counts (reduce, then apply)
-//   k_bin      scatters every listed triangle into its tiles' bins
+//   k_clip     clips the queued faces (SR/graphics.cpp:136-161) into polygons
+//              and bins their fan triangles
+//   k_front    the three of them in one launch, for smaller sequences
 //   k_raster   one workgroup per 16x16 tile: exact per-pixel coverage and
 //              depth (SR/graphics.cpp:222-233, 349-359) resolved in LDS with
 //              64-bit (depth, submission order) keys, then one fragment
@@ -65,82 +63,140 @@ struct TriS {
     float uz;            // cross product z (constant over the triangle)
     float z0, z1, z2;    // screen depths
     int x0, x1, y0, y1;  // pixel loop bounds (inclusive)
-    int tx0, ty0;        // first column and row of the triangle's tiles
+    bool fast;           // cover_is_fast
 };
 
-// Returns false for triangles that can produce no fragment: back-facing
-// (is_back_facing, SR/graphics.cpp:172-180), degenerate (|u.z| <= 1e-2, every
-// barycentric then (-1,1,1), SR/graphics.cpp:230-232) or with an empty scan.
-__device__ __forceinline__ bool tri_setup(float4 a, float4 b, float4 c, int W, int H, TriS& t) {
-    float signed_area = a.x * b.y - a.y * b.x + b.x * c.y - b.y * c.x + c.x * a.y - c.y * a.x;
-    if (signed_area <= 0) return false;
+// The screen corners, edges and depths of a triangle (SR/graphics.cpp:316-337).
+struct Screen {
+    float x0, y0, x1, y1, x2, y2;
+};
+__device__ __forceinline__ Screen tri_edges(float4 a, float4 b, float4 c, int W, int H, TriS& t) {
     float fw = (float)W, fh = (float)H;
-    float sx0 = (a.x + 1) * 0.5f * fw, sy0 = (a.y + 1) * 0.5f * fh;
-    float sx1 = (b.x + 1) * 0.5f * fw, sy1 = (b.y + 1) * 0.5f * fh;
-    float sx2 = (c.x + 1) * 0.5f * fw, sy2 = (c.y + 1) * 0.5f * fh;
+    Screen s;
+    s.x0 = (a.x + 1) * 0.5f * fw; s.y0 = (a.y + 1) * 0.5f * fh;
+    s.x1 = (b.x + 1) * 0.5f * fw; s.y1 = (b.y + 1) * 0.5f * fh;
+    s.x2 = (c.x + 1) * 0.5f * fw; s.y2 = (c.y + 1) * 0.5f * fh;
     t.z0 = (a.z + 1) * 0.5f;
     t.z1 = (b.z + 1) * 0.5f;
     t.z2 = (c.z + 1) * 0.5f;
-    t.ax = sx0;
-    t.ay = sy0;
-    t.s0x = sx2 - sx0;
-    t.s0y = sx1 - sx0;
-    t.s1x = sy2 - sy0;
-    t.s1y = sy1 - sy0;
+    t.ax = s.x0;
+    t.ay = s.y0;
+    t.s0x = s.x2 - s.x0;
+    t.s0y = s.x1 - s.x0;
+    t.s1x = s.y2 - s.y0;
+    t.s1y = s.y1 - s.y0;
     t.uz = t.s0x * t.s1y - t.s0y * t.s1x;
-    // (double)|u.z| > 1e-2 is the same test as |u.z| > 0.01f on floats
-    if (!(fabsf(t.uz) > 0.01f)) return false;
-    float mnx = FLT_MAX, mny = FLT_MAX, mxx = -FLT_MAX, mxy = -FLT_MAX;
-    float clx = (float)(W - 1), cly = (float)(H - 1);
-    mnx = smax(0.f, smin(mnx, sx0)); mxx = smin(clx, smax(mxx, sx0));
-    mny = smax(0.f, smin(mny, sy0)); mxy = smin(cly, smax(mxy, sy0));
-    mnx = smax(0.f, smin(mnx, sx1)); mxx = smin(clx, smax(mxx, sx1));
-    mny = smax(0.f, smin(mny, sy1)); mxy = smin(cly, smax(mxy, sy1));
-    mnx = smax(0.f, smin(mnx, sx2)); mxx = smin(clx, smax(mxx, sx2));
-    mny = smax(0.f, smin(mny, sy2)); mxy = smin(cly, smax(mxy, sy2));
-    // for (P.x = bboxmin.x; P.x <= bboxmax.x; P.x++): start truncates, the
-    // bound compares the int as a float
-    t.x0 = f2i(mnx);
-    t.y0 = f2i(mny);
-    if (t.x0 < 0 || t.y0 < 0) return false;
-    t.x1 = (mxx >= 0.f) ? (int)floorf(mxx) : -1;
-    t.y1 = (mxy >= 0.f) ? (int)floorf(mxy) : -1;
-    // The scan's first column (row) lies left of (above) the whole triangle
-    // unless a corner is exactly on it.  It is dropped where the rounding of
-    // the coverage test cannot reach that far: with M the largest edge
-    // component, u = 2^-24 and D the exact cross product of the rounded edges,
-    //  - P - A = b (s0y, s1y) + c (s0x, s1x) with b = Uy / D, c = Ux / D, and
-    //    |ux - Ux|, |uy - Uy| <= 4 u 2M (2M + 1): P is within 2M + 1 of A;
-    //  - |u.z - D| <= 2.1 u M^2 + u |u.z|;
-    //  - a covered P has uy / u.z >= 0, ux / u.z >= 0 and (ux + uy) / u.z <=
-    //    1 + u, so the negative parts of its exact weights sum to at most
-    //    N = u (145 M^2 + 64 M) / |u.z|, and P.x >= min x - u M - 2M N.
-    // So a column more than 2^-24 (300 M^3 + 128 M^2) / |u.z| left of the
-    // corners holds no covered pixel; the test below asks for 2^-15 (M^3 +
-    // M^2) / |u.z| (a triangle of 2 px: 2^-13 px).  Where u.z is so small that
-    // its sign is in doubt, that is more than a pixel.  Infinite and NaN
-    // operands keep the column.  A triangle of e x e px then scans about e^2
-    // pixels instead of (e + 1)^2, and one between two columns none: the
-    // shadow and main rasters of 20 M micro-triangles at 3840x2160 went from
-    // 1495 and 756 us to 948 and 555, those of a 1.3 M-triangle 1920x1080
-    // frame from 60 and 46 us to 50 and 40.  (Testing the coverage of the
-    // triangles with at most 1, 2 or 3 candidates left in set-up and dropping
-    // the uncovered ones as well took as much time there as it saved here.)
+    return s;
+}
+
+// The reference's pixel loop bounds (SR/graphics.cpp:338-347) of a triangle
+// whose u.z is not NaN, so that no corner is: its running minima and maxima,
+// clamped at every step, are then the clamped minimum and maximum of the
+// corners.  for (P.x = bboxmin.x; P.x <= bboxmax.x; P.x++): the start
+// truncates, the bound compares the int as a float.  A start beyond the
+// target (which may convert to anything over 2^30) exceeds the bound.
+struct Bounds {
+    float mnx, mny;
+};
+__device__ __forceinline__ Bounds tri_bounds(const Screen& s, int W, int H, TriS& t) {
+    Bounds b;
+    b.mnx = fmaxf(fminf(fminf(s.x0, s.x1), s.x2), 0.f);
+    b.mny = fmaxf(fminf(fminf(s.y0, s.y1), s.y2), 0.f);
+    float mxx = fminf(fmaxf(fmaxf(s.x0, s.x1), s.x2), (float)(W - 1));
+    float mxy = fminf(fmaxf(fmaxf(s.y0, s.y1), s.y2), (float)(H - 1));
+    t.x0 = (int)fminf(b.mnx, 0x1p30f);
+    t.y0 = (int)fminf(b.mny, 0x1p30f);
+    t.x1 = (int)floorf(fmaxf(mxx, -1.f));
+    t.y1 = (int)floorf(fmaxf(mxy, -1.f));
+    return b;
+}
+
+// What set-up found out about a triangle, for the rasters (in the bits of its
+// bin entry over the face index): FACE_FAST, its coverage takes the shared
+// reciprocal (cover_is_fast); FACE_SKIP_X and FACE_SKIP_Y, no pixel of the
+// first column or row of its scan is covered.
+constexpr uint32_t FACE_SKIP_X = 1u << 30, FACE_SKIP_Y = 1u << 29, FACE_FAST = 1u << 28;
+constexpr uint32_t FACE_MASK = FACE_FAST - 1u;
+
+// The first column (row) of the scan lies left of (above) the whole triangle
+// unless a corner is exactly on it.  It is dropped where the rounding of the
+// coverage test cannot reach that far: with M the largest edge component, u =
+// 2^-24 and D the exact cross product of the rounded edges,
+//  - P - A = b (s0y, s1y) + c (s0x, s1x) with b = Uy / D, c = Ux / D, and
+//    |ux - Ux|, |uy - Uy| <= 4 u 2M (2M + 1): P is within 2M + 1 of A;
+//  - |u.z - D| <= 2.1 u M^2 + u |u.z|;
+//  - a covered P has uy / u.z >= 0, ux / u.z >= 0 and (ux + uy) / u.z <= 1 + u,
+//    so the negative parts of its exact weights sum to at most N = u (145 M^2
+//    + 64 M) / |u.z|, and P.x >= min x - u M - 2M N.
+// So a column more than 2^-24 (300 M^3 + 128 M^2) / |u.z| left of the corners
+// holds no covered pixel; the test below asks for 2^-15 (M^3 + M^2) / |u.z| (a
+// triangle of 2 px: 2^-13 px).  Where u.z is so small that its sign is in
+// doubt, that is more than a pixel.  Infinite and NaN operands keep the column.
+// A triangle of e x e px then scans about e^2 pixels instead of (e + 1)^2, and
+// one between two columns none: the shadow and main rasters of 20 M
+// micro-triangles at 3840x2160 went from 1495 and 756 us to 948 and 555, those
+// of a 1.3 M-triangle 1920x1080 frame from 60 and 46 us to 50 and 40.
+// (Testing the coverage of the triangles with at most 1, 2 or 3 candidates
+// left in set-up and dropping the uncovered ones as well took as much time
+// there as it saved here.)
+__device__ __forceinline__ uint32_t tri_skips(const TriS& t, const Bounds& b) {
     float M = fmaxf(fmaxf(fabsf(t.s0x), fabsf(t.s0y)), fmaxf(fabsf(t.s1x), fabsf(t.s1y)));
     float reach = 0x1p-15f * (M * M) * (M + 1.0f), auz = fabsf(t.uz);
-    // binning keeps the reference's scan (workspaces are sized by its pairs)
-    t.tx0 = t.x0;
-    t.ty0 = t.y0;
-    if ((mnx - (float)t.x0) * auz > reach) t.x0++;
-    if ((mny - (float)t.y0) * auz > reach) t.y0++;
-    return t.x1 >= t.x0 && t.y1 >= t.y0;
+    return ((b.mnx - (float)t.x0) * auz > reach ? FACE_SKIP_X : 0u) |
+           ((b.mny - (float)t.y0) * auz > reach ? FACE_SKIP_Y : 0u);
+}
+
+// Whether the three divisions of a triangle's candidates by u.z may share a
+// refined reciprocal (tri_cover): every screen coordinate and edge within
+// 2^22, and every input zero or at least 2^-8 in magnitude.  Then a nonzero
+// numerator is at least 2^-62: ax and ay are multiples of 2^-31, so s0z and
+// s1z are (their rounding keeps that); a product of a nonzero edge component
+// and a nonzero s0z or s1z is at least 2^-39, so a multiple of 2^-62; their
+// differences and the sum stay multiples of 2^-62.
+// v is zero or at least 2^-8 in magnitude when (bits(v) << 1) - 1 >=
+// (bits(2^-8) << 1) - 1 (zero wraps to the maximum).
+__device__ __forceinline__ bool cover_is_fast(const TriS& t) {
+    float ext = fmaxf(fmaxf(fmaxf(fabsf(t.ax), fabsf(t.ay)), fmaxf(fabsf(t.s0x), fabsf(t.s0y))),
+                      fmaxf(fabsf(t.s1x), fabsf(t.s1y)));
+    const uint32_t kMin8 = ((uint32_t)(127 - 8) << 24) - 1u;
+    uint32_t mt = min(min(min((__float_as_uint(t.ax) << 1) - 1u, (__float_as_uint(t.ay) << 1) - 1u),
+                          min((__float_as_uint(t.s0x) << 1) - 1u, (__float_as_uint(t.s0y) << 1) - 1u)),
+                      min((__float_as_uint(t.s1x) << 1) - 1u, (__float_as_uint(t.s1y) << 1) - 1u));
+    return ext <= 0x1p22f && mt >= kMin8;
+}
+
+// Set-up of a triangle for binning.  Returns false for those that can produce
+// no fragment: back-facing (is_back_facing, SR/graphics.cpp:172-180),
+// degenerate (|u.z| <= 1e-2, every barycentric then (-1,1,1),
+// SR/graphics.cpp:230-232) or with an empty scan.  `flags` takes its FACE_*
+// bits; the bounds stay the reference's scan, which binning goes by.
+__device__ __forceinline__ bool tri_setup(float4 a, float4 b, float4 c, int W, int H, TriS& t, uint32_t& flags) {
+    float signed_area = a.x * b.y - a.y * b.x + b.x * c.y - b.y * c.x + c.x * a.y - c.y * a.x;
+    if (signed_area <= 0) return false;
+    Screen s = tri_edges(a, b, c, W, H, t);
+    // (double)|u.z| > 1e-2 is the same test as |u.z| > 0.01f on floats
+    if (!(fabsf(t.uz) > 0.01f)) return false;
+    Bounds bd = tri_bounds(s, W, H, t);
+    flags = tri_skips(t, bd) | (cover_is_fast(t) ? FACE_FAST : 0u);
+    return t.x1 >= t.x0 + (flags & FACE_SKIP_X ? 1 : 0) && t.y1 >= t.y0 + (flags & FACE_SKIP_Y ? 1 : 0);
+}
+
+// The same triangle in the raster, which only gets those that passed: the
+// scan of the pixels that may be covered.
+__device__ __forceinline__ void tri_raster(float4 a, float4 b, float4 c, int W, int H, TriS& t, uint32_t flags) {
+    asm("" : "+s"(W), "+s"(H));   // uniform; as fresh(): their conversions else stay in registers, or spill
+    Screen s = tri_edges(a, b, c, W, H, t);
+    tri_bounds(s, W, H, t);
+    if (flags & FACE_SKIP_X) t.x0++;
+    if (flags & FACE_SKIP_Y) t.y0++;
+    t.fast = (flags & FACE_FAST) != 0u;
 }
 
 // n / u.z as the hardware's IEEE division sequence computes it when its
 // scaling steps are no-ops, from the reciprocal r = cover_recip(u.z) that
 // sequence refines (the same operations in the same order, so the same bits):
 // q = n r; e = fma(-u.z, q, n); q = fma(e, r, q); e = fma(-u.z, q, n);
-// q = fma(e, r, q).  See tri_cover_fast for when that holds.
+// q = fma(e, r, q).  See tri_cover for when that holds.
 __device__ __forceinline__ float cover_recip(float uz) {
     float r = __builtin_amdgcn_rcpf(uz);
     float e = fmaf(-uz, r, 1.0f);
@@ -165,33 +221,16 @@ __device__ __forceinline__ float cover_quot(float n, float uz, float r) {
 // so for every numerator with |n| >= 2^-80 neither happens and cover_quot
 // gives the division's bits.  A zero numerator gives a zero of either sign,
 // which changes neither the coverage test nor the depth (summed from +0).
-// Other candidates divide.
-__device__ __forceinline__ bool tri_cover_fast(const TriS& t, int px, int py, float& wx, float& wy, float& wz, float& z) {
+// Triangles for which that is not known (cover_is_fast: rare) divide.
+__device__ __forceinline__ bool tri_cover(const TriS& t, int px, int py, float& wx, float& wy, float& wz, float& z) {
     float Px = (float)px, Py = (float)py;
     float s0z = t.ax - Px;
     float s1z = t.ay - Py;
     float ux = t.s0y * s1z - s0z * t.s1y;
     float uy = s0z * t.s1x - t.s0x * s1z;
     float sum = ux + uy;
-    float ext = fmaxf(fmaxf(fmaxf(fabsf(t.ax), fabsf(t.ay)), fmaxf(fabsf(t.s0x), fabsf(t.s0y))),
-                      fmaxf(fabsf(t.s1x), fabsf(t.s1y)));
     float r = cover_recip(t.uz);
-    // The shortcut needs every nonzero numerator to be at least 2^-80 in
-    // magnitude.  When every input of the triangle is zero or at least 2^-8 in
-    // magnitude (and at most 2^22), a nonzero numerator is at least 2^-62:
-    // ax and ay are multiples of 2^-31, so s0z and s1z are (their rounding
-    // keeps that); a product of a nonzero edge component and a nonzero s0z or
-    // s1z is at least 2^-39, so a multiple of 2^-62; their differences and
-    // the sum stay multiples of 2^-62.  Such a triangle needs no check per
-    // candidate; the others (an input under 2^-8 but not zero: rare) divide.
-    // v is zero or at least 2^-8 in magnitude when (bits(v) << 1) - 1 >=
-    // (bits(2^-8) << 1) - 1 (zero wraps to the maximum).
-    const uint32_t kMin8 = ((uint32_t)(127 - 8) << 24) - 1u;
-    uint32_t mt = min(min(min((__float_as_uint(t.ax) << 1) - 1u, (__float_as_uint(t.ay) << 1) - 1u),
-                          min((__float_as_uint(t.s0x) << 1) - 1u, (__float_as_uint(t.s0y) << 1) - 1u)),
-                      min((__float_as_uint(t.s1x) << 1) - 1u, (__float_as_uint(t.s1y) << 1) - 1u));
-    bool fast = ext <= 0x1p22f && mt >= kMin8;
-    if (fast) {
+    if (t.fast) {
         wx = 1.f - cover_quot(sum, t.uz, r);
         wy = cover_quot(uy, t.uz, r);
         wz = cover_quot(ux, t.uz, r);
@@ -225,47 +264,84 @@ __device__ __forceinline__ void stat_add(const PassDesc& P, int which, uint64_t 
 
 // Raises a flag for this sequence and in the sticky word the host reads.
 __device__ __forceinline__ void raise_flag(const Workspace& ws, uint32_t f) {
-    atomicOr(&ws.status[STATUS_SEQ_FLAGS], f);
+    atomicOr(&ws.seq[SEQ_FLAGS], f);
     atomicOr(&ws.status[STATUS_FLAGS], f);
 }
 
-// clip planes in clip_triangle's order (SR/graphics.cpp:136-161) and their
-// inside tests (is_inside_plane, SR/graphics.cpp:29-49)
-enum { PL_W, PL_PX, PL_NX, PL_PY, PL_NY, PL_PZ, PL_NZ };
+// Lanes of the mask below this one.
+__device__ __forceinline__ uint32_t mask_rank(uint64_t m) {
+    return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+}
 
+// Inclusive prefix sum over the wave: within each row of 16 lanes, then the
+// rows' last lanes into the rows after them (data-parallel primitives: no LDS
+// access, and no lane masks for the compiler to keep).
+__device__ __forceinline__ uint32_t wave_scan(uint32_t v) {
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xF, 0xF, false);   // row_shr:1
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xF, 0xF, false);   // row_shr:2
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xF, 0xF, false);   // row_shr:4
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xF, 0xF, false);   // row_shr:8
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xA, 0xF, false);   // row_bcast:15 into rows 1, 3
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xC, 0xF, false);   // row_bcast:31 into rows 2, 3
+    return v;
+}
+
+// Adds to a 64-bit counter of the sequence; returns its value before.
+__device__ __forceinline__ uint64_t seq_add64(const Workspace& ws, int which, uint64_t v) {
+    return (uint64_t)atomicAdd((unsigned long long*)(ws.seq + which), (unsigned long long)v);
+}
+
+// Zeroes the counters the launch is given to zero (Workspace::zero).
+__device__ __forceinline__ void zero_counters(const Workspace& ws) {
+    uint32_t gsize = gridDim.x * blockDim.x;
+    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < ws.zero_n; i += gsize) gst(ws.zero + i, 0u);
+}
+
+// clip planes in clip_triangle's order (SR/graphics.cpp:136-161): w >= 1e-5,
+// then x, y, z <= +w and >= -w
+constexpr int CLIP_PLANES = 7;
+
+// is_inside_plane (SR/graphics.cpp:29-49)
 __device__ __forceinline__ bool inside_plane(const float* c, int plane) {
-    switch (plane) {
-    case PL_W: return c[3] >= 1e-5f;
-    case PL_PX: return c[0] <= +c[3];
-    case PL_NX: return c[0] >= -c[3];
-    case PL_PY: return c[1] <= +c[3];
-    case PL_NY: return c[1] >= -c[3];
-    case PL_PZ: return c[2] <= +c[3];
-    default: return c[2] >= -c[3];
-    }
+    if (plane == 0) return c[3] >= 1e-5f;
+    float v = c[(plane - 1) >> 1];
+    return (plane & 1) ? v <= +c[3] : v >= -c[3];
 }
 
 // ---------------------------------------------------------------------------
 // k_vertex
 // ---------------------------------------------------------------------------
 
-__global__ __launch_bounds__(BLOCK) void k_vertex(const PassDesc* __restrict__ passes, int npasses, Workspace ws) {
-    int gtid = blockIdx.x * BLOCK + threadIdx.x;
-    int gsize = gridDim.x * BLOCK;
-    for (int i = gtid; i < ws.ntiles; i += gsize) gst(ws.tile_count + i, 0u);
-    if (gtid < STATUS_SEQ_WORDS) gst(ws.status + gtid, 0u);
-    if (gtid < 2) gst(ws.qstate + gtid, 0u);
+// A vertex after its program: outcode, NDC position and 1/w.
+struct PostVertex {
+    uint32_t code;
+    float4 r;
+};
+__device__ __forceinline__ PostVertex post_vertex(const float clip[4]) {
+    PostVertex o;
+    // is_vertex_visible (SR/graphics.cpp:132-134), then the plane tests
+    o.code = (fabsf(clip[0]) <= clip[3] && fabsf(clip[1]) <= clip[3] && fabsf(clip[2]) <= clip[3]) ? CODE_VISIBLE : 0u;
+#pragma unroll
+    for (int pl = 0; pl < CLIP_PLANES; pl++)
+        if (!inside_plane(clip, pl)) o.code |= 1u << pl;
+    // clip_pos / clip_pos[3] and 1 / clip_pos[3] (SR/graphics.cpp:317, 336)
+    o.r.w = 1 / clip[3];
+    o.r.z = clip[2] / clip[3];
+    o.r.y = clip[1] / clip[3];
+    o.r.x = clip[0] / clip[3];
+    return o;
+}
 
-    const PassDesc& P = passes[find_pass<0>(passes, npasses, blockIdx.x)];
-    Uniforms u = uniforms_of(P.u);
-    int base = (blockIdx.x - P.vblock0) * BLOCK * VPT;
+// N vertices per lane of pass P (uniform block u), from vertex `base`: the
+// loads of all N first (coalesced SoA streams), then program and stores.
+template <int N>
+__device__ __forceinline__ void vertex_block(const PassDesc& P, Uniforms u, int base) {
     bool need_n = P.kind != SHADER_SHADOW && P.kind != SHADER_TEXTURE;
     bool need_uv = P.kind != SHADER_SHADOW && P.kind != SHADER_GROUND && P.kind != SHADER_TOON;
-    // all loads of the thread's VPT vertices first (coalesced SoA streams)
-    F3 pos[VPT], nrm[VPT];
-    float tu[VPT], tv[VPT];
+    F3 pos[N], nrm[N];
+    float tu[N], tv[N];
 #pragma unroll
-    for (int k = 0; k < VPT; k++) {
+    for (int k = 0; k < N; k++) {
         int v = base + k * BLOCK + threadIdx.x;
         pos[k] = f3(0.f, 0.f, 0.f);
         nrm[k] = f3(0.f, 0.f, 0.f);
@@ -280,25 +356,14 @@ __global__ __launch_bounds__(BLOCK) void k_vertex(const PassDesc* __restrict__ p
         }
     }
 #pragma unroll
-    for (int k = 0; k < VPT; k++) {
+    for (int k = 0; k < N; k++) {
         int v = base + k * BLOCK + threadIdx.x;
         if (v < P.nverts) {
             float clip[4], vary[8];
             vertex_program(P.kind, u, pos[k], nrm[k], tu[k], tv[k], clip, vary);
-            // is_vertex_visible (SR/graphics.cpp:132-134), then the plane tests
-            uint32_t code =
-                (fabsf(clip[0]) <= clip[3] && fabsf(clip[1]) <= clip[3] && fabsf(clip[2]) <= clip[3]) ? CODE_VISIBLE : 0u;
-#pragma unroll
-            for (int pl = 0; pl < 7; pl++)
-                if (!inside_plane(clip, pl)) code |= 1u << pl;
-            gst(P.code + v, (uint8_t)code);
-            // clip_pos / clip_pos[3] and 1 / clip_pos[3] (SR/graphics.cpp:317, 336)
-            float4 r;
-            r.w = 1 / clip[3];
-            r.z = clip[2] / clip[3];
-            r.y = clip[1] / clip[3];
-            r.x = clip[0] / clip[3];
-            gst4(P.vr + v, r);
+            PostVertex o = post_vertex(clip);
+            gst(P.code + v, (uint8_t)o.code);
+            gst4(P.vr + v, o.r);
             if (P.nvary == 8) {
                 float4* d = reinterpret_cast<float4*>(P.vs + (size_t)v * 8);
                 gst4(d, make_float4(vary[0], vary[1], vary[2], vary[3]));
@@ -312,20 +377,29 @@ __global__ __launch_bounds__(BLOCK) void k_vertex(const PassDesc* __restrict__ p
     }
 }
 
+__global__ __launch_bounds__(BLOCK) void k_vertex(const PassDesc* __restrict__ passes, int npasses, Workspace ws) {
+    zero_counters(ws);
+    const PassDesc& P = passes[find_pass<0>(passes, npasses, blockIdx.x)];
+    vertex_block<VPT>(P, uniforms_of(P.u), (blockIdx.x - P.vblock0) * BLOCK * VPT);
+}
+
 // ---------------------------------------------------------------------------
 // clipping (SR/graphics.cpp:7-161), for faces failing the trivial accept
 // ---------------------------------------------------------------------------
 
+// get_intersect_ratio (SR/graphics.cpp:51-71) of the edge p -> c
 __device__ __forceinline__ float intersect_ratio(const float* p, const float* c, int plane) {
-    switch (plane) {
-    case PL_W: return (p[3] - 1e-5f) / (p[3] - c[3]);
-    case PL_PX: return (p[3] - p[0]) / ((p[3] - p[0]) - (c[3] - c[0]));
-    case PL_NX: return (p[3] + p[0]) / ((p[3] + p[0]) - (c[3] + c[0]));
-    case PL_PY: return (p[3] - p[1]) / ((p[3] - p[1]) - (c[3] - c[1]));
-    case PL_NY: return (p[3] + p[1]) / ((p[3] + p[1]) - (c[3] + c[1]));
-    case PL_PZ: return (p[3] - p[2]) / ((p[3] - p[2]) - (c[3] - c[2]));
-    default: return (p[3] + p[2]) / ((p[3] + p[2]) - (c[3] + c[2]));
+    float num, den;
+    if (plane == 0) {
+        num = p[3] - 1e-5f;
+        den = p[3] - c[3];
+    } else {
+        float pv = p[(plane - 1) >> 1], cv = c[(plane - 1) >> 1];
+        bool pos = plane & 1;
+        num = pos ? p[3] - pv : p[3] + pv;
+        den = num - (pos ? c[3] - cv : c[3] + cv);
     }
+    return num / den;
 }
 
 // Orders the LDS accesses of the lanes of one wave (the wave executes them in
@@ -341,6 +415,10 @@ __device__ __forceinline__ void wave_sync() {
 // (clip position then POLY_VARY varyings per vertex) live in LDS.
 constexpr int CLIP_GROUP = 16;
 constexpr int CLIP_THREADS = 512;
+#ifndef HANA_CLIP_GRID
+#define HANA_CLIP_GRID 2048
+#endif
+constexpr int CLIP_GRID = HANA_CLIP_GRID;
 constexpr int CLIP_FACES = CLIP_THREADS / CLIP_GROUP;   // faces per workgroup and round
 constexpr int CLIP_NF = 4 + POLY_VARY;
 static_assert(POLY_MAX <= CLIP_GROUP, "one lane per polygon vertex");
@@ -359,65 +437,15 @@ __device__ __forceinline__ float4 ndc_of(const float* v) {
 }
 
 // ---------------------------------------------------------------------------
-// binning: count the (triangle, tile) pairs and list the triangles; after the
-// scan, k_bin scatters the listed triangles into the bins
+// binning (Workspace): chunks of a set-up workgroup's pairs, descriptors of
+// single pairs, wide triangles
 // ---------------------------------------------------------------------------
 
-// Reserves one slot in counters[t] for every lane with `want`, with one atomic
-// per distinct t in the wave; returns the lane's slot.  The lanes are grouped
-// by t first, without any memory access; then every group's first lane issues
-// the group's atomic, and the returned bases are awaited once for all groups
-// (awaiting each group's atomic before forming the next group serialises their
-// round trips where a wave's tiles are scattered).  Every active lane of the
-// wave must call it together (the loop is wave-uniform).
-__device__ __forceinline__ uint32_t wave_reserve(uint32_t* counters, int t, bool want) {
-    int lane = __lane_id();
-    bool pending = want;
-    uint64_t mask = __ballot(pending);
-    int leader_of = lane;
-    uint32_t rank = 0, group = 0;
-    while (mask) {
-        int leader = __ffsll((unsigned long long)mask) - 1;
-        int lt = __shfl(t, leader);
-        bool match = pending && t == lt;
-        uint64_t same = __ballot(match);
-        if (match) {
-            leader_of = leader;
-            rank = (uint32_t)__popcll(same & ((1ull << lane) - 1ull));
-            pending = false;
-        }
-        if (lane == leader) group = (uint32_t)__popcll(same);
-        mask &= ~same;
-    }
-    uint32_t base = 0;
-    if (want && leader_of == lane) base = gadd(counters + t, group);
-    base = __shfl(base, leader_of);
-    return base + rank;
-}
-
-// Adds one to counters[t] for every lane with `want`: one atomic per distinct
-// t in the wave, none of them waited for.  Wave-uniform like wave_reserve.
-__device__ __forceinline__ void wave_count(uint32_t* counters, int t, bool want) {
-    bool pending = want;
-    uint64_t mask = __ballot(pending);
-    int lane = __lane_id();
-    while (mask) {
-        int leader = __ffsll((unsigned long long)mask) - 1;
-        int lt = __shfl(t, leader);
-        bool match = pending && t == lt;
-        uint64_t same = __ballot(match);
-        if (lane == leader) gadd(counters + lt, (uint32_t)__popcll(same));
-        if (match) pending = false;
-        mask = __ballot(pending);
-    }
-}
-
 // The tiles of one workgroup's (triangle, tile) pairs in an LDS hash table:
-// open addressing over BIN_HASH slots, a bounded probe; a tile that finds no
-// slot goes through the global cursors instead.
-// k_setup and k_bin size their tables by the sequence: 512 slots when every
-// pass has small triangles (a segment of 1024 faces then touches a few dozen
-// tiles, and a smaller table is quicker to clear and scan), more otherwise.
+// open addressing over 2^BITS slots, a bounded probe; a tile that finds no
+// slot takes a descriptor per pair instead.  512 slots when every pass has
+// small triangles (a segment of 1024 faces then touches a few dozen tiles,
+// and a smaller table is quicker to clear and scan), more otherwise.
 constexpr int BIN_PROBES = 32;
 constexpr uint32_t BIN_EMPTY = 0xFFFFFFFFu;
 
@@ -438,15 +466,6 @@ __device__ __forceinline__ int bin_slot(uint32_t* keys, uint32_t gt, bool insert
     return -1;
 }
 
-// Counts one (triangle, tile) pair in the workgroup's LDS table, or in the
-// global counter when the table has no slot left for the tile.
-template <int BITS>
-__device__ __forceinline__ void lds_count(uint32_t* keys, uint32_t* cnt, uint32_t* global, uint32_t gt) {
-    int sl = bin_slot<BITS>(keys, gt, true);
-    if (sl >= 0) atomicAdd(&cnt[sl], 1u);
-    else gadd(global + gt, 1u);
-}
-
 // A workgroup barrier that orders LDS accesses only: unlike __syncthreads it
 // does not wait for the wave's outstanding global loads first, so loads
 // issued before it stay in flight across it.
@@ -456,65 +475,125 @@ __device__ __forceinline__ void lds_barrier() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-// Triangles over more tiles than this are counted and binned by a whole wave
-// (or workgroup), their tiles spread over the lanes.
-constexpr int WIDE_TILES = 16;
+// Stores descriptor idx of tile gt: past the tile's places, in the list of the
+// sequence; past that it is lost, the sequence rasterises nothing and the host
+// renders it again with more of both.
+__device__ __forceinline__ void put_chunk(const Workspace& ws, uint32_t gt, uint32_t idx, uint2 d) {
+    if (idx < ws.chunk_cap) {
+        gst2(ws.chunks + ((size_t)gt * ws.chunk_cap + idx), d);
+        return;
+    }
+    atomicMax(&ws.seq[SEQ_MAX_CHUNKS], idx + 1u);
+    uint32_t o = atomicAdd(&ws.seq[SEQ_OVER], 1u);
+    if (o < ws.over_cap) ws.over[o] = make_uint4(gt, d.x, d.y, 0u);
+}
 
-// Counts every (triangle, tile) pair of one lane's triangle and writes its
-// record (bin entry, pass, first and last tile) for k_bin to ws.tris[slot];
-// wave-uniform.  With BITS > 0 the pairs of triangles over at most WIDE_TILES
-// tiles go to the workgroup's LDS table (keys, cnt), which the caller adds to
-// the global counts; with BITS == 0 they go to the global counts directly,
-// one atomic per distinct tile of the wave.
-struct SegTables {       // k_setup's LDS tables of one segment
-    uint32_t* keys;
-    uint32_t* cnt;
-    uint16_t* wide;      // segment-local indices of the triangles over more than WIDE_TILES tiles
-    uint32_t* nwide;
+// The tiles of a triangle to be binned: bin entry, first and last tile.
+struct TileSpan {
+    uint32_t entry, t0, t1;   // x | y << 16
+    __device__ __forceinline__ int x0() const { return (int)(t0 & 0xFFFFu); }
+    __device__ __forceinline__ int y0() const { return (int)(t0 >> 16); }
+    __device__ __forceinline__ int nx() const { return (int)(t1 & 0xFFFFu) - x0() + 1; }
+    __device__ __forceinline__ int ny() const { return (int)(t1 >> 16) - y0() + 1; }
+};
+template <int TS>
+__device__ __forceinline__ TileSpan span_of(const TriS& t, uint32_t entry) {
+    TileSpan s;
+    s.entry = entry;
+    s.t0 = (uint32_t)(t.x0 >> TS) | ((uint32_t)(t.y0 >> TS) << 16);
+    s.t1 = (uint32_t)(t.x1 >> TS) | ((uint32_t)(t.y1 >> TS) << 16);
+    return s;
+}
+
+// The first and last tile of a wide triangle in one word, in units of 2^shift
+// tiles that 8 bits hold; a tile's own position in those units.
+__device__ __forceinline__ int wide_shift(const PassDesc& P) {
+    return max(24 - __clz(max(P.tiles_x, P.tiles_y) - 1), 0);
+}
+__device__ __forceinline__ uint32_t wide_box(int shift, int x0, int y0, int x1, int y1) {
+    return (uint32_t)(x0 >> shift) | ((uint32_t)(y0 >> shift) << 8) | ((uint32_t)(x1 >> shift) << 16) |
+           ((uint32_t)(y1 >> shift) << 24);
+}
+
+// Bins the triangles over more than WIDE_TILES tiles (`wide`): into their
+// pass's list while it has room, else by the whole wave into each of their
+// tiles (unless the pairs pass the bins' capacity anyway).  Every active lane
+// of the wave must call it together.
+__device__ __forceinline__ void bin_wide(const PassDesc& P, const Workspace& ws, bool wide, const TileSpan& s) {
+    if (!__ballot(wide)) return;
+    uint32_t n = 0;
+    bool each = false;
+    if (wide) {
+        n = (uint32_t)s.nx() * (uint32_t)s.ny();
+        uint32_t idx = gadd(ws.wide_count + P.index, 1u);
+        if (idx < ws.wide_cap) {
+            gst2(ws.wide + (size_t)P.index * ws.wide_cap + idx,
+                 make_uint2(wide_box(wide_shift(P), s.x0(), s.y0(), s.x0() + s.nx() - 1, s.y0() + s.ny() - 1), s.entry));
+            seq_add64(ws, SEQ_WIDE_PAIRS, n);
+        } else {
+            each = ws.seg_region + seq_add64(ws, SEQ_PAIRS, n) + n <= ws.bin_cap;
+        }
+    }
+    uint64_t mask = __ballot(each);
+    int tile0 = P.tile0, tiles_x = P.tiles_x;
+    while (mask) {
+        int src = __ffsll((unsigned long long)mask) - 1;
+        mask &= mask - 1;
+        int wn = __shfl((int)n, src), wnx = __shfl(s.nx(), src), wx0 = __shfl(s.x0(), src), wy0 = __shfl(s.y0(), src);
+        int wt0 = __shfl(tile0, src), wtx = __shfl(tiles_x, src);
+        uint32_t we = __shfl(s.entry, src);
+        for (int k = __lane_id(); k < wn; k += 64) {
+            uint32_t gt = (uint32_t)(wt0 + (wy0 + k / wnx) * wtx + wx0 + k % wnx);
+            put_chunk(ws, gt, gadd(ws.tile_chunks + gt, 1u), make_uint2(we, CHUNK_INLINE));
+        }
+    }
+}
+
+// k / w for 0 <= k < 1024 and 1 <= w <= 32 (a tile's pixels and row widths)
+// as (k * magic) >> 16 with magic = ceil(2^16 / w): the excess
+// k * (magic - 2^16/w) / 2^16 stays below 1024 / 2^16 = 1/64, less than the
+// gap 1/w >= 1/32 between k/w and the next integer.
+__device__ __forceinline__ uint32_t tile_div_magic(int w) { return (65536u + (uint32_t)w - 1u) / (uint32_t)w; }
+__device__ __forceinline__ int tile_div(int k, uint32_t magic) { return (int)(((uint32_t)k * magic) >> 16); }
+
+// The LDS of one workgroup's binning: the tile table, and the list of the
+// triangles to bin (bin entry, first and last tile).  Set-up lists a
+// workgroup's triangles, about half of its faces, before it bins them: the
+// lanes of the counting and placing loops are then full, and their code is
+// there once and not per face of a lane.
+template <int BITS, int THREADS, int CAP>
+struct SegLds {
+    static constexpr int WAVES = THREADS / 64;
+    uint32_t keys[1 << BITS];
+    uint32_t cnt[1 << BITS];   // a slot's pairs, then its next bin position
+    uint32_t entry[CAP], t0[CAP], t1[CAP];
+    uint32_t n;
+    uint32_t tiles[WAVES], lo[WAVES], hi[WAVES];   // the waves' SegSums
+    uint32_t sum[WAVES], base, spilled;
 };
 
-template <int BITS, int TS>
-__device__ __forceinline__ void count_tiles(const PassDesc& P, const Workspace& ws, int pass, bool ok, const TriS& t,
-                                            uint32_t entry, uint32_t slot, uint32_t local, const SegTables* L) {
-    int tx0 = 0, ty0 = 0, tx1 = 0, ty1 = 0, nx = 0, n = 0;
-    if (ok) {
-        tx0 = t.tx0 >> TS;
-        ty0 = t.ty0 >> TS;
-        tx1 = t.x1 >> TS;
-        ty1 = t.y1 >> TS;
-        nx = tx1 - tx0 + 1;
-        n = nx * (ty1 - ty0 + 1);
-        gst4(ws.tris + slot, make_uint4(entry, (uint32_t)pass, (uint32_t)tx0 | ((uint32_t)ty0 << 16),
-                                        (uint32_t)tx1 | ((uint32_t)ty1 << 16)));
+// Of the narrow triangles that a lane, and then its wave, listed: their tiles,
+// and the bounds of those (x | y << 16).
+struct SegSums {
+    uint32_t tiles = 0u, lo = 0xFFFFFFFFu, hi = 0u;
+};
+typedef uint16_t us2_vec __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t min_xy(uint32_t a, uint32_t b) {
+    return __builtin_bit_cast(uint32_t, __builtin_elementwise_min(__builtin_bit_cast(us2_vec, a), __builtin_bit_cast(us2_vec, b)));
+}
+__device__ __forceinline__ uint32_t max_xy(uint32_t a, uint32_t b) {
+    return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(us2_vec, a), __builtin_bit_cast(us2_vec, b)));
+}
+
+template <int BITS, int THREADS, int CAP>
+__device__ __forceinline__ void seg_clear(SegLds<BITS, THREADS, CAP>& L) {
+    for (int i = threadIdx.x; i < (1 << BITS); i += THREADS) {
+        L.keys[i] = BIN_EMPTY;
+        L.cnt[i] = 0u;
     }
-    // a triangle over more than WIDE_TILES tiles is counted by the whole wave
-    int tile0 = P.tile0, tiles_x = P.tiles_x;
-    if constexpr (BITS > 0) {
-        if (n > WIDE_TILES) L->wide[atomicAdd(L->nwide, 1u)] = (uint16_t)local;
-    }
-    uint64_t wide = __ballot(n > WIDE_TILES);
-    while (wide) {
-        int src = __ffsll((unsigned long long)wide) - 1;
-        wide &= wide - 1;
-        int wn = __shfl(n, src), wnx = __shfl(nx, src), wx0 = __shfl(tx0, src), wy0 = __shfl(ty0, src);
-        int wt0 = __shfl(tile0, src), wtx = __shfl(tiles_x, src);
-        for (int k = __lane_id(); k < wn; k += 64)
-            gadd(ws.tile_count + (wt0 + (wy0 + k / wnx) * wtx + wx0 + k % wnx), 1u);
-    }
-    int ns = n > WIDE_TILES ? 0 : n;
-    if constexpr (BITS == 0) {
-        for (int k = 0; __ballot(k < ns); k++) {
-            bool want = k < ns;
-            int gt = want ? tile0 + (ty0 + k / nx) * tiles_x + tx0 + k % nx : 0;
-            wave_count(ws.tile_count, gt, want);
-        }
-    } else {
-        for (int k = 0; k < ns; k++)
-            lds_count<BITS>(L->keys, L->cnt, ws.tile_count, (uint32_t)(tile0 + (ty0 + k / nx) * tiles_x + tx0 + k % nx));
-    }
-    if (P.stats) {
-        for (int off = 32; off > 0; off >>= 1) n += __shfl_xor(n, off);
-        if (__lane_id() == 0) stat_add(P, ST_ENTRIES, (uint64_t)n);
+    if (threadIdx.x == 0) {
+        L.spilled = 0u;
+        L.n = 0u;
     }
 }
 
@@ -527,7 +606,181 @@ __device__ __forceinline__ uint32_t wave_reserve_lds(uint32_t* counter, bool wan
     int leader = m ? __ffsll((unsigned long long)m) - 1 : 0;
     if (m && lane == leader) base = atomicAdd(counter, (uint32_t)__popcll(m));
     base = __shfl(base, leader);
-    return base + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
+    return base + mask_rank(m);
+}
+
+// Lists the triangle of every lane with `ok`; returns its place.
+template <int BITS, int THREADS, int CAP>
+__device__ __forceinline__ uint32_t seg_list(SegLds<BITS, THREADS, CAP>& L, SegSums& a, bool ok, const TileSpan& s) {
+    uint32_t i = wave_reserve_lds(&L.n, ok);
+    if (ok) {
+        L.entry[i] = s.entry;
+        L.t0[i] = s.t0;
+        L.t1[i] = s.t1;
+        const int n = s.nx() * s.ny();
+        if (n <= WIDE_TILES) {
+            a.tiles += (uint32_t)n;
+            a.lo = min_xy(a.lo, s.t0);
+            a.hi = max_xy(a.hi, s.t1);
+        }
+    }
+    return i;
+}
+
+// Leaves the wave's sums for bin_segment; a barrier must follow.
+template <int BITS, int THREADS, int CAP>
+__device__ __forceinline__ void seg_sums(SegLds<BITS, THREADS, CAP>& L, SegSums& a) {
+#define HANA_DPP_STEP(ctrl, rows)                                                                            \
+    a.lo = min_xy(a.lo, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)a.lo, ctrl, rows, 0xF, false));        \
+    a.hi = max_xy(a.hi, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)a.hi, ctrl, rows, 0xF, false));
+    HANA_DPP_STEP(0x111, 0xF)
+    HANA_DPP_STEP(0x112, 0xF)
+    HANA_DPP_STEP(0x114, 0xF)
+    HANA_DPP_STEP(0x118, 0xF)
+    HANA_DPP_STEP(0x142, 0xA)
+    HANA_DPP_STEP(0x143, 0xC)
+#undef HANA_DPP_STEP
+    a.tiles = wave_scan(a.tiles);
+    if (__lane_id() == 63) {
+        const int w = threadIdx.x >> 6;
+        L.tiles[w] = a.tiles;
+        L.lo[w] = a.lo;
+        L.hi[w] = a.hi;
+    }
+    a = SegSums();
+}
+
+// Bins the listed triangles, of passes pass_of(place).  Their pairs are
+// counted per tile in the LDS table, the workgroup takes a descriptor per
+// distinct tile with one global atomic each, all in flight together; then
+// every pair takes its place with an LDS atomic.
+//  - SPREAD (the one-launch geometry, all triangles of one pass, the sums made):
+//    1, 2 or 4 lanes go to a triangle, by the mean number of its tiles, and the
+//    table holds the rectangle of tiles that the triangles lie in, where that
+//    fits -- a workgroup's faces follow one another in the mesh and mostly lie
+//    close together --, else the distinct tiles by a hash, whose probes are a
+//    chain of LDS accesses.  There one workgroup's chain is the launch's time
+//    (thumbnail, 300x300 with 1,160 faces: 15.4 -> 13.3 us a frame).  Where
+//    workgroups fill the chip it is the instructions that count, and the plain
+//    loop is faster (460,800 faces at 1080p: set-up 28.7 us against 32.8).
+//  - The pairs go to the workgroup's own entries of the bins, [own, own_end),
+//    or, where there are more, to a range of the shared rest.  (One shared
+//    range for all, taken with an atomic on one counter, serialised the
+//    workgroups: with 39,000 of them set-up took 818 us instead of 546.)
+// Returns the own entries taken.  The table was cleared, the list and the sums
+// made and a barrier passed since.
+template <bool SPREAD, int BITS, int THREADS, int CAP, class PassOf>
+__device__ __forceinline__ uint32_t bin_segment(SegLds<BITS, THREADS, CAP>& L, const PassOf& pass_of, const Workspace& ws,
+                                                uint32_t own, uint32_t own_end) {
+    constexpr int SLOTS = 1 << BITS, PER = SLOTS / THREADS, WAVES = THREADS / 64;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const uint32_t n = L.n;
+    if (!n) return 0u;
+    uint32_t tiles = 0u, lo = 0xFFFFFFFFu, hi = 0u;
+#pragma unroll
+    for (int w = 0; SPREAD && w < WAVES; w++) {
+        tiles += L.tiles[w];
+        lo = min_xy(lo, L.lo[w]);
+        hi = max_xy(hi, L.hi[w]);
+    }
+    tiles = __builtin_amdgcn_readfirstlane(tiles);
+    lo = __builtin_amdgcn_readfirstlane(lo);
+    hi = __builtin_amdgcn_readfirstlane(hi);
+    const int bx = (int)(lo & 0xFFFFu), by = (int)(lo >> 16), bw = (int)(hi & 0xFFFFu) - bx + 1, bh = (int)(hi >> 16) - by + 1;
+    const bool dense = SPREAD && tiles && bw * bh <= SLOTS;   // uniform
+    const int sh = !SPREAD ? 0 : tiles > 4u * n ? 2 : (tiles > 2u * n ? 1 : 0);
+    for (uint32_t i0 = 0; i0 < n; i0 += THREADS >> sh) {   // uniform
+        const uint32_t i = i0 + (uint32_t)(tid >> sh);
+        const bool have = i < n;
+        TileSpan t{0u, 0u, 0u};
+        if (have) t = TileSpan{L.entry[i], L.t0[i], L.t1[i]};
+        const PassDesc& P = pass_of(have ? i : 0u);
+        const int nx = t.nx(), nt = nx * t.ny(), k0 = tid & ((1 << sh) - 1);
+        const bool wide = have && nt > WIDE_TILES;
+        bin_wide(P, ws, wide && k0 == 0, t);
+        if (have && k0 == 0 && P.stats) stat_add(P, ST_ENTRIES, (uint64_t)nt);
+        if (!have || wide) continue;
+        const uint32_t magic = tile_div_magic(nx);
+        const int first = dense ? (t.y0() - by) * bw + t.x0() - bx : P.tile0 + t.y0() * P.tiles_x + t.x0();
+        const int pitch = dense ? bw : P.tiles_x;
+        for (int k = k0; k < nt; k += 1 << sh) {
+            const int y = tile_div(k, magic), at = first + y * pitch + k - y * nx;
+            const int sl = dense ? at : bin_slot<BITS>(L.keys, (uint32_t)at, true);
+            if (sl >= 0) {
+                atomicAdd(&L.cnt[sl], 1u);
+            } else {
+                atomicAdd(&L.spilled, 1u);
+                put_chunk(ws, (uint32_t)at, gadd(ws.tile_chunks + at, 1u), make_uint2(t.entry, CHUNK_INLINE));
+            }
+        }
+    }
+    lds_barrier();
+    // this lane's PER consecutive slots: their descriptors' places are fetched
+    // while the workgroup's range is
+    uint32_t key[PER], c[PER], idx[PER], sum = 0;
+    const float inv = 1.0f / (float)bw;
+#pragma unroll
+    for (int i = 0; i < PER; i++) {
+        const int sl = tid * PER + i;
+        c[i] = L.cnt[sl];
+        if (dense) {
+            const PassDesc& P = pass_of(0u);
+            const int y = (int)(((float)sl + 0.5f) * inv);   // sl / bw: exact for such small integers
+            key[i] = (uint32_t)(P.tile0 + (by + y) * P.tiles_x + bx + sl - y * bw);
+        } else {
+            key[i] = L.keys[sl];
+        }
+        idx[i] = c[i] ? gadd(ws.tile_chunks + key[i], 1u) : 0u;
+        sum += c[i];
+    }
+    uint32_t incl = wave_scan(sum);
+    if (lane == 63) L.sum[tid >> 6] = incl;
+    lds_barrier();
+    uint32_t before = 0, total = 0;
+#pragma unroll
+    for (int w = 0; w < WAVES; w++) {
+        uint32_t v = L.sum[w];
+        if (w < (tid >> 6)) before += v;
+        total += v;
+    }
+    const uint32_t all = total + L.spilled;
+    uint32_t first = own, took = total;
+    bool fits = true;
+    if (total > own_end - own || all != total) {   // uniform
+        if (tid == 0) {
+            uint64_t b = ws.seg_region + seq_add64(ws, SEQ_PAIRS, all);
+            L.base = b + all <= ws.bin_cap ? (uint32_t)b : ws.bin_cap;   // past the capacity nothing is kept
+        }
+        lds_barrier();
+        first = L.base;
+        fits = first < ws.bin_cap;
+        took = 0u;
+    }
+    uint32_t pos = first + before + incl - sum;
+#pragma unroll
+    for (int i = 0; i < PER; i++)
+        if (c[i]) {
+            put_chunk(ws, key[i], idx[i], make_uint2(pos, c[i]));
+            L.cnt[tid * PER + i] = pos;
+            pos += c[i];
+        }
+    lds_barrier();
+    if (!fits) return took;
+    for (uint32_t i = (uint32_t)(tid >> sh); i < n; i += THREADS >> sh) {
+        TileSpan t{L.entry[i], L.t0[i], L.t1[i]};
+        const int nx = t.nx(), nt = nx * t.ny();
+        if (nt > WIDE_TILES) continue;
+        const PassDesc& P = pass_of(i);
+        const uint32_t magic = tile_div_magic(nx);
+        const int at0 = dense ? (t.y0() - by) * bw + t.x0() - bx : P.tile0 + t.y0() * P.tiles_x + t.x0();
+        const int pitch = dense ? bw : P.tiles_x;
+        for (int k = tid & ((1 << sh) - 1); k < nt; k += 1 << sh) {
+            const int y = tile_div(k, magic), at = at0 + y * pitch + k - y * nx;
+            const int sl = dense ? at : bin_slot<BITS>(L.keys, (uint32_t)at, false);
+            if (sl >= 0) gst(ws.bins + atomicAdd(&L.cnt[sl], 1u), t.entry);
+        }
+    }
+    return took;
 }
 
 // Faces that fail the trivial accept, from the outcodes of their vertices:
@@ -543,72 +796,319 @@ __device__ __forceinline__ bool dies_at_first_crossed_plane(uint32_t c0, uint32_
 }
 
 // FPT faces per lane.  Trivially accepted faces are set up from the shared
-// post-transform vertices and listed in this workgroup's segment of ws.tris
-// (BLOCK * FPT records from blockIdx.x * BLOCK * FPT; the count goes to
-// ws.seg_count); faces that clipping would remove are dropped; the others are
-// queued for k_clip with one global atomic per workgroup.
+// post-transform vertices and binned; faces that clipping would remove are
+// dropped; the others are queued for k_clip with one global atomic per
+// workgroup.
 // Six waves per SIMD: the gathers of all FPT faces in flight take about 80
 // VGPRs; at 64 (eight waves) the compiler serialises them and the kernel is
 // slower, at 97 (five) it is slower too.
 template <int BITS, int TS>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(6))) void k_setup(const PassDesc* __restrict__ passes, int npasses, Workspace ws) {
-    constexpr int SLOTS = 1 << BITS;
-    __shared__ uint64_t s_queue[BLOCK * FPT];
-    __shared__ uint32_t s_keys[SLOTS], s_cnt[SLOTS];   // tile counts of the workgroup's triangles
-    __shared__ uint16_t s_wide[BLOCK * FPT];
-    __shared__ uint32_t s_ntri, s_nq, s_qbase, s_nwide, s_nlist;
-    if (threadIdx.x == 0) { s_ntri = 0; s_nq = 0; s_nwide = 0; s_nlist = 0; }
-    const SegTables L{s_keys, s_cnt, s_wide, &s_nwide};
+    __shared__ SegLds<BITS, BLOCK, BLOCK * FPT> L;
+    __shared__ uint32_t s_nq, s_qbase;
+    if (threadIdx.x == 0) s_nq = 0;
     int pass = find_pass<1>(passes, npasses, blockIdx.x);
     const PassDesc& P = passes[pass];
     int base = (blockIdx.x - P.fblock0) * BLOCK * FPT;
-    uint32_t seg = (uint32_t)blockIdx.x * (BLOCK * FPT);
-    // Lanes past the pass's last face load that face (a pass that owns a
-    // workgroup has one), so that no load waits on a branch: the indices of
-    // all FPT faces are in flight together, then the outcodes and
-    // post-transform vertices of all of them (gathered together, so the
-    // vertices do not wait for the trivial-accept test).  They are issued
-    // before the tile table is cleared, so that the clear and its barrier
-    // overlap them.
-    int ids[FPT][3];
-    bool valid[FPT];
+    // FPR faces per lane at a time.  Lanes past the pass's last face load that
+    // face (a pass that owns a workgroup has one), so that no load waits on a
+    // branch: the indices of all FPR faces are in flight together, then the
+    // outcodes and post-transform vertices of all of them (gathered together,
+    // so the vertices do not wait for the trivial-accept test).  The first are
+    // issued before the tile table is cleared, so that the clear and its
+    // barrier overlap them.
+    constexpr int FPR = 4;
+    static_assert(FPT % FPR == 0, "whole rounds");
+    SegSums sums;
+#pragma unroll 1
+    for (int r = 0; r < FPT; r += FPR) {
+        int ids[FPR][3];
+        bool valid[FPR];
 #pragma unroll
-    for (int k = 0; k < FPT; k++) {
+        for (int k = 0; k < FPR; k++) {
+            int f = base + (r + k) * BLOCK + threadIdx.x;
+            valid[k] = f < P.nfaces;
+            int fl = valid[k] ? f : P.nfaces - 1;
+            ids[k][0] = gld(P.idx + 3 * fl);
+            ids[k][1] = gld(P.idx + 3 * fl + 1);
+            ids[k][2] = gld(P.idx + 3 * fl + 2);
+        }
+        uint32_t codes[FPR][3];
+        float4 va[FPR], vb[FPR], vc[FPR];
+#pragma unroll
+        for (int k = 0; k < FPR; k++) {
+            for (int j = 0; j < 3; j++) codes[k][j] = gld(P.code + ids[k][j]);
+            va[k] = gld4(P.vr + ids[k][0]);
+            vb[k] = gld4(P.vr + ids[k][1]);
+            vc[k] = gld4(P.vr + ids[k][2]);
+        }
+        if (r == 0) {
+            seg_clear(L);
+            lds_barrier();
+        }
+#pragma unroll
+        for (int k = 0; k < FPR; k++)
+            for (int j = 0; j < 3; j++) codes[k][j] = valid[k] ? codes[k][j] : 0u;
+#pragma unroll
+        for (int k = 0; k < FPR; k++) {
+            int f = base + (r + k) * BLOCK + threadIdx.x;
+            bool trivial = valid[k] && (codes[k][0] & codes[k][1] & codes[k][2] & CODE_VISIBLE);
+            bool clipped = valid[k] && !trivial;
+            bool clipq = clipped && !dies_at_first_crossed_plane(codes[k][0], codes[k][1], codes[k][2]);
+            if (clipped && !clipq) gst(P.poly_of_face + f, -1);
+            // faces to clip take the list's places from its end: a face is either
+            uint32_t q = wave_reserve_lds(&s_nq, clipq);
+            if (clipq) L.entry[BLOCK * FPT - 1 - q] = (uint32_t)f;
+            if (P.stats) {
+                uint64_t nv = __popcll(__ballot(valid[k])), nc = __popcll(__ballot(clipped));
+                if (__lane_id() == 0) {
+                    stat_add(P, ST_FACES, nv);
+                    stat_add(P, ST_CLIPPED, nc);
+                }
+            }
+            TriS t;
+            uint32_t flags = 0;
+            bool ok = trivial && tri_setup(va[k], vb[k], vc[k], P.width, P.height, t, flags);
+            seg_list(L, sums, ok, ok ? span_of<TS>(t, (uint32_t)f | flags) : TileSpan{0u, 0u, 0u});
+        }
+    }
+    lds_barrier();
+    if (threadIdx.x == 0) s_qbase = s_nq ? atomicAdd(&ws.seq[SEQ_CLIPQ], s_nq) : 0u;
+    const uint32_t own = blockIdx.x * (SEG_PAIRS * BLOCK * FPT);
+    bin_segment<false>(L, [&](uint32_t) -> const PassDesc& { return P; }, ws, own, own + SEG_PAIRS * BLOCK * FPT);
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < s_nq; i += BLOCK) {
+        uint32_t q = s_qbase + i;
+        if (q < ws.clipq_cap) gst(ws.clip_queue + q, ((uint64_t)(uint32_t)pass << 32) | L.entry[BLOCK * FPT - 1 - i]);
+        else raise_flag(ws, FLAG_CLIPQ_OVERFLOW);
+    }
+}
+
+// The LDS of a clipping round of FACES faces.
+template <int FACES>
+struct ClipLds {
+    float buf[FACES][2][POLY_MAX][CLIP_NF];
+    float4 ndc[FACES][POLY_MAX];
+    uint32_t npoly, poly0;
+};
+
+// Clips one face per group of CLIP_GROUP lanes (`have`, uniform within the
+// group) and lists its fan triangles in B (at most POLY_MAX - 2 per face) for
+// bin_segment, handing their places to listed(); the whole workgroup calls it
+// together.  Per
+// group: the vertex program runs on the three corners in three lanes (the same
+// program as k_vertex, so the same bits); then each of the seven planes of
+// clip_triangle (SR/graphics.cpp:136-161) in order, one Sutherland-Hodgman
+// stage (SR/graphics.cpp:73-110) computed vertex-parallel: lane i looks at the
+// edge (i-1, i) and emits the intersection when the two ends differ in side
+// and vertex i when it is inside, at the place the prefix sum of the lanes'
+// emissions gives it -- the order and the arithmetic of the sequential loop.
+// A stage with every vertex inside would copy the polygon unchanged and is
+// skipped.  Pool slots (one per polygon) are reserved once per workgroup and
+// round.
+template <int TS, int FACES, class Seg, class Listed>
+__device__ __forceinline__ void clip_round(ClipLds<FACES>& L, Seg& B, SegSums& sums, const PassDesc& P, Uniforms u, const Workspace& ws,
+                                           bool have, int f, const Listed& listed) {
+    const int tid = threadIdx.x, lane = tid & 63, g = tid / CLIP_GROUP, li = tid % CLIP_GROUP;
+    const uint64_t gmask = 0xFFFFull << (lane & ~(CLIP_GROUP - 1));
+    if (tid == 0) L.npoly = 0;
+    if (have && li < 3) {
+        int v = gld(P.idx + 3 * f + li);
+        bool need_n = P.kind != SHADER_SHADOW && P.kind != SHADER_TEXTURE;
+        F3 p = f3(gld(P.px + v), gld(P.py + v), gld(P.pz + v));
+        F3 nn = need_n ? f3(gld(P.nx + v), gld(P.ny + v), gld(P.nz + v)) : f3(0.f, 0.f, 0.f);
+        float clip[4], vary[8];
+        for (int c = 0; c < 8; c++) vary[c] = 0.0f;
+        vertex_program(P.kind, u, p, nn, gld(P.tu + v), gld(P.tv + v), clip, vary);
+        for (int c = 0; c < 4; c++) L.buf[g][0][li][c] = clip[c];
+        for (int c = 0; c < POLY_VARY; c++) L.buf[g][0][li][4 + c] = vary[c];
+    }
+    wave_sync();
+    int n = have ? 3 : 0, cur = 0;
+    bool too_large = false;
+    for (int plane = 0; plane < CLIP_PLANES; plane++) {
+        bool act = li < n;
+        bool cin = act && inside_plane(L.buf[g][cur][li], plane);
+        uint64_t am = __ballot(act) & gmask, im = __ballot(cin) & gmask;
+        if (n < 3 || am == im) continue;         // dead, or every vertex inside
+        int prev = li == 0 ? n - 1 : li - 1;
+        bool pin = act && inside_plane(L.buf[g][cur][prev], plane);
+        int emit = act ? (pin != cin) + (cin ? 1 : 0) : 0;
+        int incl = emit;
+        for (int d = 1; d < CLIP_GROUP; d <<= 1) {
+            int o = __shfl_up(incl, d, CLIP_GROUP);
+            if (li >= d) incl += o;
+        }
+        int m = __shfl(incl, CLIP_GROUP - 1, CLIP_GROUP);
+        if (m > POLY_MAX) {                      // only possible through rounding
+            too_large = true;
+            n = 0;
+            continue;
+        }
+        int o = incl - emit;
+        float(*in)[CLIP_NF] = L.buf[g][cur];
+        float(*out)[CLIP_NF] = L.buf[g][cur ^ 1];
+        if (act && pin != cin) {
+            float t = intersect_ratio(in[prev], in[li], plane);
+            for (int k = 0; k < CLIP_NF; k++) {
+                float fv = in[prev][k];
+                out[o][k] = fv + (in[li][k] - fv) * t;
+            }
+            o++;
+        }
+        if (cin)
+            for (int k = 0; k < CLIP_NF; k++) out[o][k] = in[li][k];
+        n = m < 3 ? 0 : m;
+        cur ^= 1;
+        wave_sync();
+    }
+    if (too_large && li == 0) raise_flag(ws, FLAG_POLY_TOO_LARGE);
+    float(*poly)[CLIP_NF] = L.buf[g][cur];
+    bool keep = n >= 3;                          // uniform within the group
+    float4 own = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (keep && li < n) L.ndc[g][li] = own = ndc_of(poly[li]);
+    wave_sync();
+    // fan triangle (0, li+1, li+2) of the polygon in lane li
+    TriS t;
+    uint32_t flags = 0;   // found again by the raster
+    bool ok = keep && li < n - 2 && tri_setup(L.ndc[g][0], L.ndc[g][li + 1], L.ndc[g][li + 2], P.width, P.height, t, flags);
+    __syncthreads();
+    uint32_t lpoly = wave_reserve_lds(&L.npoly, keep && li == 0);
+    __syncthreads();
+    if (tid == 0) L.poly0 = L.npoly ? atomicAdd(&ws.seq[SEQ_POLYS], L.npoly) : 0u;
+    __syncthreads();
+    uint32_t pid = __shfl(L.poly0 + lpoly, lane & ~(CLIP_GROUP - 1));
+    if (keep && pid >= ws.poly_cap) {
+        // nothing is rasterised; its triangles are still binned, for the needs
+        if (li == 0) raise_flag(ws, FLAG_POLY_OVERFLOW);
+        keep = false;
+    }
+    if (keep && li < n) {
+        gst4(ws.pool_vr + ((size_t)pid * POLY_MAX + li), own);
+        for (int c = 0; c < POLY_VARY; c++) gst(ws.pool_vs + (((size_t)pid * POLY_MAX + li) * POLY_VARY + c), poly[li][4 + c]);
+    }
+    if (have && li == 0) {
+        if (keep) {
+            gst(ws.pool_face + pid, f);
+            stat_add(P, ST_POLYS, 1);
+        }
+        gst(P.poly_of_face + f, keep ? (int)pid : -1);
+    }
+    uint32_t at = seg_list(B, sums, ok, ok ? span_of<TS>(t, CLIPPED_BIT | (pid << FAN_BITS) | (uint32_t)li) : TileSpan{0u, 0u, 0u});
+    if (ok) listed(at);
+    __syncthreads();
+}
+
+// Clips the queued faces, CLIP_FACES per workgroup and round, grid-stride over
+// the queue.
+template <int TS>
+__global__ __launch_bounds__(CLIP_THREADS) void k_clip(const PassDesc* __restrict__ passes, Workspace ws) {
+    constexpr int FANS = CLIP_FACES * (POLY_MAX - 2);
+    __shared__ ClipLds<CLIP_FACES> L;
+    __shared__ SegLds<10, CLIP_THREADS, FANS> B;
+    __shared__ int fan_pass[FANS];
+    uint32_t count = min(ws.seq[SEQ_CLIPQ], ws.clipq_cap);
+    for (uint32_t base = blockIdx.x * CLIP_FACES; base < count; base += gridDim.x * CLIP_FACES) {
+        seg_clear(B);
+        SegSums sums;
+        uint32_t q = base + threadIdx.x / CLIP_GROUP;
+        bool have = q < count;
+        uint64_t e = have ? gld(ws.clip_queue + q) : 0ull;
+        const int pass = (int)(e >> 32);
+        const PassDesc& P = passes[pass];
+        clip_round<TS, CLIP_FACES>(L, B, sums, P, uniforms_of(P.u), ws, have, (int)(uint32_t)e,
+                                   [&](uint32_t at) { fan_pass[at] = pass; });
+        lds_barrier();
+        bin_segment<false>(B, [&](uint32_t i) -> const PassDesc& { return passes[fan_pass[i]]; }, ws, 0u, 0u);
+        __syncthreads();
+    }
+}
+
+// The geometry of a whole sequence in one launch.  Workgroups below nfb take
+// FRONT_FPT faces per lane: they run the vertex program on the faces' own
+// corners instead of waiting for the vertices of a launch before (each vertex
+// is then transformed about six times, by the same program, so to the same
+// bits), bin the trivially accepted faces and clip the others themselves, 16
+// at a time.  The other workgroups run the vertex program once per vertex for
+// the rasters' interpolation.  Three launches and two waits for their tails
+// become one, and a workgroup of 256 faces instead of 1024 spreads small
+// meshes over more CUs.  With ARGS the sequence's tables (at most two passes)
+// come with the launch, and its first workgroup stores them for the rasters:
+// no copy is enqueued before it.
+template <int TS, bool ARGS>
+__global__ __launch_bounds__(BLOCK) void k_front(FrontTables tables, PassDesc* __restrict__ d_passes,
+                                                 DevUniforms* __restrict__ d_unis, int npasses, Workspace ws, int nfb) {
+    constexpr int FACES = BLOCK / CLIP_GROUP, FANS = FACES * (POLY_MAX - 2);
+    __shared__ SegLds<10, BLOCK, BLOCK * FRONT_FPT + FANS> L;
+    __shared__ ClipLds<FACES> C;
+    __shared__ uint32_t s_queue[BLOCK * FRONT_FPT];
+    __shared__ uint32_t s_nq;
+    zero_counters(ws);
+    const PassDesc* passes = d_passes;
+    const HANA_CONST_AS FrontTables* args = nullptr;
+    if constexpr (ARGS) {
+        // the launch's own argument memory, read through the scalar cache
+        args = (const HANA_CONST_AS FrontTables*)__builtin_amdgcn_kernarg_segment_ptr();
+        passes = (const PassDesc*)&args->d[0];
+        if (blockIdx.x == gridDim.x - 1) {
+            const HANA_CONST_AS uint32_t* sd = (const HANA_CONST_AS uint32_t*)&args->d[0];
+            const HANA_CONST_AS uint32_t* su = (const HANA_CONST_AS uint32_t*)&args->u[0];
+            for (int i = threadIdx.x; i < npasses * (int)(sizeof(PassDesc) / 4); i += BLOCK) gst((uint32_t*)d_passes + i, sd[i]);
+            for (int i = threadIdx.x; i < npasses * (int)(sizeof(DevUniforms) / 4); i += BLOCK) gst((uint32_t*)d_unis + i, su[i]);
+        }
+    }
+    if ((int)blockIdx.x >= nfb) {
+        int vb = (int)blockIdx.x - nfb;
+        int pass = find_pass<0>(passes, npasses, vb);
+        const PassDesc& P = passes[pass];
+        if constexpr (ARGS) vertex_block<FRONT_VPT>(P, args->u[pass], (vb - P.vblock0) * BLOCK * FRONT_VPT);
+        else vertex_block<FRONT_VPT>(P, uniforms_of(P.u), (vb - P.vblock0) * BLOCK * FRONT_VPT);
+        return;
+    }
+    if (threadIdx.x == 0) s_nq = 0;
+    const int pass = find_pass<1>(passes, npasses, blockIdx.x);
+    const PassDesc& P = passes[pass];
+    const HANA_CONST_AS DevUniforms* up;
+    if constexpr (ARGS) up = &args->u[pass];
+    else up = (const HANA_CONST_AS DevUniforms*)P.u;
+    const int base = ((int)blockIdx.x - P.fblock0) * BLOCK * FRONT_FPT;
+    // lanes past the pass's last face take that face, so that no load waits on a branch
+    F3 corner[FRONT_FPT][3];
+    bool valid[FRONT_FPT];
+#pragma unroll
+    for (int k = 0; k < FRONT_FPT; k++) {
         int f = base + k * BLOCK + threadIdx.x;
         valid[k] = f < P.nfaces;
         int fl = valid[k] ? f : P.nfaces - 1;
-        ids[k][0] = gld(P.idx + 3 * fl);
-        ids[k][1] = gld(P.idx + 3 * fl + 1);
-        ids[k][2] = gld(P.idx + 3 * fl + 2);
+        int ids[3];
+        for (int j = 0; j < 3; j++) ids[j] = gld(P.idx + 3 * fl + j);
+        for (int j = 0; j < 3; j++) corner[k][j] = f3(gld(P.px + ids[j]), gld(P.py + ids[j]), gld(P.pz + ids[j]));
     }
-    uint32_t codes[FPT][3];
-    float4 va[FPT], vb[FPT], vc[FPT];
-#pragma unroll
-    for (int k = 0; k < FPT; k++) {
-        for (int j = 0; j < 3; j++) codes[k][j] = gld(P.code + ids[k][j]);
-        va[k] = gld4(P.vr + ids[k][0]);
-        vb[k] = gld4(P.vr + ids[k][1]);
-        vc[k] = gld4(P.vr + ids[k][2]);
-    }
-    for (int i = threadIdx.x; i < SLOTS; i += BLOCK) {
-        s_keys[i] = BIN_EMPTY;
-        s_cnt[i] = 0u;
-    }
+    seg_clear(L);
     lds_barrier();
+    const F3 none = f3(0.f, 0.f, 0.f);
+    SegSums sums;
 #pragma unroll
-    for (int k = 0; k < FPT; k++)
-        for (int j = 0; j < 3; j++) codes[k][j] = valid[k] ? codes[k][j] : 0u;
-    bool trivial[FPT];
-#pragma unroll
-    for (int k = 0; k < FPT; k++) trivial[k] = valid[k] && (codes[k][0] & codes[k][1] & codes[k][2] & CODE_VISIBLE);
-#pragma unroll
-    for (int k = 0; k < FPT; k++) {
+    for (int k = 0; k < FRONT_FPT; k++) {
         int f = base + k * BLOCK + threadIdx.x;
-        bool clipped = valid[k] && !trivial[k];
-        bool clipq = clipped && !dies_at_first_crossed_plane(codes[k][0], codes[k][1], codes[k][2]);
+        PostVertex va{}, vb{}, vc{};
+        F3 p = corner[k][0];
+#pragma unroll 1
+        for (int j = 0; j < 3; j++) {   // one copy of the code: a small sequence waits for its fetch
+            // the clip position alone: no normal or uv goes into it
+            float clip[4], vary[8];
+            vertex_program(P.kind == SHADER_SHADOW ? SHADER_SHADOW : SHADER_TEXTURE, *up, p, none, 0.f, 0.f, clip, vary);
+            va = vb;
+            vb = vc;
+            vc = post_vertex(clip);
+            p = j == 0 ? corner[k][1] : corner[k][2];
+        }
+        bool trivial = valid[k] && (va.code & vb.code & vc.code & CODE_VISIBLE);
+        bool clipped = valid[k] && !trivial;
+        bool clipq = clipped && !dies_at_first_crossed_plane(va.code, vb.code, vc.code);
         if (clipped && !clipq) gst(P.poly_of_face + f, -1);
         uint32_t q = wave_reserve_lds(&s_nq, clipq);
-        if (clipq) s_queue[q] = ((uint64_t)(uint32_t)pass << 32) | (uint32_t)f;
+        if (clipq) s_queue[q] = (uint32_t)f;
         if (P.stats) {
             uint64_t nv = __popcll(__ballot(valid[k])), nc = __popcll(__ballot(clipped));
             if (__lane_id() == 0) {
@@ -617,401 +1117,66 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(6))) void
             }
         }
         TriS t;
-        bool ok = trivial[k] && tri_setup(va[k], vb[k], vc[k], P.width, P.height, t);
-        uint32_t slot = wave_reserve_lds(&s_ntri, ok);
-        count_tiles<BITS, TS>(P, ws, pass, ok, t, (uint32_t)f, seg + slot, slot, &L);
+        uint32_t flags = 0;
+        bool ok = trivial && tri_setup(va.r, vb.r, vc.r, P.width, P.height, t, flags);
+        seg_list(L, sums, ok, ok ? span_of<TS>(t, (uint32_t)f | flags) : TileSpan{0u, 0u, 0u});
     }
-    __syncthreads();
-    // add the segment's counts to the global ones, and hand k_bin the list of
-    // its tiles with their counts and the list of its wide triangles
-    uint2* list = ws.seg_tiles + (size_t)blockIdx.x * SLOTS;
-    for (int i = threadIdx.x; i < SLOTS; i += BLOCK)
-        if (s_keys[i] != BIN_EMPTY) {
-            gadd(ws.tile_count + s_keys[i], s_cnt[i]);
-            gst2(list + atomicAdd(&s_nlist, 1u), make_uint2(s_keys[i], s_cnt[i]));
+    lds_barrier();
+    // clip until the list may not hold another round's fans, bin, go on
+    const uint32_t nq = s_nq;
+    uint32_t own = blockIdx.x * (SEG_PAIRS * BLOCK * FRONT_FPT);
+    const uint32_t own_end = own + SEG_PAIRS * BLOCK * FRONT_FPT;
+    for (uint32_t q0 = 0;;) {
+        while (q0 < nq && L.n <= BLOCK * FRONT_FPT) {   // uniform
+            uint32_t q = q0 + threadIdx.x / CLIP_GROUP;
+            bool have = q < nq;
+            clip_round<TS, FACES>(C, L, sums, P, *up, ws, have, have ? (int)s_queue[q] : 0, [](uint32_t) {});
+            q0 += FACES;
         }
-    uint32_t nwide = s_nwide;
-    for (uint32_t i = threadIdx.x; i < nwide; i += BLOCK) gst(ws.seg_wide + (size_t)blockIdx.x * (BLOCK * FPT) + i, s_wide[i]);
-    if (threadIdx.x == 0) {
-        gst(ws.seg_count + blockIdx.x, s_ntri);
-        s_qbase = s_nq ? atomicAdd(&ws.status[STATUS_CLIPQ], s_nq) : 0u;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) gst(ws.seg_info + blockIdx.x, s_nlist | (nwide << 16));
-    for (uint32_t i = threadIdx.x; i < s_nq; i += BLOCK) {
-        uint32_t q = s_qbase + i;
-        if (q < ws.clipq_cap) gst(ws.clip_queue + q, s_queue[i]);
-        else raise_flag(ws, FLAG_CLIPQ_OVERFLOW);
-    }
-}
-
-// Clips the queued faces, CLIP_FACES per workgroup and round, grid-stride
-// over the queue.  Per group of CLIP_GROUP lanes: the vertex program runs on
-// the three corners in three lanes (the same program as k_vertex, so the
-// same bits); then each of the seven planes of clip_triangle
-// (SR/graphics.cpp:136-161) in order, one Sutherland-Hodgman stage
-// (SR/graphics.cpp:73-110) computed vertex-parallel: lane i looks at the edge
-// (i-1, i) and emits the intersection when the two ends differ in side and
-// vertex i when it is inside, at the place the prefix sum of the lanes'
-// emissions gives it -- the order and the arithmetic of the sequential loop.
-// A stage with every vertex inside would copy the polygon unchanged and is
-// skipped.  Pool slots (one per polygon) and the fan triangles' records
-// (after the setup segments of ws.tris) are reserved once per workgroup and
-// round.
-template <int TS>
-__global__ __launch_bounds__(CLIP_THREADS) void k_clip(const PassDesc* __restrict__ passes, Workspace ws) {
-    __shared__ float buf[CLIP_FACES][2][POLY_MAX][CLIP_NF];
-    __shared__ uint32_t s_npoly, s_ntri, s_poly0, s_tri0;
-    uint32_t count = min(ws.status[STATUS_CLIPQ], ws.clipq_cap);
-    uint32_t clip_cap = ws.tris_cap - ws.seg_region;
-    const int tid = threadIdx.x, lane = tid & 63, g = tid / CLIP_GROUP, li = tid % CLIP_GROUP;
-    const uint64_t gmask = 0xFFFFull << (lane & ~(CLIP_GROUP - 1));
-    for (uint32_t base = blockIdx.x * CLIP_FACES; base < count; base += gridDim.x * CLIP_FACES) {
-        if (tid == 0) { s_npoly = 0; s_ntri = 0; }
-        uint32_t q = base + (uint32_t)g;
-        bool have = q < count;                       // uniform within the group
-        int pass = 0, f = 0;
-        if (have) {
-            uint64_t e = gld(ws.clip_queue + q);
-            pass = (int)(e >> 32);
-            f = (int)(uint32_t)e;
-        }
-        const PassDesc& P = passes[pass];
-        if (have && li < 3) {
-            int v = gld(P.idx + 3 * f + li);
-            bool need_n = P.kind != SHADER_SHADOW && P.kind != SHADER_TEXTURE;
-            F3 p = f3(gld(P.px + v), gld(P.py + v), gld(P.pz + v));
-            F3 nn = need_n ? f3(gld(P.nx + v), gld(P.ny + v), gld(P.nz + v)) : f3(0.f, 0.f, 0.f);
-            float clip[4], vary[8];
-            for (int c = 0; c < 8; c++) vary[c] = 0.0f;
-            vertex_program(P.kind, uniforms_of(P.u), p, nn, gld(P.tu + v), gld(P.tv + v), clip, vary);
-            for (int c = 0; c < 4; c++) buf[g][0][li][c] = clip[c];
-            for (int c = 0; c < POLY_VARY; c++) buf[g][0][li][4 + c] = vary[c];
-        }
-        wave_sync();
-        int n = have ? 3 : 0, cur = 0;
-        bool too_large = false;
-        for (int plane = PL_W; plane <= PL_NZ; plane++) {
-            bool act = li < n;
-            bool cin = act && inside_plane(buf[g][cur][li], plane);
-            uint64_t am = __ballot(act) & gmask, im = __ballot(cin) & gmask;
-            if (n < 3 || am == im) continue;         // dead, or every vertex inside
-            int prev = (li - 1 + n) % n;
-            bool pin = act && inside_plane(buf[g][cur][prev], plane);
-            int emit = act ? (pin != cin) + (cin ? 1 : 0) : 0;
-            int incl = emit;
-            for (int d = 1; d < CLIP_GROUP; d <<= 1) {
-                int o = __shfl_up(incl, d, CLIP_GROUP);
-                if (li >= d) incl += o;
-            }
-            int m = __shfl(incl, CLIP_GROUP - 1, CLIP_GROUP);
-            if (m > POLY_MAX) {                      // only possible through rounding
-                too_large = true;
-                n = 0;
-                continue;
-            }
-            int o = incl - emit;
-            float(*in)[CLIP_NF] = buf[g][cur];
-            float(*out)[CLIP_NF] = buf[g][cur ^ 1];
-            if (act && pin != cin) {
-                float t = intersect_ratio(in[prev], in[li], plane);
-                for (int k = 0; k < CLIP_NF; k++) {
-                    float fv = in[prev][k];
-                    out[o][k] = fv + (in[li][k] - fv) * t;
-                }
-                o++;
-            }
-            if (cin)
-                for (int k = 0; k < CLIP_NF; k++) out[o][k] = in[li][k];
-            n = m < 3 ? 0 : m;
-            cur ^= 1;
-            wave_sync();
-        }
-        if (too_large && li == 0) raise_flag(ws, FLAG_POLY_TOO_LARGE);
-        float(*poly)[CLIP_NF] = buf[g][cur];
-        bool keep = n >= 3;                          // uniform within the group
-        // fan triangle (0, li+1, li+2) of the polygon in lane li
-        TriS t;
-        bool ok = keep && li < n - 2 && tri_setup(ndc_of(poly[0]), ndc_of(poly[li + 1]), ndc_of(poly[li + 2]), P.width,
-                                                P.height, t);
+        seg_sums(L, sums);
+        lds_barrier();
+        own += bin_segment<true>(L, [&](uint32_t) -> const PassDesc& { return P; }, ws, own, own_end);
+        if (q0 >= nq) break;
         __syncthreads();
-        uint32_t lpoly = wave_reserve_lds(&s_npoly, keep && li == 0);
-        uint32_t ltri = wave_reserve_lds(&s_ntri, ok);
-        __syncthreads();
-        if (tid == 0) {
-            s_poly0 = s_npoly ? atomicAdd(&ws.status[STATUS_POLYS], s_npoly) : 0u;
-            s_tri0 = s_ntri ? atomicAdd(&ws.status[STATUS_TRIS], s_ntri) : 0u;
-        }
-        __syncthreads();
-        uint32_t pid = __shfl(s_poly0 + lpoly, lane & ~(CLIP_GROUP - 1));
-        bool reserved = ok;
-        if (keep && pid >= ws.poly_cap) {
-            if (li == 0) raise_flag(ws, FLAG_POLY_OVERFLOW);
-            keep = false;
-            ok = false;
-        }
-        uint32_t slot = s_tri0 + ltri;
-        if (reserved && slot >= clip_cap) {
-            raise_flag(ws, FLAG_TRIS_OVERFLOW);
-            ok = reserved = false;
-        }
-        // a reserved record of a dropped polygon is written empty (no tiles) for k_bin
-        if (reserved && !ok) gst4(ws.tris + (ws.seg_region + slot), make_uint4(0u, 0u, 1u, 0u));
-        if (keep && li < n) {
-            gst4(ws.pool_vr + ((size_t)pid * POLY_MAX + li), ndc_of(poly[li]));
-            for (int c = 0; c < POLY_VARY; c++) gst(ws.pool_vs + (((size_t)pid * POLY_MAX + li) * POLY_VARY + c), poly[li][4 + c]);
-        }
-        if (have && li == 0) {
-            if (keep) {
-                gst(ws.pool_face + pid, f);
-                gst(ws.pool_pass + pid, pass);
-                gst(ws.pool_n + pid, n);
-                stat_add(P, ST_POLYS, 1);
-            }
-            gst(P.poly_of_face + f, keep ? (int)pid : -1);
-        }
-        count_tiles<0, TS>(P, ws, pass, ok, t, CLIPPED_BIT | (pid << FAN_BITS) | (uint32_t)li, ws.seg_region + slot,
-                           0u, nullptr);
+        seg_clear(L);
         __syncthreads();
     }
 }
 
-// Scatters one listed triangle into the bins of its tiles; wave-uniform.
-__device__ __forceinline__ void bin_record(const PassDesc* passes, const Workspace& ws, bool have, uint4 r) {
-    int tx0 = 0, ty0 = 0, nx = 0, n = 0, tile0 = 0, tiles_x = 0;
-    if (have) {
-        const PassDesc& P = passes[r.y];
-        tx0 = (int)(r.z & 0xFFFFu);
-        ty0 = (int)(r.z >> 16);
-        nx = (int)(r.w & 0xFFFFu) - tx0 + 1;
-        n = nx * ((int)(r.w >> 16) - ty0 + 1);
-        tile0 = P.tile0;
-        tiles_x = P.tiles_x;
-    }
-    uint64_t wide = __ballot(n > WIDE_TILES);
-    while (wide) {
-        int src = __ffsll((unsigned long long)wide) - 1;
-        wide &= wide - 1;
-        int wn = __shfl(n, src), wnx = __shfl(nx, src), wx0 = __shfl(tx0, src), wy0 = __shfl(ty0, src);
-        int wt0 = __shfl(tile0, src), wtx = __shfl(tiles_x, src);
-        uint32_t we = __shfl(r.x, src);
-        for (int k = __lane_id(); k < wn; k += 64) {
-            uint32_t pos = gadd(ws.tile_cursor + (wt0 + (wy0 + k / wnx) * wtx + wx0 + k % wnx), 1u);
-            if (pos < ws.bin_cap) gst(ws.bins + pos, we);
-        }
-    }
-    int ns = n > WIDE_TILES ? 0 : n;
-    for (int k = 0; __ballot(k < ns); k++) {
-        bool want = k < ns;
-        int gt = want ? tile0 + (ty0 + k / nx) * tiles_x + tx0 + k % nx : 0;
-        uint32_t pos = wave_reserve(ws.tile_cursor, gt, want);
-        if (want && pos < ws.bin_cap) gst(ws.bins + pos, r.x);
-    }
-}
-
-// Workgroups below nseg scatter the setup segment of their index: the
-// segment's per-tile pair counts (listed by k_setup) go into an LDS table,
-// each distinct tile reserves its range of the bin with one global atomic,
-// then every pair takes a place in that range with an LDS atomic.  The other
-// workgroups stride over the clipped fan triangles listed after the segments.
-template <int BITS>
-__global__ __launch_bounds__(BLOCK) void k_bin(const PassDesc* __restrict__ passes, Workspace ws, int nseg) {
-    constexpr int BIN_HASH = 1 << BITS;
-    if (ws.status[STATUS_SEQ_FLAGS] & FLAG_NO_RASTER) return;   // nothing is rasterised
-    if ((int)blockIdx.x < nseg) {
-        __shared__ uint32_t keys[BIN_HASH];
-        __shared__ uint32_t cnt[BIN_HASH];   // a slot's next bin position, set when its tile is inserted
-        // the segment's sizes (written by k_setup, uniform: scalar loads) are
-        // read before the table is cleared, so that they are not awaited after it
-        const uint32_t n = *(const HANA_CONST_AS uint32_t*)(ws.seg_count + blockIdx.x);
-        const uint32_t info = *(const HANA_CONST_AS uint32_t*)(ws.seg_info + blockIdx.x);
-        const uint4* rec = ws.tris + (size_t)blockIdx.x * (BLOCK * FPT);
-        // a segment's triangles are all of one pass (one k_setup workgroup's faces)
-        const uint32_t spass = n ? *(const HANA_CONST_AS uint32_t*)&rec[0].y : 0u;
-        for (int i = threadIdx.x; i < BIN_HASH; i += BLOCK) keys[i] = BIN_EMPTY;
-        __syncthreads();
-        const PassDesc& P = passes[spass];
-        // the segment's distinct tiles and their pair counts, as k_setup listed
-        // them (a tile that found no slot there, or finds none here, goes
-        // through the global cursor pair by pair below)
-        uint32_t nlist = info & 0xFFFFu, nw = info >> 16;
-        const uint2* list = ws.seg_tiles + (size_t)blockIdx.x * ws.seg_stride;
-        // listed tiles are distinct, so an inserted slot is this thread's:
-        // it reserves the tile's range of the bin at once
-        for (uint32_t i = threadIdx.x; i < nlist; i += BLOCK) {
-            uint2 e = gld2(list + i);
-            int sl = bin_slot<BITS>(keys, e.x, true);
-            if (sl >= 0) cnt[sl] = gadd(ws.tile_cursor + e.x, e.y);
-        }
-        __syncthreads();
-        for (uint32_t i = threadIdx.x; i < n; i += BLOCK) {
-            uint4 r = gld4(rec + i);
-            int tx0 = (int)(r.z & 0xFFFFu), ty0 = (int)(r.z >> 16);
-            int tx1 = (int)(r.w & 0xFFFFu), ty1 = (int)(r.w >> 16);
-            if ((tx1 - tx0 + 1) * (ty1 - ty0 + 1) > WIDE_TILES) continue;
-            for (int ty = ty0; ty <= ty1; ty++)
-                for (int tx = tx0; tx <= tx1; tx++) {
-                    uint32_t gt = (uint32_t)(P.tile0 + ty * P.tiles_x + tx);
-                    int sl = bin_slot<BITS>(keys, gt, false);
-                    uint32_t pos = sl >= 0 ? atomicAdd(&cnt[sl], 1u) : gadd(ws.tile_cursor + gt, 1u);
-                    if (pos < ws.bin_cap) gst(ws.bins + pos, r.x);
-                }
-        }
-        // wide triangles, one per wave at a time, their tiles spread over its lanes
-        const uint16_t* wide = ws.seg_wide + (size_t)blockIdx.x * (BLOCK * FPT);
-        for (uint32_t w = threadIdx.x >> 6; w < nw; w += BLOCK / 64) {
-            uint4 r = gld4(rec + gld(wide + w));
-            int tx0 = (int)(r.z & 0xFFFFu), ty0 = (int)(r.z >> 16);
-            int nx = (int)(r.w & 0xFFFFu) - tx0 + 1;
-            int nt = nx * ((int)(r.w >> 16) - ty0 + 1);
-            for (int k = threadIdx.x & 63; k < nt; k += 64) {
-                uint32_t pos = gadd(ws.tile_cursor + (P.tile0 + (ty0 + k / nx) * P.tiles_x + tx0 + k % nx), 1u);
-                if (pos < ws.bin_cap) gst(ws.bins + pos, r.x);
-            }
-        }
-        return;
-    }
-    uint32_t count = min(ws.status[STATUS_TRIS], ws.tris_cap - ws.seg_region);
-    uint32_t stride = (gridDim.x - (uint32_t)nseg) * BLOCK;
-    for (uint32_t base = (blockIdx.x - (uint32_t)nseg) * BLOCK; base < count; base += stride) {
-        uint32_t i = base + threadIdx.x;
-        bool have = i < count;
-        bin_record(passes, ws, have, have ? gld4(ws.tris + (ws.seg_region + i)) : make_uint4(0, 0, 0, 0));
-    }
-}
-
-// ---------------------------------------------------------------------------
-// k_scan_reduce / k_scan_apply: exclusive scan of the tile counts into
-// tile_offset (and tile_cursor, the scatter cursors).  Each workgroup owns
-// SCAN_CHUNK counters; the apply kernel adds the sums of the chunks before.
-// ---------------------------------------------------------------------------
-
-// Sums are 64-bit so that a total past 2^32 pairs is seen, not wrapped.
-__device__ __forceinline__ uint64_t shfl_xor64(uint64_t v, int m) {
-    uint32_t lo = __shfl_xor((uint32_t)v, m), hi = __shfl_xor((uint32_t)(v >> 32), m);
-    return ((uint64_t)hi << 32) | lo;
-}
-__device__ __forceinline__ uint64_t shfl_up64(uint64_t v, int d) {
-    uint32_t lo = __shfl_up((uint32_t)v, d), hi = __shfl_up((uint32_t)(v >> 32), d);
-    return ((uint64_t)hi << 32) | lo;
-}
-__device__ __forceinline__ uint64_t block_sum(uint64_t v, uint64_t* sh) {
-    for (int off = 32; off > 0; off >>= 1) v += shfl_xor64(v, off);
-    int w = threadIdx.x >> 6;
-    __syncthreads();
-    if ((threadIdx.x & 63) == 0) sh[w] = v;
-    __syncthreads();
-    uint64_t t = 0;
-    for (int i = 0; i < SCAN_THREADS / 64; i++) t += sh[i];
-    return t;
-}
-
-// A thread's SCAN_PER_THREAD consecutive counters from b (a multiple of 16,
-// so whole runs load as 16-byte vectors; buffers are 256-byte aligned).
-__device__ __forceinline__ void load_counts(const uint32_t* c, int b, int n, uint32_t (&v)[SCAN_PER_THREAD]) {
-    if (b + SCAN_PER_THREAD <= n) {
-        const uint4* q = reinterpret_cast<const uint4*>(c + b);
-#pragma unroll
-        for (int i = 0; i < SCAN_PER_THREAD / 4; i++) {
-            uint4 x = q[i];
-            v[4 * i] = x.x; v[4 * i + 1] = x.y; v[4 * i + 2] = x.z; v[4 * i + 3] = x.w;
-        }
+// The sequence's totals, once geometry is complete: the needs the host sizes
+// the next workspace by, and the flags.  Past the pair limit no workspace
+// would do: that flag alone.  Returns whether the sequence is rasterised.
+__device__ __forceinline__ bool sequence_fits(const Workspace& ws, bool publish) {
+    typedef uint32_t u8_vec __attribute__((ext_vector_type(8)));
+    u8_vec q = *(const HANA_CONST_AS u8_vec*)ws.seq;
+    uint64_t pairs = ((uint64_t)q[SEQ_PAIRS] | ((uint64_t)q[SEQ_PAIRS + 1] << 32)) + ws.seg_region;
+    uint64_t wide = (uint64_t)q[SEQ_WIDE_PAIRS] | ((uint64_t)q[SEQ_WIDE_PAIRS + 1] << 32);
+    uint32_t f = q[SEQ_FLAGS];
+    if (pairs + wide > MAX_PAIRS) {
+        f |= FLAG_PAIR_LIMIT;
     } else {
-#pragma unroll
-        for (int i = 0; i < SCAN_PER_THREAD; i++) v[i] = (b + i < n) ? c[b + i] : 0u;
+        if (pairs > ws.bin_cap) f |= FLAG_BIN_OVERFLOW;
+        if (q[SEQ_OVER] > ws.over_cap) f |= FLAG_CHUNK_OVERFLOW;
     }
-}
-
-// Set-up and clipping are complete when the scan runs: their counts become
-// the needs the host sizes the next launch sequence by.
-__device__ __forceinline__ void note_clip_needs(const Workspace& ws) {
-    atomicMax(&ws.status[STATUS_NEED_POLYS], ws.status[STATUS_POLYS]);
-    atomicMax(&ws.status[STATUS_NEED_TRIS], ws.status[STATUS_TRIS]);
-}
-
-__global__ __launch_bounds__(SCAN_THREADS) void k_scan_reduce(Workspace ws) {
-    __shared__ uint64_t sh[SCAN_THREADS / 64];
-    int n = ws.ntiles;
-    int b = blockIdx.x * SCAN_CHUNK + threadIdx.x * SCAN_PER_THREAD;
-    uint32_t v[SCAN_PER_THREAD];
-    load_counts(ws.tile_count, b, n, v);
-    uint64_t s = 0;
-#pragma unroll
-    for (int i = 0; i < SCAN_PER_THREAD; i++) s += v[i];
-    uint64_t t = block_sum(s, sh);
-    if (threadIdx.x == 0) ws.scan_part[blockIdx.x] = t;
-    if (blockIdx.x == 0 && threadIdx.x == 0) note_clip_needs(ws);
-}
-
-// With a single chunk k_scan_reduce is not launched and this kernel alone
-// scans the counts.
-__global__ __launch_bounds__(SCAN_THREADS) void k_scan_apply(Workspace ws) {
-    __shared__ uint64_t sh[SCAN_THREADS / 64];
-    __shared__ uint64_t wsum[SCAN_THREADS / 64];
-    int n = ws.ntiles;
-    int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-    if (gridDim.x == 1 && tid == 0) note_clip_needs(ws);
-    // sum of the chunks before this one
-    uint64_t before = 0;
-    for (int i = tid; i < (int)blockIdx.x; i += SCAN_THREADS) before += ws.scan_part[i];
-    before = block_sum(before, sh);
-    // this thread's counters, then an exclusive scan of the thread sums
-    int b = blockIdx.x * SCAN_CHUNK + tid * SCAN_PER_THREAD;
-    uint32_t v[SCAN_PER_THREAD];
-    load_counts(ws.tile_count, b, n, v);
-    uint64_t s = 0;
-#pragma unroll
-    for (int i = 0; i < SCAN_PER_THREAD; i++) s += v[i];
-    uint64_t incl = s;
-    for (int d = 1; d < 64; d <<= 1) {
-        uint64_t o = shfl_up64(incl, d);
-        if (lane >= d) incl += o;
-    }
-    if (lane == 63) wsum[w] = incl;
-    __syncthreads();
-    uint64_t wbefore = 0;
-    for (int i = 0; i < w; i++) wbefore += wsum[i];
-    uint64_t run = before + wbefore + incl - s;
-    // offsets past MAX_PAIRS are cut off (the sequence then rasterises nothing)
-    if (b + SCAN_PER_THREAD <= n) {
-        uint4* qo = reinterpret_cast<uint4*>(ws.tile_offset + b);
-        uint4* qc = reinterpret_cast<uint4*>(ws.tile_cursor + b);
-#pragma unroll
-        for (int i = 0; i < SCAN_PER_THREAD / 4; i++) {
-            uint4 x;
-            x.x = (uint32_t)min(run, (uint64_t)MAX_PAIRS); run += v[4 * i];
-            x.y = (uint32_t)min(run, (uint64_t)MAX_PAIRS); run += v[4 * i + 1];
-            x.z = (uint32_t)min(run, (uint64_t)MAX_PAIRS); run += v[4 * i + 2];
-            x.w = (uint32_t)min(run, (uint64_t)MAX_PAIRS); run += v[4 * i + 3];
-            qo[i] = x;
-            qc[i] = x;
-        }
-    } else {
-        for (int i = 0; i < SCAN_PER_THREAD; i++)
-            if (b + i < n) {
-                ws.tile_offset[b + i] = (uint32_t)min(run, (uint64_t)MAX_PAIRS);
-                ws.tile_cursor[b + i] = (uint32_t)min(run, (uint64_t)MAX_PAIRS);
-                run += v[i];
+    if (publish) {
+        if (!(f & FLAG_PAIR_LIMIT)) {
+            atomicMax(&ws.status[STATUS_NEED_BINS], (uint32_t)pairs);
+            if (f & FLAG_CHUNK_OVERFLOW) {
+                uint64_t slots = ((uint64_t)ws.seq[SEQ_MAX_CHUNKS] + CHUNK_SLACK) * ws.q_items >> 10;
+                uint32_t wide = 0u;
+                for (const uint32_t* w = ws.wide_count; w < ws.tile_chunks; w++) wide = max(wide, *w);
+                atomicMax(&ws.status[STATUS_NEED_CHUNKS], (uint32_t)(slots < 0xFFFFFFFFu ? slots + 1u : slots));
+                atomicMax(&ws.status[STATUS_NEED_OVER], q[SEQ_OVER]);
+                atomicMax(&ws.status[STATUS_NEED_WIDE], wide);
             }
-    }
-    if (blockIdx.x == gridDim.x - 1 && tid == SCAN_THREADS - 1) {
-        // `run` of the last thread is the grand total
-        uint32_t total = (uint32_t)min(run, (uint64_t)MAX_PAIRS);
-        ws.tile_offset[n] = total;
-        ws.status[STATUS_BINS_NEEDED] = total;
-        // past the pair limit no workspace would do: that flag alone, and no need
-        // for the host to grow the bins by
-        if (run > MAX_PAIRS) {
-            raise_flag(ws, FLAG_PAIR_LIMIT);
-        } else {
-            atomicMax(&ws.status[STATUS_NEED_BINS], total);
-            if (run > ws.bin_cap) raise_flag(ws, FLAG_BIN_OVERFLOW);
         }
-        // every status word is final now (binning only reads them)
+        atomicMax(&ws.status[STATUS_NEED_POLYS], q[SEQ_POLYS]);
+        if (f) atomicOr(&ws.status[STATUS_FLAGS], f);
         if (ws.status_out)
             for (int i = 0; i < STATUS_WORDS; i++)
                 ws.status_out[i] = __hip_atomic_load(&ws.status[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
+    return !(f & FLAG_NO_RASTER);
 }
 
 // ---------------------------------------------------------------------------
@@ -1020,12 +1185,8 @@ __global__ __launch_bounds__(SCAN_THREADS) void k_scan_apply(Workspace ws) {
 
 constexpr int SMALL_PIX = HANA_SMALL_PIX;   // triangles with at most this many candidate pixels: one lane each
 
-// k / w for 0 <= k < 1024 and 1 <= w <= 32 (a tile's pixels and row widths)
-// as (k * magic) >> 16 with magic = ceil(2^16 / w): the excess
-// k * (magic - 2^16/w) / 2^16 stays below 1024 / 2^16 = 1/64, less than the
-// gap 1/w >= 1/32 between k/w and the next integer.
-__device__ __forceinline__ uint32_t tile_div_magic(int w) { return (65536u + (uint32_t)w - 1u) / (uint32_t)w; }
-__device__ __forceinline__ int tile_div(int k, uint32_t magic) { return (int)(((uint32_t)k * magic) >> 16); }
+// A tile's entries are swept from an LDS list of this many at a time.
+constexpr uint32_t TILE_LIST = 512;
 
 // The LDS of one raster workgroup: RB lanes (2 or 4 waves) over a tile of
 // 2^TS pixels a side.
@@ -1038,27 +1199,45 @@ struct TileLds {
     float ax[RB], ay[RB], s0x[RB], s0y[RB], s1x[RB], s1y[RB], uz[RB];
     float z0[RB], z1[RB], z2[RB];
     uint32_t lo[RB], box[RB];
-    int big[RB], med[RB];
+    uint8_t big[RB], med[RB];
+    uint32_t list[TILE_LIST];   // the tile's entries from some position on
+    uint32_t hits[2][RB / 64];  // wide triangles that touch the tile, per wave
     // staging counters of sweep round r in set r % 3 (nbig, head, nmed, mhead):
     // round r clears set (r + 2) % 3 once every wave is past round r - 1
     int cnt[3][4];
     int nan_seen;
 };
 
-__device__ __forceinline__ bool load_tri(const PassDesc& P, const Workspace& ws, uint32_t e, TriS& t, uint32_t& order) {
-    float4 a, b, c;
+// The arguments of the raster kernels, and their workspace read from there:
+// like fresh(P), for the fields that only clipped triangles need.
+struct RasterArgs {
+    const PassDesc* passes;
+    int npasses;
+    Workspace ws;
+};
+__device__ __forceinline__ const Workspace& raster_ws() {
+    const HANA_CONST_AS RasterArgs* a = (const HANA_CONST_AS RasterArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+    asm("" : "+s"(a));
+    return *(const Workspace*)&a->ws;
+}
+
+__device__ __forceinline__ void load_tri(const PassDesc& P, uint32_t e, TriS& t, uint32_t& order) {
     if (!(e & CLIPPED_BIT)) {
-        int f = (int)e;
+        int f = (int)(e & FACE_MASK);
         int i0 = gld(P.idx + 3 * f), i1 = gld(P.idx + 3 * f + 1), i2 = gld(P.idx + 3 * f + 2);
-        a = gld4(P.vr + i0); b = gld4(P.vr + i1); c = gld4(P.vr + i2);
         order = (uint32_t)f << 4;
+        tri_raster(gld4(P.vr + i0), gld4(P.vr + i1), gld4(P.vr + i2), P.width, P.height, t, e);
     } else {
         uint32_t pid = (e & ~CLIPPED_BIT) >> FAN_BITS, j = e & ((1u << FAN_BITS) - 1u);
+        const Workspace& ws = raster_ws();
         const float4* pv = ws.pool_vr + (size_t)pid * POLY_MAX;
-        a = gld4(pv); b = gld4(pv + j + 1); c = gld4(pv + j + 2);
         order = ((uint32_t)gld(ws.pool_face + pid) << 4) + 1u + j;
+        uint32_t flags = 0;
+        tri_setup(gld4(pv), gld4(pv + j + 1), gld4(pv + j + 2), P.width, P.height, t, flags);
+        if (flags & FACE_SKIP_X) t.x0++;
+        if (flags & FACE_SKIP_Y) t.y0++;
+        t.fast = (flags & FACE_FAST) != 0u;
     }
-    return tri_setup(a, b, c, P.width, P.height, t);
 }
 
 // One fragment of triangle t at tile-local pixel (lx, ly).
@@ -1066,22 +1245,19 @@ template <int TS, int RB>
 __device__ __forceinline__ void frag_resolve(TileLds<TS, RB>& L, const TriS& t, uint32_t lo, int xb, int yb, int lx, int ly,
                                              bool second) {
     float wx, wy, wz, z;
-    if (!tri_cover_fast(t, xb + lx, yb + ly, wx, wy, wz, z)) return;
+    if (!tri_cover(t, xb + lx, yb + ly, wx, wy, wz, z)) return;
     int i = (ly << TS) | lx;
-    if (!second) {
-        if (z != z) {
-            atomicMax(&L.nan_order[i], (0xFFFFFFFEu - lo) + 1u);
+    if (z != z || second) {
+        uint32_t order = 0xFFFFFFFEu - lo;
+        if (!second) {
+            atomicMax(&L.nan_order[i], order + 1u);
             L.nan_seen = 1;
             return;
         }
-        atomicMin((unsigned long long*)&L.key[i], ((uint64_t)depth_bits(z) << 32) | lo);
-    } else {
         uint32_t no = L.nan_order[i];
-        if (no == 0u || z != z) return;
-        uint32_t order = 0xFFFFFFFEu - lo;
-        if (order + 1u <= no) return;   // only fragments after the last NaN one
-        atomicMin((unsigned long long*)&L.key[i], ((uint64_t)depth_bits(z) << 32) | lo);
+        if (no == 0u || z != z || order + 1u <= no) return;   // only fragments after the last NaN one
     }
+    atomicMin((unsigned long long*)&L.key[i], ((uint64_t)depth_bits(z) << 32) | lo);
 }
 
 // A triangle staged in LDS by lane s of the sweep, with its candidate box.
@@ -1097,17 +1273,122 @@ __device__ __forceinline__ TriS staged_tri(const TileLds<TS, RB>& L, int s, uint
     x0 = box & 0xFF;
     y0 = (box >> 16) & 0xFF;
     wdt = (int)((box >> 8) & 0xFF) - x0 + 1;
-    npix = wdt * ((int)(box >> 24) - y0 + 1);
+    npix = wdt * ((int)((box >> 24) & 0x7F) - y0 + 1);
+    t.fast = (box >> 31) != 0u;
     return t;
 }
 
-// One sweep over the tile's bin: small triangles one per lane (in passes that
+// v, but unknown to the compiler, which would otherwise compute what follows
+// from it early and keep it in registers, or spill it, until then.
+__device__ __forceinline__ int fresh(int v) {
+    asm("" : "+v"(v));
+    return v;
+}
+
+// The same for a uniform pointer: its fields are loaded where they are used, not
+// together at the start, where they would not all fit in scalar registers.
+__device__ __forceinline__ const PassDesc& fresh(const PassDesc& P) {
+    const HANA_CONST_AS PassDesc* p = (const HANA_CONST_AS PassDesc*)&P;
+    asm("" : "+s"(p));
+    return *(const PassDesc*)p;
+}
+
+// A counter of the sequence (uniform; written by earlier launches of it only,
+// so read through the scalar cache).
+__device__ __forceinline__ uint32_t seq_count(const uint32_t* c, int i) { return *(const HANA_CONST_AS uint32_t*)(c + i); }
+
+// What a tile has to sweep: its chunks and its pass's wide triangles.
+struct TileBin {
+    const uint2* chunks;
+    const uint2* wide;      // boxes and entries
+    int nchunks, nwide;
+    int end;                // of the steps over the chunks: nchunks, or past whole 64s of them the list of the sequence
+    uint32_t tx, ty;        // the tile in the boxes' units
+};
+__device__ __forceinline__ bool wide_hits(const TileBin& B, uint32_t box) {
+    return B.tx >= (box & 0xFFu) && B.tx <= ((box >> 16) & 0xFFu) && B.ty >= ((box >> 8) & 0xFFu) && B.ty <= (box >> 24);
+}
+
+// Lists the wide triangles that touch the tile, from position w0 on (as many
+// as fit in L.list), and returns their number; the whole workgroup calls it.
+// (On a target of over 256 tiles a side a box may reach a little further than
+// its triangle, which the sweep then drops.)
+template <int TS, int RB>
+__device__ __forceinline__ uint32_t list_wide(TileLds<TS, RB>& L, const TileBin& B, uint32_t w0) {
+    const int wave = threadIdx.x >> 6;
+    uint32_t n = 0;
+    for (int i0 = 0; i0 < B.nwide; i0 += RB) {   // uniform
+        const int i = fresh(i0 + (int)threadIdx.x);
+        uint2 w = make_uint2(0u, 0u);
+        if (i < B.nwide) w = gld2(B.wide + i);
+        const bool hit = i < B.nwide && wide_hits(B, w.x);
+        const uint64_t m = __ballot(hit);
+        uint32_t* hits = L.hits[(i0 / RB) & 1];
+        if (__lane_id() == 0) hits[wave] = (uint32_t)__popcll(m);
+        lds_barrier();
+        uint32_t p = n + mask_rank(m) - w0;
+#pragma unroll
+        for (int k = 0; k < RB / 64; k++) {
+            uint32_t h = __builtin_amdgcn_readfirstlane(hits[k]);
+            if (k < wave) p += h;
+            n += h;
+        }
+        if (hit && p < TILE_LIST) L.list[p] = w.y;
+    }
+    return n;
+}
+
+// Lists the entries of the tile's chunks behind those, from position w0 on.
+// Every wave prefix-sums the descriptors, 64 at a time, one a lane, and copies
+// its share of the chunks, 4, 16 or 64 lanes to a chunk by their mean length,
+// so that no barrier stands between the descriptors and the entries' loads.
+// Where the tile's places were too few, the list of the sequence follows, with
+// the other tiles' descriptors counted as empty.  Returns the number of all
+// entries; a barrier must follow.
+template <int TS, int RB>
+__device__ __forceinline__ uint32_t list_chunks(TileLds<TS, RB>& L, const TileBin& B, const Workspace& ws, int gt,
+                                                uint32_t w0, uint32_t base) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    for (int g0 = 0; g0 < B.end; g0 += 64) {   // uniform
+        int nc = min(B.nchunks - g0, 64);
+        uint2 d;
+        if (__builtin_expect(nc > 0, 1)) {
+            d = gld2(B.chunks + g0 + min(lane, nc - 1));
+        } else {
+            nc = min(B.end - g0, 64);
+            const uint4 e = ws.over[g0 - ((B.nchunks + 63) & ~63) + min(lane, nc - 1)];
+            d = make_uint2(e.y, e.x == (uint32_t)gt ? e.z : 0u);
+        }
+        if (lane >= nc) d.y = 0u;
+        const uint32_t n = (d.y & CHUNK_INLINE) ? 1u : d.y;
+        const uint32_t incl = wave_scan(n), total = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
+        const uint32_t at = base + incl - n - w0;   // in the list; wraps before it
+        if (base < w0 + TILE_LIST && base + total > w0) {
+            const int sh = total > 24u * nc ? 6 : (total > 6u * nc ? 4 : 2);
+            for (int c0 = wave << (6 - sh); c0 < nc; c0 += (RB / 64) << (6 - sh)) {
+                const int c = c0 + (lane >> sh);
+                const uint32_t o = __shfl(d.x, c), y = __shfl(d.y, c), p = __shfl(at, c);
+                if (c >= nc) continue;
+                if (y & CHUNK_INLINE) {
+                    if ((lane & ((1 << sh) - 1)) == 0 && p < TILE_LIST) L.list[p] = o;
+                } else {
+                    for (uint32_t i = lane & ((1 << sh) - 1); i < y; i += 1u << sh)
+                        if (p + i < TILE_LIST) L.list[p + i] = gld(ws.bins + (o + i));
+                }
+            }
+        }
+        base += total;
+    }
+    return base;
+}
+
+// One sweep over the first cnt listed entries of the tile: small triangles one per lane (in passes that
 // share them, those of more than HANA_MED_PIX candidates HANA_MED_LANES lanes
 // each), larger ones one per wave with the lanes spread over their candidate
 // pixels.
 template <int TS, int RB>
-__device__ int sweep(TileLds<TS, RB>& L, const PassDesc& P, const Workspace& ws, uint32_t beg, uint32_t cnt, int xb, int yb,
-                     bool second, int set) {
+__device__ __forceinline__ int sweep(TileLds<TS, RB>& L, const PassDesc& P, uint32_t cnt, int xb, int yb,
+                                     bool second, int set) {
     constexpr int EDGE = 1 << TS;
     int tid = threadIdx.x, lane = tid & 63;
     for (uint32_t base = 0; base < cnt; base += RB) {
@@ -1115,7 +1396,10 @@ __device__ int sweep(TileLds<TS, RB>& L, const PassDesc& P, const Workspace& ws,
         bool ok = false;
         TriS t;
         uint32_t order = 0;
-        if (base + tid < cnt) ok = load_tri(P, ws, gld(ws.bins + (beg + base + tid)), t, order);
+        if (base + tid < cnt) {
+            load_tri(P, L.list[base + tid], t, order);
+            ok = true;
+        }
         int bx0 = 0, bx1 = -1, by0 = 0, by1 = -1;
         if (ok) {
             bx0 = max(t.x0, xb) - xb; bx1 = min(t.x1, xb + EDGE - 1) - xb;
@@ -1134,9 +1418,10 @@ __device__ int sweep(TileLds<TS, RB>& L, const PassDesc& P, const Workspace& ws,
                 L.s1x[tid] = t.s1x; L.s1y[tid] = t.s1y; L.uz[tid] = t.uz;
                 L.z0[tid] = t.z0; L.z1[tid] = t.z1; L.z2[tid] = t.z2;
                 L.lo[tid] = lo;
-                L.box[tid] = (uint32_t)bx0 | ((uint32_t)bx1 << 8) | ((uint32_t)by0 << 16) | ((uint32_t)by1 << 24);
-                if (npix <= SMALL_PIX) L.med[atomicAdd(&C[2], 1)] = tid;
-                else L.big[atomicAdd(&C[0], 1)] = tid;
+                L.box[tid] = (uint32_t)bx0 | ((uint32_t)bx1 << 8) | ((uint32_t)by0 << 16) | ((uint32_t)by1 << 24) |
+                             (t.fast ? 1u << 31 : 0u);
+                if (npix <= SMALL_PIX) L.med[atomicAdd(&C[2], 1)] = (uint8_t)tid;
+                else L.big[atomicAdd(&C[0], 1)] = (uint8_t)tid;
             }
         }
         __syncthreads();
@@ -1198,7 +1483,7 @@ __device__ __forceinline__ void load_varyings8(const float* row, float* y) {
 
 // Interpolates, shades and writes the winning fragment of one pixel
 // (interpolate_varyings + fragment + set_depth/set_color, SR/graphics.cpp:205-220, 362-373).
-__device__ __forceinline__ void shade_pixel(const PassDesc& P, const Workspace& ws, uint32_t order, int px, int py) {
+__device__ __forceinline__ void shade_pixel(const PassDesc& P, uint32_t order, int px, int py) {
     uint32_t f = order >> 4, slot = order & 15u;
     float4 va, vb, vc;
     const float *sa, *sb, *sc;
@@ -1211,6 +1496,7 @@ __device__ __forceinline__ void shade_pixel(const PassDesc& P, const Workspace& 
     } else {
         int pid = gld(P.poly_of_face + f);
         uint32_t j = slot - 1;
+        const Workspace& ws = raster_ws();
         size_t base = (size_t)pid * POLY_MAX;
         va = gld4(ws.pool_vr + base); vb = gld4(ws.pool_vr + base + j + 1); vc = gld4(ws.pool_vr + base + j + 2);
         nv = POLY_VARY;
@@ -1232,15 +1518,16 @@ __device__ __forceinline__ void shade_pixel(const PassDesc& P, const Workspace& 
         if (cnt == 2) { ya[1] = gld(sa + 1); yb[1] = gld(sb + 1); yc[1] = gld(sc + 1); }
     }
     TriS t;
-    tri_setup(va, vb, vc, P.width, P.height, t);
+    tri_edges(va, vb, vc, P.width, P.height, t);
+    t.fast = cover_is_fast(t);
     // The weights take the same quotients as the resolve.  Where a numerator
-    // is zero, tri_cover_fast may give a zero weight of the other sign than the
+    // is zero, tri_cover may give a zero weight of the other sign than the
     // division: wx = 1 - q is then 1 either way, and a zero wy or wz only adds
     // a signed zero beside the nonzero va.w * wx in the normaliser and in each
     // varying's sum, so no sum changes unless it is exactly zero, and then only
     // in the sign of that zero.  Depth is summed from +0 and does not change.
     float wx, wy, wz, z;
-    tri_cover_fast(t, px, py, wx, wy, wz, z);
+    tri_cover(t, px, py, wx, wy, wz, z);
     float k0 = va.w * wx, k1 = vb.w * wy, k2 = vc.w * wz;
     float normalizer = 1 / (k0 + k1 + k2);
     float vy[8];
@@ -1288,83 +1575,96 @@ __device__ __forceinline__ int xcd_logical_block(int b, int nb) {
     return ((slot / ch) * kXcd + xcd) * ch + slot % ch;
 }
 
-// Renders tile lt of pass P: the visibility of its pixels in LDS, then one
-// fragment program per covered pixel; a tile no triangle reaches only takes
-// the pass's clear.  The workgroup's threads all call it; it leaves L in use
-// until they have all returned.
+// Renders tile lt of pass P (global tile gt, of nchunks chunks): the
+// visibility of its pixels in LDS, then one fragment program per covered
+// pixel; a tile no triangle reaches only takes the pass's clear.  The
+// workgroup's threads all call it; it leaves L in use until they have all
+// returned.
 template <int TS, int RB>
-__device__ void raster_tile(TileLds<TS, RB>& L, const PassDesc& P, const Workspace& ws, int lt, uint32_t beg,
-                            uint32_t cnt) {
+__device__ void raster_tile(TileLds<TS, RB>& L, const PassDesc& P, const Workspace& ws, int lt, int gt, uint32_t nchunks,
+                            uint32_t nwide) {
     constexpr int EDGE = 1 << TS, PIX = 1 << (2 * TS);
     int tx = lt % P.tiles_x, ty = lt / P.tiles_x;
     int xb = tx << TS, yb = ty << TS;
     int tid = threadIdx.x;
     int W = P.width, H = P.height;
+    const int ws_shift = wide_shift(P);
+    TileBin B{ws.chunks + (size_t)gt * ws.chunk_cap, ws.wide + (size_t)P.index * ws.wide_cap,
+              (int)min(nchunks, ws.chunk_cap), (int)min(nwide, ws.wide_cap), 0, (uint32_t)(tx >> ws_shift),
+              (uint32_t)(ty >> ws_shift)};
+    B.end = B.nchunks;
+    if (__builtin_expect(nchunks > ws.chunk_cap, 0)) B.end = ((B.nchunks + 63) & ~63) + (int)min(seq_count(ws.seq, SEQ_OVER), ws.over_cap);
 
-    if (beg >= ws.bin_cap) cnt = 0;
-    else if (cnt > ws.bin_cap - beg) cnt = ws.bin_cap - beg;
-    if (cnt == 0) {   // uniform: no fragment, the clear only
-        for (int i = tid; i < PIX; i += RB) {
-            int px = xb + (i & (EDGE - 1)), py = yb + (i >> TS);
-            if (px >= W || py >= H) continue;
-            size_t pix = (size_t)py * W + px;
-            if (P.clear) {
-                gst(P.color + pix, P.clear_rgba);
-                gst(P.depth + pix, P.clear_depth);
+    // One copy of the code for every list of a long bin and for the second
+    // sweep after NaN fragments.  Every wave reads a round's entries ahead of
+    // the round's last barrier, so the next list may overwrite them.
+    bool first = true, second = false;
+    int set = 0;
+#pragma unroll 1
+    for (uint32_t w0 = 0;;) {
+        const uint32_t nw = list_wide<TS, RB>(L, B, w0);
+        if (nw + (uint32_t)B.nchunks == 0u) {   // uniform: no fragment, the clear only
+            const PassDesc& Q = fresh(P);
+            for (int i = fresh(tid); i < PIX; i += RB) {
+                int px = xb + (i & (EDGE - 1)), py = yb + (i >> TS);
+                if (px >= W || py >= H) continue;
+                size_t pix = (size_t)py * W + px;
+                if (Q.clear) {
+                    gst(Q.color + pix, Q.clear_rgba);
+                    gst(Q.depth + pix, Q.clear_depth);
+                }
+                if (Q.winner) gst(Q.winner + pix, NO_WINNER);
             }
-            if (P.winner) gst(P.winner + pix, NO_WINNER);
+            return;
         }
-        return;
-    }
-
-    for (int i = tid; i < PIX; i += RB) {
-        int px = xb + (i & (EDGE - 1)), py = yb + (i >> TS);
-        uint64_t k = ~0ull;
-        if (px < W && py < H) k = init_key(P.clear ? P.clear_depth : gld(P.depth + ((size_t)py * W + px)));
-        L.key[i] = k;
-        L.nan_order[i] = 0u;
-    }
-    if (tid < 12) (&L.cnt[0][0])[tid] = 0;
-    if (tid == 0) L.nan_seen = 0;
-    __syncthreads();
-
-    int set = sweep<TS, RB>(L, P, ws, beg, cnt, xb, yb, false, 0);
-
-    if (L.nan_seen) {
+        if (first) {
+            const PassDesc& Q = fresh(P);
+            for (int i = fresh(tid); i < PIX; i += RB) {
+                int px = xb + (i & (EDGE - 1)), py = yb + (i >> TS);
+                uint64_t k = ~0ull;
+                if (px < W && py < H) k = init_key(Q.clear ? Q.clear_depth : gld(Q.depth + ((size_t)py * W + px)));
+                L.key[i] = k;
+                L.nan_order[i] = 0u;
+            }
+            if (tid < 12) (&L.cnt[0][0])[tid] = 0;
+            if (tid == 0) L.nan_seen = 0;
+        }
+        const uint32_t n = list_chunks<TS, RB>(L, B, ws, gt, w0, nw);
+        first = false;
+        __syncthreads();
+        set = sweep<TS, RB>(L, P, min(n - w0, TILE_LIST), xb, yb, second, set);
+        w0 += TILE_LIST;
+        if (n > w0) continue;
+        if (second || !L.nan_seen) break;
         // pixels that saw a NaN-depth fragment restart after the last one
-        for (int i = tid; i < PIX; i += RB) {
+        for (int i = fresh(tid); i < PIX; i += RB) {
             uint32_t no = L.nan_order[i];
             if (no) L.key[i] = (0xFFFFFFFFull << 32) | (uint64_t)(0xFFFFFFFEu - (no - 1u));
         }
         __syncthreads();
-        sweep<TS, RB>(L, P, ws, beg, cnt, xb, yb, true, set);
+        second = true;
+        w0 = 0;
     }
 
     uint32_t written = 0;
-    for (int i = tid; i < PIX; i += RB) {
+    const PassDesc& Q = fresh(P);
+    for (int i = fresh(tid); i < PIX; i += RB) {
         int px = xb + (i & (EDGE - 1)), py = yb + (i >> TS);
         if (px >= W || py >= H) continue;
         uint32_t lo = (uint32_t)L.key[i];
         size_t pix = (size_t)py * W + px;
         if (lo == 0xFFFFFFFFu) {
-            if (P.clear) {
-                gst(P.color + pix, P.clear_rgba);
-                gst(P.depth + pix, P.clear_depth);
+            if (Q.clear) {
+                gst(Q.color + pix, Q.clear_rgba);
+                gst(Q.depth + pix, Q.clear_depth);
             }
-            if (P.winner) gst(P.winner + pix, NO_WINNER);
+            if (Q.winner) gst(Q.winner + pix, NO_WINNER);
             continue;
         }
-        shade_pixel(P, ws, 0xFFFFFFFEu - lo, px, py);
+        shade_pixel(Q, 0xFFFFFFFEu - lo, px, py);
         written++;
     }
-    if (P.stats) stat_add(P, ST_PIXELS, written);
-}
-
-// The bin range of global tile gt (uniform; written by earlier launches of
-// the sequence only, so read through the scalar cache).
-__device__ __forceinline__ uint2 tile_range(const Workspace& ws, int gt) {
-    return make_uint2(*(const HANA_CONST_AS uint32_t*)(ws.tile_offset + gt),
-                      *(const HANA_CONST_AS uint32_t*)(ws.tile_count + gt));
+    if (Q.stats) stat_add(Q, ST_PIXELS, written);
 }
 
 // Waves per SIMD that the raster's LDS allows (160 KiB per CU, 4 SIMDs, at
@@ -1408,17 +1708,14 @@ __global__ __launch_bounds__(RB) __attribute__((amdgpu_waves_per_eu(raster_occup
 void k_raster(const PassDesc* __restrict__ passes, int npasses, Workspace ws) {
     __shared__ TileLds<TS, RB> L;
     // the loads that decide the workgroup's work are issued before any of
-    // them is awaited: the sequence flags, the pass lookup, the bin range
-    uint32_t flags = *(const HANA_CONST_AS uint32_t*)(ws.status + STATUS_SEQ_FLAGS);
+    // them is awaited: the pass lookup, the tile's chunks, the sequence's totals
     int blk = xcd_logical_block(blockIdx.x, gridDim.x);
     int gt;
     const PassDesc& P = passes[raster_pass<GROUP>(passes, npasses, ws, blk, gt)];
-    uint2 range = tile_range(ws, gt);
-    // an incomplete sequence leaves its targets untouched: the host renders it
-    // again.  (Bin offsets never reach 2^32 - 1; testing the range as well
-    // keeps its loads ahead of the flags' wait.)
-    if ((flags & FLAG_NO_RASTER) | (uint32_t)((range.x & range.y) == 0xFFFFFFFFu)) return;
-    raster_tile<TS, RB>(L, P, ws, blk - P.tblock0, range.x, range.y);
+    uint32_t nchunks = seq_count(ws.tile_chunks, gt), nwide = seq_count(ws.wide_count, P.index);
+    // an incomplete sequence leaves its targets untouched: the host renders it again
+    if (!sequence_fits(ws, blockIdx.x == 0 && threadIdx.x == 0)) return;
+    raster_tile<TS, RB>(L, P, ws, blk - P.tblock0, gt, nchunks, nwide);
 }
 
 // The persistent raster: a fixed grid of workgroups takes the tiles of every
@@ -1456,12 +1753,12 @@ __global__ __launch_bounds__(RB) __attribute__((amdgpu_waves_per_eu(raster_occup
 void k_raster_q(const PassDesc* __restrict__ passes, int npasses, Workspace ws) {
     __shared__ TileLds<TS, RB> L;
     __shared__ uint32_t s_first;
-    if (ws.status[STATUS_SEQ_FLAGS] & FLAG_NO_RASTER) return;
+    if (!sequence_fits(ws, blockIdx.x == 0 && threadIdx.x == 0)) return;
     const int tid = threadIdx.x;
     uint32_t mine = 0;   // shadow tiles finished here, not yet published
     bool published = false, ready = false;
     for (;;) {
-        if (tid == 0) s_first = atomicAdd(&ws.qstate[0], RQ_CHUNK);
+        if (tid == 0) s_first = atomicAdd(&ws.seq[SEQ_QUEUE], RQ_CHUNK);
         __syncthreads();
         // uniform: the tile's pass, bounds and tables then live in SGPRs
         uint32_t first = __builtin_amdgcn_readfirstlane(s_first);
@@ -1469,20 +1766,20 @@ void k_raster_q(const PassDesc* __restrict__ passes, int npasses, Workspace ws) 
         uint32_t end = min(first + RQ_CHUNK, ws.q_items);
         if (!published && (first >= ws.q_g0 || first >= ws.q_items)) {
             if (tid == 0 && mine)
-                __hip_atomic_fetch_add(&ws.qstate[1], mine, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+                __hip_atomic_fetch_add(&ws.seq[SEQ_QUEUE_DONE], mine, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
             published = true;
         }
         if (first >= ws.q_items) break;
         for (uint32_t it = first; it < end; it++) {
             if (!published && it >= ws.q_g0) {
                 if (tid == 0 && mine)
-                    __hip_atomic_fetch_add(&ws.qstate[1], mine, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+                    __hip_atomic_fetch_add(&ws.seq[SEQ_QUEUE_DONE], mine, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
                 published = true;
             }
             if (!ready && it >= ws.q_dep_from) {
                 if (tid == 0) {
                     uint32_t spins = 0;
-                    while (__hip_atomic_load(&ws.qstate[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < ws.q_g0) {
+                    while (__hip_atomic_load(&ws.seq[SEQ_QUEUE_DONE], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < ws.q_g0) {
                         if (++spins > RQ_SPIN_LIMIT) {
                             raise_flag(ws, FLAG_QUEUE_STALL);
                             break;
@@ -1495,8 +1792,8 @@ void k_raster_q(const PassDesc* __restrict__ passes, int npasses, Workspace ws) 
                 ready = true;
             }
             const PassDesc& P = passes[pass_of_item(passes, npasses, it)];
-            uint2 range = tile_range(ws, (int)it);
-            raster_tile<TS, RB>(L, P, ws, (int)(it - (uint32_t)P.tile0), range.x, range.y);
+            raster_tile<TS, RB>(L, P, ws, (int)(it - (uint32_t)P.tile0), (int)it, seq_count(ws.tile_chunks, (int)it),
+                                seq_count(ws.wide_count, P.index));
             __syncthreads();   // the tile's writes are issued and L is free again
             if (it < ws.q_g0) mine++;
         }
@@ -1529,8 +1826,8 @@ __global__ void k_present(const uint32_t* __restrict__ src, uint32_t* __restrict
 
 hipError_t launch_vertex(const PassDesc* d_passes, int npasses, const Workspace& ws, int blocks, hipStream_t s) {
     if (npasses <= 0) return hipSuccess;
-    // k_vertex also zeroes the tile counters and the status words of the
-    // sequence, so it runs even when no pass has a vertex
+    // k_vertex also zeroes the sequence's counters, so it runs even when no
+    // pass has a vertex
     blocks = std::max(blocks, 1);
     hipLaunchKernelGGL(k_vertex, dim3(blocks), dim3(BLOCK), 0, s, d_passes, npasses, ws);
     return hipGetLastError();
@@ -1549,28 +1846,24 @@ hipError_t launch_setup(const PassDesc* d_passes, int npasses, const Workspace& 
 }
 hipError_t launch_clip(const PassDesc* d_passes, const Workspace& ws, hipStream_t s) {
     // grid-stride: the queue length is only known on the device
-    if (ws.tile_shift == 5) hipLaunchKernelGGL(k_clip<5>, dim3(2048), dim3(CLIP_THREADS), 0, s, d_passes, ws);
-    else hipLaunchKernelGGL(k_clip<4>, dim3(2048), dim3(CLIP_THREADS), 0, s, d_passes, ws);
+    if (ws.tile_shift == 5) hipLaunchKernelGGL(k_clip<5>, dim3(CLIP_GRID), dim3(CLIP_THREADS), 0, s, d_passes, ws);
+    else hipLaunchKernelGGL(k_clip<4>, dim3(CLIP_GRID), dim3(CLIP_THREADS), 0, s, d_passes, ws);
     return hipGetLastError();
 }
-int scan_chunks(int ntiles) { return ntiles > 0 ? (ntiles + SCAN_CHUNK - 1) / SCAN_CHUNK : 1; }
-hipError_t launch_scan(const Workspace& ws, hipStream_t s) {
-    int chunks = scan_chunks(ws.ntiles);
-    if (chunks > 1) {
-        hipLaunchKernelGGL(k_scan_reduce, dim3(chunks), dim3(SCAN_THREADS), 0, s, ws);
-        hipError_t e = hipGetLastError();
-        if (e != hipSuccess) return e;
+hipError_t launch_front(const FrontTables* tables, PassDesc* d_passes, DevUniforms* d_unis, int npasses, const Workspace& ws,
+                        int fblocks, int vblocks, hipStream_t s) {
+    static const FrontTables none{};
+    if (npasses <= 0) return hipSuccess;
+    // the last workgroup stores the tables, so one runs even for empty meshes
+    dim3 grid(std::max(fblocks + vblocks, 1)), block(BLOCK);
+    const FrontTables& t = tables ? *tables : none;
+    if (ws.tile_shift == 5) {
+        if (tables) hipLaunchKernelGGL((k_front<5, true>), grid, block, 0, s, t, d_passes, d_unis, npasses, ws, fblocks);
+        else hipLaunchKernelGGL((k_front<5, false>), grid, block, 0, s, t, d_passes, d_unis, npasses, ws, fblocks);
+    } else {
+        if (tables) hipLaunchKernelGGL((k_front<4, true>), grid, block, 0, s, t, d_passes, d_unis, npasses, ws, fblocks);
+        else hipLaunchKernelGGL((k_front<4, false>), grid, block, 0, s, t, d_passes, d_unis, npasses, ws, fblocks);
     }
-    hipLaunchKernelGGL(k_scan_apply, dim3(chunks), dim3(SCAN_THREADS), 0, s, ws);
-    return hipGetLastError();
-}
-hipError_t launch_bin(const PassDesc* d_passes, const Workspace& ws, int nseg, bool small_tris, hipStream_t s) {
-    // one workgroup per setup segment, then a grid-stride tail for the
-    // clipped fan triangles (their count is only known on the device)
-    if (small_tris)
-        hipLaunchKernelGGL(k_bin<9>, dim3(nseg + 512), dim3(BLOCK), 0, s, d_passes, ws, nseg);
-    else
-        hipLaunchKernelGGL(k_bin<11>, dim3(nseg + 512), dim3(BLOCK), 0, s, d_passes, ws, nseg);
     return hipGetLastError();
 }
 template <int TS, int RB>

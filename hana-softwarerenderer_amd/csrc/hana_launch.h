@@ -10,10 +10,10 @@ hipError_t launch_vertex(const PassDesc* d_passes, int npasses, const Workspace&
 hipError_t launch_setup(const PassDesc* d_passes, int npasses, const Workspace& ws, int blocks, bool small_tris,
                         hipStream_t s);
 hipError_t launch_clip(const PassDesc* d_passes, const Workspace& ws, hipStream_t s);
-int scan_chunks(int ntiles);
-hipError_t launch_scan(const Workspace& ws, hipStream_t s);
-// small_tris: every pass averages at most 4 pixels per face (smaller tile table)
-hipError_t launch_bin(const PassDesc* d_passes, const Workspace& ws, int nseg, bool small_tris, hipStream_t s);
+// vertex, set-up and clipping in one launch; `tables` (or null: they are in
+// device memory already) come with it and are stored at d_passes and d_unis
+hipError_t launch_front(const FrontTables* tables, PassDesc* d_passes, DevUniforms* d_unis, int npasses, const Workspace& ws,
+                        int fblocks, int vblocks, hipStream_t s);
 // one workgroup per tile of dependency group `group` (ws.tile_shift selects the tile size)
 hipError_t launch_raster(const PassDesc* d_passes, int npasses, const Workspace& ws, int blocks, int group,
                          hipStream_t s);

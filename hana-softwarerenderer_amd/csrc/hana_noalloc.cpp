@@ -145,6 +145,7 @@ extern "C" int hana_render_frame_noalloc(hana_ctx* c, const hana_frame_desc* f) 
         tile0 += d.tiles_x * d.tiles_y;
         d.tblock0 = tb[s.group];
         tb[s.group] += d.tiles_x * d.tiles_y;
+        d.index = i;
         if (!group_count[s.group]) group_first[s.group] = i;
         group_count[s.group]++;
         // clears fuse into the first pass writing the target
@@ -155,52 +156,95 @@ extern "C" int hana_render_frame_noalloc(hana_ctx* c, const hana_frame_desc* f) 
         }
     }
 
+    // The frames that fit are fixed by a nominal size, so that callers can rely
+    // on it whatever the layout below needs: 12 bytes per tile, the vertices'
+    // and faces' arrays, 28 KiB (24 in passes of small triangles) per 1,024
+    // faces, the clip pool and, at least, four bin entries per face and two
+    // per tile.
+    const size_t ntiles = (size_t)std::max(tile0, 1), segs = std::max<size_t>(fb, 1);
+    const uint64_t poly_cap = std::min<uint64_t>(tf / 256 + 1024, POOL_CAP_MAX);
+    {
+        Carver nom{nullptr, 0, kNoAllocScratchBytes};
+        nom.take<char>(2 * 264);
+        nom.take<DevUniforms>(2);
+        nom.take<uint32_t>(9);
+        nom.take<uint32_t>(2);
+        for (int k = 0; k < 3; k++) nom.take<uint32_t>((size_t)tile0 + 1);
+        nom.take<uint64_t>(((size_t)tile0 + 4095) / 4096);
+        nom.take<float4>(tv);
+        nom.take<float>(tvs);
+        nom.take<uint8_t>(tv);
+        nom.take<int32_t>(tf);
+        nom.take<uint32_t>(segs);
+        nom.take<uint2>(segs * (small_tris ? 512 : 1024));
+        nom.take<uint16_t>(segs * 1024);
+        nom.take<uint32_t>(segs);
+        nom.take<uint64_t>(std::max<size_t>(tf, 1024));
+        nom.take<float4>(POLY_MAX * poly_cap);
+        nom.take<float>(POLY_MAX * POLY_VARY * poly_cap);
+        for (int k = 0; k < 3; k++) nom.take<int32_t>(poly_cap);
+        nom.take<uint4>((size_t)fb * 1024 + 8 * poly_cap);
+        size_t words = nom.fits() ? (kNoAllocScratchBytes - nom.off) / sizeof(uint32_t) : 0;
+        if (!nom.fits() || words < 64 + 4 * tf + 2 * ((size_t)tile0 + 1))
+            return fail(c, HANA_E_NOMEM,
+                        "hana_render_frame_noalloc: the frame needs more workspace than the " +
+                            std::to_string(kNoAllocScratchBytes >> 20) + " MiB no-alloc scratch holds; use hana_render_frame");
+    }
+
     // the workspace, carved from the scratch array
     Carver cv{static_cast<char*>(c->scratch), 0, kNoAllocScratchBytes};
-    const size_t ntiles = (size_t)tile0 + 1, nsegs = (size_t)std::max(fb, 1);
-    const uint32_t seg_stride = small_tris ? 512u : 1024u;
-    const uint64_t poly_cap = std::min<uint64_t>(tf / 256 + 1024, POOL_CAP_MAX);
-    const uint64_t seg_region = (uint64_t)fb * BLOCK * FPT;
-    const uint64_t tris_cap = seg_region + 8 * poly_cap;
     PassDesc* d_desc = cv.take<PassDesc>(2);
     DevUniforms* d_uni = cv.take<DevUniforms>(2);
     Workspace ws{};
     ws.status = cv.take<uint32_t>(STATUS_WORDS);
-    ws.qstate = cv.take<uint32_t>(2);
-    ws.tile_count = cv.take<uint32_t>(ntiles);
-    ws.tile_offset = cv.take<uint32_t>(ntiles);
-    ws.tile_cursor = cv.take<uint32_t>(ntiles);
-    ws.scan_part = cv.take<uint64_t>((size_t)scan_chunks(tile0));
+    const size_t counters = (size_t)SEQ_WORDS + 4 + ((ntiles + 3) & ~(size_t)3);
+    ws.seq = cv.take<uint32_t>(counters);
     float4* vr = cv.take<float4>(tv);
     float* vs = cv.take<float>(tvs);
     uint8_t* code = cv.take<uint8_t>(tv);
     int32_t* pof = cv.take<int32_t>(tf);
-    ws.seg_count = cv.take<uint32_t>(nsegs);
-    ws.seg_tiles = cv.take<uint2>(nsegs * seg_stride);
-    ws.seg_wide = cv.take<uint16_t>(nsegs * BLOCK * FPT);
-    ws.seg_info = cv.take<uint32_t>(nsegs);
+    // every wide triangle is listed: a descriptor in each of its tiles would
+    // take more than the bin entry there that the nominal size counts
+    const size_t wide_cap = (size_t)f->mesh->F + 8 * poly_cap;
+    ws.wide = cv.take<uint2>(wide_cap * n);
     ws.clip_queue = cv.take<uint64_t>(std::max<size_t>(tf, 1024));
     ws.pool_vr = cv.take<float4>(POLY_MAX * poly_cap);
     ws.pool_vs = cv.take<float>(POLY_MAX * POLY_VARY * poly_cap);
     ws.pool_face = cv.take<int32_t>(poly_cap);
-    ws.pool_pass = cv.take<int32_t>(poly_cap);
-    ws.pool_n = cv.take<int32_t>(poly_cap);
-    ws.tris = cv.take<uint4>(tris_cap);
-    // the bins take what is left, at least four entries per face
+    // of what is left, the set-up workgroups' own bin entries and beside them
+    // as many as the nominal size counts (narrow triangles have at most 16
+    // each), then of the spare words half for the tiles' chunk descriptors, or
+    // a quarter where that is more than an allocated workspace starts with
+    // (bind_plan), and a quarter for the list behind them
+    const uint64_t seg_region = (uint64_t)fb * SEG_PAIRS * BLOCK * FPT;
+    const size_t min_bins = (size_t)seg_region + std::min(16 * tf, 4 * tf + 2 * ((size_t)tile0 + 1)) + 64;
     size_t left = cv.fits() ? (kNoAllocScratchBytes - cv.off) / sizeof(uint32_t) : 0;
-    size_t bins_cap = std::min<size_t>(left > 64 ? left - 64 : 0, MAX_PAIRS);
-    ws.bins = bins_cap ? cv.take<uint32_t>(bins_cap) : nullptr;
-    if (!cv.fits() || !ws.bins || bins_cap < 4 * tf + 2 * ntiles || tris_cap > 0xFFFFFFF0ull)
-        return fail(c, HANA_E_NOMEM,
-                    "hana_render_frame_noalloc: the frame needs more workspace than the " +
-                        std::to_string(kNoAllocScratchBytes >> 20) + " MiB no-alloc scratch holds; use hana_render_frame");
-    ws.ntiles = tile0;
+    left = left > 256 ? left - 256 : 0;
+    const size_t spare = left > min_bins ? left - min_bins : 0;
+    const size_t per_face = tf / ntiles + 1;
+    const size_t want_cap = std::max<size_t>(std::min<size_t>(8 * per_face, std::max<size_t>(512, 2 * per_face)), 64) + CHUNK_SLACK;
+    size_t cap = std::min(spare / 4 / ntiles, std::max(want_cap, spare / 8 / ntiles));
+    if (cap >= 8) cap = 4 * (cap / 4 - 1 + (cap / 4 & 1));   // an odd number of 32-byte groups
+    cap = std::max<size_t>(cap, 1);
+    const size_t over_cap = spare > 2 * cap * ntiles ? std::min(spare / 4, spare - 2 * cap * ntiles) / 4 : 0;
+    ws.chunks = cv.take<uint2>(cap * ntiles);
+    ws.chunk_cap = (uint32_t)cap;
+    ws.over = cv.take<uint4>(over_cap);
+    ws.over_cap = (uint32_t)over_cap;
+    ws.wide_cap = (uint32_t)wide_cap;
+    left = cv.fits() ? (kNoAllocScratchBytes - cv.off) / sizeof(uint32_t) : 0;
+    const size_t bins_cap = std::min<size_t>(left, MAX_PAIRS);
+    ws.bins = bins_cap > seg_region ? cv.take<uint32_t>(bins_cap) : nullptr;
+    if (!cv.fits() || !ws.bins || !ws.chunks)
+        return fail(c, HANA_E_NOMEM, "internal error: a frame of nominal size does not fit the no-alloc scratch");
+    ws.wide_count = ws.seq + SEQ_WORDS;
+    ws.tile_chunks = ws.wide_count + 4;
+    ws.zero = ws.seq;
+    ws.zero_n = (uint32_t)counters;
     ws.bin_cap = (uint32_t)bins_cap;
+    ws.seg_region = (uint32_t)seg_region;
     ws.poly_cap = (uint32_t)poly_cap;
     ws.clipq_cap = (uint32_t)std::max<size_t>(tf, 1024);
-    ws.tris_cap = (uint32_t)tris_cap;
-    ws.seg_region = (uint32_t)seg_region;
-    ws.seg_stride = seg_stride;
     ws.status_out = c->noalloc_status_dev;
     ws.q_items = (uint32_t)tile0;
     ws.q_g0 = (uint32_t)tb[0];
@@ -232,8 +276,6 @@ extern "C" int hana_render_frame_noalloc(hana_ctx* c, const hana_frame_desc* f) 
     NA_TRY(launch_vertex(d_desc, n, ws, vb, s));
     NA_TRY(launch_setup(d_desc, n, ws, fb, small_tris, s));
     NA_TRY(launch_clip(d_desc, ws, s));
-    NA_TRY(launch_scan(ws, s));
-    NA_TRY(launch_bin(d_desc, ws, fb, small_tris, s));
     if (c->tuning.raster_wgs_per_cu > 0) {
         NA_TRY(launch_raster_queue(d_desc, n, ws, c->tuning.raster_wgs_per_cu * c->num_cus, s));
     } else {

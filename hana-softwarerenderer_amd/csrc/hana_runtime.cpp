@@ -4,10 +4,10 @@
 // A pass is one graphics_draw_triangle call (SR/graphics.cpp:378-407).  A
 // frame is DrawModel::draw (SR/scene.h:53-99): an optional shadow pass into
 // the shadow map, the main pass sampling it, then the shadow-map clear.  Any
-// set of passes is rendered by one launch sequence of five kernels over
-// per-pass descriptor tables (vertex, setup-count, scan, setup-scatter,
-// raster per dependency group), so a single frame and a batch of hundreds of
-// frames run the same code; batches are captured once into a hipGraph.
+// set of passes is rendered by one launch sequence over per-pass descriptor
+// tables (geometry in one launch or three, then the raster of each dependency
+// group), so a single frame and a batch of hundreds of frames run the same
+// code; batches are captured once into a hipGraph.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -70,14 +70,19 @@ static std::vector<hana_target*> touched_targets(const std::vector<PassSpec>& sp
             if (x && std::find(t.begin(), t.end(), x) == t.end()) t.push_back(x);
     return t;
 }
-static bool shares_target(const std::vector<hana_target*>& a, const std::vector<hana_target*>& b) {
-    for (hana_target* x : a)
-        if (std::find(b.begin(), b.end(), x) != b.end()) return true;
+// Whether a call on slot a that touches targets t must wait for slot k: only
+// for the calls that touched one of them last (each waited for the ones before
+// it), unless slot a's stream has waited for them already.
+static bool must_wait(const hana_ctx* c, int k, int a, const std::vector<hana_target*>& t) {
+    const std::vector<hana_target*>& pend = c->pend[k][a];
+    for (hana_target* x : t)
+        if (x->slot == k && std::find(pend.begin(), pend.end(), x) != pend.end()) return true;
     return false;
 }
 // Notes work on slot k's stream, complete at slot_done[k], that touches
 // targets t, for every other slot to wait for before it touches them.
 static void note_pending(hana_ctx* c, int k, const std::vector<hana_target*>& t) {
+    for (hana_target* x : t) x->slot = k;
     for (int b = 0; b < c->nslots; b++)
         if (b != k)
             for (hana_target* x : t)
@@ -150,6 +155,11 @@ int build_plan(hana_ctx* c, std::vector<PassSpec> specs, Plan& pl, const Tuning&
     const int tshift = tu.tile_shift, tedge = tile_edge(tu.tile_shift);
     pl.specs = specs;
     int n = (int)specs.size();
+    size_t faces = 0;
+    for (const PassSpec& s : specs) faces += (size_t)s.mesh->F;
+    pl.front = faces <= kFrontFaces;
+    pl.args = pl.front && n <= FRONT_PASSES;
+    const size_t vchunk = (size_t)BLOCK * (pl.front ? FRONT_VPT : VPT), fchunk = (size_t)BLOCK * (pl.front ? FRONT_FPT : FPT);
     pl.descs.resize(n);
     pl.unis.resize(n);
     size_t voff = 0, vsoff = 0, fo = 0;
@@ -188,7 +198,6 @@ int build_plan(hana_ctx* c, std::vector<PassSpec> specs, Plan& pl, const Tuning&
         d.tiles_y = (t->h + tedge - 1) / tedge;
         d.share_small = (int64_t)t->w * t->h > 4 * (int64_t)m->F;
         if (d.share_small) pl.small_tris = false;
-        const size_t vchunk = (size_t)BLOCK * VPT, fchunk = (size_t)BLOCK * FPT;
         size_t vpad = (V + vchunk - 1) / vchunk * vchunk;
         // slices: pointers are resolved by bind_plan once the arena exists
         pl.v_off.push_back(voff);
@@ -205,6 +214,7 @@ int build_plan(hana_ctx* c, std::vector<PassSpec> specs, Plan& pl, const Tuning&
         tile0 += d.tiles_x * d.tiles_y;
         d.tblock0 = tb[s.group];
         tb[s.group] += d.tiles_x * d.tiles_y;
+        d.index = i;
     }
     pl.vblocks = vb;
     pl.fblocks = fb;
@@ -233,7 +243,7 @@ int build_plan(hana_ctx* c, std::vector<PassSpec> specs, Plan& pl, const Tuning&
     // passes are contiguous, in tblock0 order): one scalar load per workgroup
     // instead of a binary search over the group's descriptors
     pl.tile_pass.clear();
-    for (int g = 0; g < 2; g++) {
+    for (int g = 0; g < 2 && !pl.args; g++) {
         pl.tp_first[g] = (int)pl.tile_pass.size();
         const int first = pl.group_first[g], cnt = pl.group_count[g], nb = pl.group_blocks[g];
         const int run = 1 << TILE_PASS_SHIFT;
@@ -249,9 +259,42 @@ int build_plan(hana_ctx* c, std::vector<PassSpec> specs, Plan& pl, const Tuning&
     return HANA_OK;
 }
 
+// Words of a sequence's counters: the SEQ_* words, the passes' wide triangles,
+// the tiles' chunks.
+static size_t counter_words(const Plan& pl) {
+    return (size_t)SEQ_WORDS + ((pl.descs.size() + 3) & ~(size_t)3) + (((size_t)pl.total_tiles + 3) & ~(size_t)3);
+}
+
+// Points the plan's workspace at counter set k of the arena.
+static void set_counters(Plan& pl, Arena& A, int k) {
+    Workspace& ws = pl.ws;
+    ws.seq = A.counters[k].as<uint32_t>();
+    ws.wide_count = ws.seq + SEQ_WORDS;
+    ws.tile_chunks = ws.wide_count + ((pl.descs.size() + 3) & ~(size_t)3);
+}
+
+// Per-call sequences: the arena's next counter set, which the call before left
+// zeroed, with the other one to be zeroed by this call's first launch.
+static int take_counters(hana_ctx* c, Plan& pl, Arena& A, hipStream_t s) {
+    const int k = A.counters_next;
+    if (A.counters_used[k]) {   // a call before failed to launch
+        HIP_TRY(c, launch_fill32(A.counters[k].as<uint32_t>(), 0u, A.counters_used[k], s));
+        A.counters_used[k] = 0;
+    }
+    set_counters(pl, A, k);
+    pl.ws.zero = A.counters[k ^ 1].as<uint32_t>();
+    pl.ws.zero_n = (uint32_t)A.counters_used[k ^ 1];
+    A.counters_used[k] = counter_words(pl);
+    return HANA_OK;
+}
+static void counters_launched(Arena& A) {
+    A.counters_used[A.counters_next ^ 1] = 0;
+    A.counters_next ^= 1;
+}
+
 // Allocates the arena for a plan and resolves the slice pointers.
-int bind_plan(hana_ctx* c, Plan& pl, Arena& A, uint32_t min_bins, uint32_t min_polys, uint32_t min_tris,
-              bool with_stats, hipStream_t s) {
+int bind_plan(hana_ctx* c, Plan& pl, Arena& A, uint32_t min_bins, uint32_t min_polys, bool with_stats,
+              hipStream_t s) {
     int n = (int)pl.descs.size();
     int r;
     pl.uni_off = (sizeof(PassDesc) * std::max(n, 1) + 255) & ~(size_t)255;
@@ -262,51 +305,53 @@ int bind_plan(hana_ctx* c, Plan& pl, Arena& A, uint32_t min_bins, uint32_t min_p
     if ((r = ensure(c, A.code, std::max<size_t>(pl.total_v, 4)))) return r;
     if ((r = ensure(c, A.pof, sizeof(int32_t) * std::max<size_t>(pl.total_f, 1)))) return r;
     size_t nt = (size_t)pl.total_tiles + 1;
-    if ((r = ensure(c, A.tile_count, sizeof(uint32_t) * nt))) return r;
-    if ((r = ensure(c, A.tile_offset, sizeof(uint32_t) * nt))) return r;
-    if ((r = ensure(c, A.tile_cursor, sizeof(uint32_t) * nt))) return r;
-    if ((r = ensure(c, A.scan_part, sizeof(uint64_t) * (size_t)scan_chunks(pl.total_tiles)))) return r;
     // (triangle, tile) entries: most triangles touch one tile and about half
-    // are culled; the scan reports the exact need if this is exceeded
-    uint64_t want_bins = std::max<uint64_t>({(uint64_t)min_bins, (uint64_t)4 * pl.total_f + 2 * nt, 1u << 22});
+    // are culled; the raster reports the exact need if this is exceeded
+    const uint64_t seg_region = (uint64_t)pl.fblocks * SEG_PAIRS * BLOCK * (pl.front ? FRONT_FPT : FPT);
+    uint64_t want_bins = std::max<uint64_t>({(uint64_t)min_bins, (uint64_t)4 * pl.total_f + 2 * nt, 1u << 22,
+                                             seg_region + (uint64_t)pl.total_f + 4096});
+    if (seg_region + 4096 > MAX_PAIRS) return fail(c, HANA_E_NOMEM, "launch sequence too large (triangle list)");
     want_bins = std::min<uint64_t>(want_bins, MAX_PAIRS);
     if (want_bins > A.bin_cap) {
         if ((r = ensure(c, A.bins, sizeof(uint32_t) * want_bins))) return r;
         A.bin_cap = (uint32_t)want_bins;
     }
+    // chunk descriptors: a tile has one per set-up workgroup whose faces touch
+    // it.  Meshes whose neighbouring faces follow one another need a few
+    // dozen; eight per face over all tiles hold even scattered ones, and
+    // beyond 512 a tile two per face do
+    const uint64_t tiles = (uint64_t)std::max(pl.total_tiles, 1), per_face = pl.total_f / tiles + 1;
+    uint64_t want_cap = std::min<uint64_t>(8 * per_face, std::max<uint64_t>(512, 2 * per_face));
+    want_cap = std::max<uint64_t>(want_cap, tiles > (1u << 20) ? 16 : 64) + CHUNK_SLACK;
+    uint64_t want_slots = tiles * want_cap;
+    if (want_slots > A.chunk_slots) {
+        if ((r = ensure(c, A.chunks, sizeof(uint2) * want_slots))) return r;
+        A.chunk_slots = want_slots;
+    }
+    A.over_cap = std::max(A.over_cap, OVER_MIN);
+    if ((r = ensure(c, A.over, sizeof(uint4) * A.over_cap))) return r;
+    if ((r = ensure(c, A.wide, sizeof(uint2) * A.wide_cap * std::max(n, 1)))) return r;
     uint64_t want_polys = std::max<uint64_t>({(uint64_t)min_polys, pl.total_f / 16 + 4096});
     want_polys = std::min<uint64_t>(want_polys, POOL_CAP_MAX);
     if (want_polys > A.poly_cap) {
         if ((r = ensure(c, A.pool_vr, sizeof(float4) * POLY_MAX * want_polys))) return r;
         if ((r = ensure(c, A.pool_vs, sizeof(float) * POLY_MAX * POLY_VARY * want_polys))) return r;
         if ((r = ensure(c, A.pool_face, sizeof(int32_t) * want_polys))) return r;
-        if ((r = ensure(c, A.pool_pass, sizeof(int32_t) * want_polys))) return r;
-        if ((r = ensure(c, A.pool_n, sizeof(int32_t) * want_polys))) return r;
         A.poly_cap = (uint32_t)want_polys;
     }
-    // listed triangles: a segment of BLOCK*FPT records per k_setup workgroup,
-    // then at most eight fan triangles per clipped polygon
-    uint64_t seg_region = (uint64_t)pl.fblocks * BLOCK * FPT;
-    uint64_t want_tris = seg_region + std::max<uint64_t>({(uint64_t)min_tris, 8ull * A.poly_cap, 1024});
-    if (want_tris > 0xFFFFFFF0ull) return fail(c, HANA_E_NOMEM, "launch sequence too large (triangle list)");
-    if (want_tris > A.tris_cap) {
-        if ((r = ensure(c, A.tris, sizeof(uint4) * want_tris))) return r;
-        A.tris_cap = (uint32_t)want_tris;
-    }
-    if ((r = ensure(c, A.seg_count, sizeof(uint32_t) * std::max(pl.fblocks, 1)))) return r;
-    // k_setup's per-segment tile lists, as long as its LDS table (launch_setup)
-    uint32_t seg_stride = pl.small_tris ? 512u : 1024u;
-    size_t nsegs = (size_t)std::max(pl.fblocks, 1);
-    if ((r = ensure(c, A.seg_tiles, sizeof(uint2) * seg_stride * nsegs))) return r;
-    if ((r = ensure(c, A.seg_wide, sizeof(uint16_t) * BLOCK * FPT * nsegs))) return r;
-    if ((r = ensure(c, A.seg_info, sizeof(uint32_t) * nsegs))) return r;
-    if ((r = ensure(c, A.qstate, 256))) return r;
     // every face may fail the trivial accept (camera inside the mesh)
     uint64_t want_q = std::max<uint64_t>(pl.total_f, 1024);
     want_q = std::min<uint64_t>(want_q, 0xFFFFFFF0ull);
     if (want_q > A.clipq_cap) {
         if ((r = ensure(c, A.clip_queue, sizeof(uint64_t) * want_q))) return r;
         A.clipq_cap = (uint32_t)want_q;
+    }
+    for (int k = 0; k < 2; k++) {
+        const size_t bytes = sizeof(uint32_t) * counter_words(pl);
+        if (bytes <= A.counters[k].cap) continue;
+        if ((r = ensure(c, A.counters[k], bytes))) return r;
+        HIP_TRY(c, launch_fill32(A.counters[k].as<uint32_t>(), 0u, A.counters[k].cap / sizeof(uint32_t), s));
+        A.counters_used[k] = 0;
     }
     bool fresh_status = A.status.p == nullptr;
     if ((r = ensure(c, A.status, sizeof(uint32_t) * STATUS_WORDS))) return r;
@@ -323,39 +368,38 @@ int bind_plan(hana_ctx* c, Plan& pl, Arena& A, uint32_t min_bins, uint32_t min_p
         d.stats = with_stats ? A.stats.as<uint64_t>() + (size_t)ST_WORDS * i : nullptr;
     }
     Workspace& ws = pl.ws;
-    ws.tile_count = A.tile_count.as<uint32_t>();
-    ws.tile_offset = A.tile_offset.as<uint32_t>();
-    ws.tile_cursor = A.tile_cursor.as<uint32_t>();
     ws.bins = A.bins.as<uint32_t>();
+    ws.chunks = A.chunks.as<uint2>();
+    // whole 32-byte groups of descriptors (loaded four at a time), an odd
+    // number of them so that the tiles' first groups spread over the caches
+    uint64_t groups = std::min<uint64_t>(A.chunk_slots / tiles / 4, 1u << 28);
+    ws.chunk_cap = (uint32_t)(4 * (groups - 1 + (groups & 1)));
+    ws.over = A.over.as<uint4>();
+    ws.over_cap = A.over_cap;
+    ws.wide = A.wide.as<uint2>();
+    ws.wide_cap = A.wide_cap;
     ws.pool_vr = A.pool_vr.as<float4>();
     ws.pool_vs = A.pool_vs.as<float>();
     ws.pool_face = A.pool_face.as<int32_t>();
-    ws.pool_pass = A.pool_pass.as<int32_t>();
-    ws.pool_n = A.pool_n.as<int32_t>();
     ws.clip_queue = A.clip_queue.as<uint64_t>();
-    ws.tris = A.tris.as<uint4>();
-    ws.tris_cap = A.tris_cap;
-    ws.seg_region = (uint32_t)seg_region;
-    ws.seg_count = A.seg_count.as<uint32_t>();
-    ws.seg_tiles = A.seg_tiles.as<uint2>();
-    ws.seg_wide = A.seg_wide.as<uint16_t>();
-    ws.seg_info = A.seg_info.as<uint32_t>();
-    ws.seg_stride = seg_stride;
-    ws.scan_part = A.scan_part.as<uint64_t>();
     ws.clipq_cap = A.clipq_cap;
+    // the counters zeroed by the sequence itself; per-call sequences take
+    // theirs at the launch (take_counters)
+    set_counters(pl, A, 0);
+    ws.zero = ws.seq;
+    ws.zero_n = (uint32_t)counter_words(pl);
     ws.status = A.status.as<uint32_t>();
     ws.status_out = nullptr;
-    ws.ntiles = pl.total_tiles;
     ws.bin_cap = A.bin_cap;
+    ws.seg_region = (uint32_t)seg_region;
     ws.poly_cap = A.poly_cap;
-    ws.qstate = A.qstate.as<uint32_t>();
     ws.q_items = (uint32_t)pl.total_tiles;
     ws.q_g0 = pl.q_g0;
     ws.q_dep_from = pl.q_dep_from;
     ws.tile_shift = pl.tile_shift;
     ws.raster_waves = pl.raster_waves;
     for (int g = 0; g < 2; g++)
-        ws.tile_pass[g] = pl.group_count[g] > 0
+        ws.tile_pass[g] = pl.group_count[g] > 0 && !pl.args
                               ? reinterpret_cast<const uint2*>(A.tables.as<char>() + pl.tp_off) + pl.tp_first[g]
                               : nullptr;
     return HANA_OK;
@@ -406,10 +450,31 @@ struct StageTimer {
     }
 };
 
-// The geometry stages: vertex, set-up, clipping, tile scan, binning.
+// The geometry stages: vertex, set-up with binning, clipping; or all of them
+// in one launch (timed as set-up), before which a sequence that zeroes its own
+// counters does so.
 int enqueue_geometry(hana_ctx* c, const Plan& pl, const Arena& A, hipStream_t s, bool timed) {
-    const PassDesc* d = A.tables.as<PassDesc>();
+    PassDesc* d = A.tables.as<PassDesc>();
     int n = (int)pl.descs.size();
+    if (pl.front) {
+        DevUniforms* u = reinterpret_cast<DevUniforms*>(A.tables.as<char>() + pl.uni_off);
+        Workspace ws = pl.ws;
+        FrontTables t;
+        if (pl.args) {
+            for (int i = 0; i < n; i++) {
+                t.d[i] = pl.descs[i];
+                t.u[i] = pl.unis[i];
+            }
+        }
+        StageTimer timer(c, 1, timed, s);
+        if (ws.zero == ws.seq) {
+            HIP_TRY(c, launch_fill32(ws.zero, 0u, ws.zero_n, s));
+            ws.zero_n = 0;
+        }
+        HIP_TRY(c, launch_front(pl.args ? &t : nullptr, d, u, n, ws, pl.fblocks, pl.vblocks, s));
+        timer.done(s);
+        return HANA_OK;
+    }
     {
         StageTimer t(c, 0, timed, s);
         HIP_TRY(c, launch_vertex(d, n, pl.ws, pl.vblocks, s));
@@ -423,16 +488,6 @@ int enqueue_geometry(hana_ctx* c, const Plan& pl, const Arena& A, hipStream_t s,
     {
         StageTimer t(c, 2, timed, s);
         HIP_TRY(c, launch_clip(d, pl.ws, s));
-        t.done(s);
-    }
-    {
-        StageTimer t(c, 3, timed, s);
-        HIP_TRY(c, launch_scan(pl.ws, s));
-        t.done(s);
-    }
-    {
-        StageTimer t(c, 4, timed, s);
-        HIP_TRY(c, launch_bin(d, pl.ws, pl.fblocks, pl.small_tris, s));
         t.done(s);
     }
     return HANA_OK;
@@ -498,10 +553,40 @@ int upload_tables(hana_ctx* c, const Plan& pl, Arena& A, hipStream_t s) {
     return HANA_OK;
 }
 
-// Grows an arena's bins, clip pool and triangle list to the needs reported
+// The largest needs (STATUS_NEED_*) that sequences reported, and their flags.
+struct Needs {
+    uint32_t w[STATUS_WORDS] = {};
+    void take(const uint32_t* status) {
+        w[STATUS_FLAGS] |= status[STATUS_FLAGS];
+        for (int i = STATUS_FLAGS + 1; i < STATUS_WORDS; i++) w[i] = std::max(w[i], status[i]);
+    }
+};
+
+// Grows an arena's chunk descriptors to the needs of an overflow.  The list
+// behind the tiles' places holds all that came after those; the places grow to
+// the fullest tile's need where that is up to 2^25 over all tiles (256 MB),
+// else, for few crowded tiles of large targets, by as many as came after.
+// More than 2^26 of them are wide triangles in each of their tiles: those are
+// then listed once each.
+static int grow_chunks(hana_ctx* c, Arena& A, const Needs& need) {
+    int r;
+    const uint64_t past = need.w[STATUS_NEED_OVER], full = (uint64_t)need.w[STATUS_NEED_CHUNKS] * 1024 / 4 * 5;
+    if (past > (1u << 26)) {
+        A.wide_cap = std::max(A.wide_cap, need.w[STATUS_NEED_WIDE]);   // bind_plan allocates
+    } else {
+        const uint64_t want = full <= (1u << 25) ? std::max(full, A.chunk_slots) : A.chunk_slots + past / 4 * 5;
+        if ((r = ensure(c, A.chunks, sizeof(uint2) * want))) return r;
+        A.chunk_slots = want;
+        A.over_cap = std::max<uint32_t>(A.over_cap, (uint32_t)(past / 4 * 5 + OVER_MIN));
+    }
+    return HANA_OK;
+}
+
+// Grows an arena's bins, chunk descriptors and clip pool to the needs reported
 // by an overflow (capacities never shrink).
-static int grow_arena(hana_ctx* c, Arena& A, uint32_t flags, uint32_t need_bins, uint32_t need_polys,
-                      uint32_t need_tris) {
+static int grow_arena(hana_ctx* c, Arena& A, const Needs& need) {
+    const uint32_t flags = need.w[STATUS_FLAGS], need_bins = need.w[STATUS_NEED_BINS],
+                   need_polys = need.w[STATUS_NEED_POLYS];
     if (flags & FLAG_BIN_OVERFLOW) {
         uint64_t want = std::max<uint64_t>((uint64_t)need_bins + need_bins / 4 + 1024, A.bin_cap);
         want = std::min<uint64_t>(want, MAX_PAIRS);
@@ -509,11 +594,9 @@ static int grow_arena(hana_ctx* c, Arena& A, uint32_t flags, uint32_t need_bins,
         if (r) return r;
         A.bin_cap = (uint32_t)want;
     }
-    if (flags & FLAG_TRIS_OVERFLOW) {
-        uint64_t want = std::min<uint64_t>((uint64_t)A.tris_cap + need_tris + need_tris / 4 + 1024, 0xFFFFFFF0ull);
-        int r = ensure(c, A.tris, sizeof(uint4) * want);
+    if (flags & FLAG_CHUNK_OVERFLOW) {
+        int r = grow_chunks(c, A, need);
         if (r) return r;
-        A.tris_cap = (uint32_t)want;
     }
     if (flags & FLAG_POLY_OVERFLOW) {
         uint64_t want = std::max<uint64_t>((uint64_t)need_polys + need_polys / 4 + 1024, A.poly_cap);
@@ -522,8 +605,6 @@ static int grow_arena(hana_ctx* c, Arena& A, uint32_t flags, uint32_t need_bins,
         if ((r = ensure(c, A.pool_vr, sizeof(float4) * POLY_MAX * want))) return r;
         if ((r = ensure(c, A.pool_vs, sizeof(float) * POLY_MAX * POLY_VARY * want))) return r;
         if ((r = ensure(c, A.pool_face, sizeof(int32_t) * want))) return r;
-        if ((r = ensure(c, A.pool_pass, sizeof(int32_t) * want))) return r;
-        if ((r = ensure(c, A.pool_n, sizeof(int32_t) * want))) return r;
         A.poly_cap = (uint32_t)want;
     }
     return HANA_OK;
@@ -535,10 +616,12 @@ static int replay_call(hana_ctx* c, LoggedCall& L) {
     int r;
     Plan& pl = L.pl;
     Arena& A = slot_arena(c, 0);
-    if ((r = bind_plan(c, pl, A, 0, 0, 0, false, c->stream))) return r;
+    if ((r = bind_plan(c, pl, A, 0, 0, false, c->stream))) return r;
     pl.ws.status_out = c->status_dev[0];
-    if ((r = upload_tables(c, pl, A, c->stream))) return r;
+    if ((r = take_counters(c, pl, A, c->stream))) return r;
+    if (!pl.args && (r = upload_tables(c, pl, A, c->stream))) return r;
     if ((r = enqueue_geometry(c, pl, A, c->stream, false))) return r;
+    counters_launched(A);
     for (const Fill& f : L.fills) {
         size_t n = (size_t)f.target->w * f.target->h;
         HIP_TRY(c, launch_fill32(f.target->color, f.rgba, n, c->stream));
@@ -551,7 +634,7 @@ static int replay_call(hana_ctx* c, LoggedCall& L) {
 
 // Reads the sticky status of every sequence since the last check, over all
 // draw slots (waits for every stream).
-// - A capacity overflow (bins, clip pool, clip queue, triangle list) left its
+// - A capacity overflow (bins, chunk descriptors, clip pool, clip queue) left its
 //   sequence's targets untouched.  Every slot's workspace is grown to the
 //   largest need seen and the calls since the last check are rendered again
 //   in call order; a draw over the same state twice leaves it as drawn once
@@ -568,25 +651,21 @@ int check_status(hana_ctx* c) {
     uint32_t seen = 0;
     for (int attempt = 0;; attempt++) {
         if ((r = sync_all(c))) return r;
-        uint32_t flags = 0, need_bins = 0, need_polys = 0, need_tris = 0;
+        Needs need;
         for (int k = 0; k < c->nslots; k++) {
             const uint32_t* host = slot_status(c, k);
             if (!host) continue;
-            flags |= host[STATUS_FLAGS];
-            need_bins = std::max(need_bins, host[STATUS_NEED_BINS]);
-            need_polys = std::max(need_polys, host[STATUS_NEED_POLYS]);
-            need_tris = std::max(need_tris, host[STATUS_NEED_TRIS]);
+            need.take(host);
         }
+        const uint32_t flags = need.w[STATUS_FLAGS];
         seen |= flags;
         if (flags) {
             for (int k = 0; k < c->nslots; k++) {
                 uint32_t* host = slot_status(c, k);
                 if (!host) continue;
                 Arena& A = slot_arena(c, k);
-                if (A.status.p)
-                    HIP_TRY(c, launch_fill32(A.status.as<uint32_t>() + STATUS_SEQ_WORDS, 0u,
-                                             STATUS_WORDS - STATUS_SEQ_WORDS, c->stream));
-                std::memset(host + STATUS_SEQ_WORDS, 0, sizeof(uint32_t) * (STATUS_WORDS - STATUS_SEQ_WORDS));
+                if (A.status.p) HIP_TRY(c, launch_fill32(A.status.as<uint32_t>(), 0u, STATUS_WORDS, c->stream));
+                std::memset(host, 0, sizeof(uint32_t) * STATUS_WORDS);
             }
             // the next geometry stages may run on any stream
             HIP_TRY(c, hipStreamSynchronize(c->stream));
@@ -594,7 +673,7 @@ int check_status(hana_ctx* c) {
         uint32_t cap = flags & FLAG_CAPACITY;
         if (cap)
             for (int k = 0; k < c->nslots; k++)
-                if ((r = grow_arena(c, slot_arena(c, k), flags, need_bins, need_polys, need_tris))) {
+                if ((r = grow_arena(c, slot_arena(c, k), need))) {
                     c->log.clear();
                     c->status_pending = false;
                     return r;
@@ -667,24 +746,29 @@ int run_passes(hana_ctx* c, std::vector<PassSpec> specs) {
     // while frames of up to 400 k faces ran 6 % faster.
     int nslots = pl.total_f >= kLargeSequenceFaces ? std::min(2, c->nslots) : c->nslots;
     int a = rotate ? c->next_slot % nslots : 0;
+    const int last = pl.specs.back().target->slot;
+    const bool stay = rotate && pl.total_f <= kStayFaces && last >= 0 && last < nslots;
+    if (stay) a = last;
     hipStream_t S = slot_stream(c, a);
     Arena& A = slot_arena(c, a);
     // the slots' workspaces grow together, so that a sequence of calls
     // allocates (and waits for the streams) once, not once per slot
     if (rotate)
         for (int k = 0; k < nslots; k++)
-            if (k != a && (r = bind_plan(c, pl, slot_arena(c, k), 0, 0, 0, false, slot_stream(c, k)))) return r;
-    if ((r = bind_plan(c, pl, A, 0, 0, 0, c->stats_enabled, S))) return r;
-    pl.ws.status_out = c->status_dev[a];   // the scan leaves the status words in host memory
+            if (k != a && (r = bind_plan(c, pl, slot_arena(c, k), 0, 0, false, slot_stream(c, k)))) return r;
+    if ((r = bind_plan(c, pl, A, 0, 0, c->stats_enabled, S))) return r;
+    pl.ws.status_out = c->status_dev[a];   // the raster leaves the status words in host memory
     // a target sampled as a shadow map by a pass of the same plan must be drawn
     // by an earlier group; clears fuse into the first pass writing the target
     take_clears(pl);
-    if ((r = upload_tables(c, pl, A, S))) return r;
+    if ((r = take_counters(c, pl, A, S))) return r;
+    if (!pl.args && (r = upload_tables(c, pl, A, S))) return r;
     int n = (int)pl.descs.size();
     if (c->stats_enabled) {
         HIP_TRY(c, launch_fill32(reinterpret_cast<uint32_t*>(A.stats.p), 0u, (size_t)ST_WORDS * 2 * n, S));
     }
     if ((r = enqueue_geometry(c, pl, A, S, true))) return r;
+    counters_launched(A);
     // the raster waits for the calls in flight on other slots that touch one
     // of its targets; calls on disjoint targets run concurrently.  After a
     // no-alloc frame (context stream, targets not noted) every slot waits once.
@@ -693,7 +777,7 @@ int run_passes(hana_ctx* c, std::vector<PassSpec> specs) {
         c->noalloc_wait_mask &= ~(1u << a);
     }
     for (int k = 0; k < c->nslots; k++)
-        if (k != a && (c->pend[k][a].size() > kMaxPendingTargets || shares_target(c->pend[k][a], touched))) {
+        if (k != a && (c->pend[k][a].size() > kMaxPendingTargets || must_wait(c, k, a, touched))) {
             HIP_TRY(c, hipStreamWaitEvent(S, c->slot_done[k], 0));
             c->pend[k][a].clear();
         }
@@ -717,7 +801,7 @@ int run_passes(hana_ctx* c, std::vector<PassSpec> specs) {
         c->stats_passes = n;
     }
     if (c->pipelined) note_pending(c, a, touched);   // else no other slot ever draws
-    c->next_slot = (a + 1) % nslots;
+    if (!stay) c->next_slot = (a + 1) % nslots;
     c->status_pending = true;
     c->log.push_back({std::move(pl), std::move(fills)});
     return HANA_OK;
@@ -804,17 +888,19 @@ int create_context(int device, int nslots, hana_ctx** out) {
 extern "C" {
 
 static void free_arena(Arena& a) {
-    DevBuf* bufs[] = {&a.tables, &a.vr, &a.vs, &a.code, &a.tris, &a.seg_count, &a.seg_tiles, &a.seg_wide,
-                      &a.seg_info, &a.qstate, &a.scan_part, &a.pof, &a.tile_count, &a.tile_offset, &a.tile_cursor,
-                      &a.bins, &a.pool_vr, &a.pool_vs, &a.pool_face, &a.pool_pass, &a.pool_n, &a.clip_queue,
-                      &a.status, &a.stats};
+    DevBuf* bufs[] = {&a.tables, &a.vr, &a.vs, &a.code, &a.pof, &a.bins, &a.chunks, &a.over, &a.wide, &a.pool_vr,
+                      &a.pool_vs, &a.pool_face, &a.clip_queue, &a.status, &a.stats, &a.counters[0], &a.counters[1]};
     for (DevBuf* b : bufs)
         if (b->p) {
             (void)hipFree(b->p);
             b->p = nullptr;
             b->cap = 0;
         }
-    a.bin_cap = a.poly_cap = a.clipq_cap = a.tris_cap = 0;
+    a.bin_cap = a.poly_cap = a.clipq_cap = 0;
+    a.chunk_slots = 0;
+    a.over_cap = 0;
+    a.wide_cap = WIDE_MAX;
+    a.counters_used[0] = a.counters_used[1] = 0;
 }
 
 int hana_gpu_destroy(hana_ctx* c) {
@@ -1278,10 +1364,10 @@ static int batch_enqueue(hana_ctx* c, hana_batch* b, bool timed) {
 static int batch_size_part(hana_ctx* c, hana_batch* b, hana_batch_part& part) {
     int r;
     if ((r = build_plan(c, part.specs, part.plan, b->tuning))) return r;
-    uint32_t min_bins = 0, min_polys = 0, min_tris = 0;
+    uint32_t min_bins = 0, min_polys = 0;
     Arena& A = *part.arena;
     for (int attempt = 0; attempt < 3; attempt++) {
-        if ((r = bind_plan(c, part.plan, A, min_bins, min_polys, min_tris, false, c->stream))) return r;
+        if ((r = bind_plan(c, part.plan, A, min_bins, min_polys, false, c->stream))) return r;
         batch_clear_flags(part);
         HIP_TRY(c, hipMemcpy(A.tables.p, part.plan.descs.data(), sizeof(PassDesc) * part.plan.descs.size(),
                              hipMemcpyHostToDevice));
@@ -1297,8 +1383,7 @@ static int batch_size_part(hana_ctx* c, hana_batch* b, hana_batch_part& part) {
         HIP_TRY(c, hipStreamSynchronize(c->stream));
         batch_drop_pending(b);
         if (!st[STATUS_FLAGS]) return HANA_OK;
-        HIP_TRY(c, launch_fill32(A.status.as<uint32_t>() + STATUS_SEQ_WORDS, 0u, STATUS_WORDS - STATUS_SEQ_WORDS,
-                                 c->stream));
+        HIP_TRY(c, launch_fill32(A.status.as<uint32_t>(), 0u, STATUS_WORDS, c->stream));
         if (st[STATUS_FLAGS] & FLAG_QUEUE_STALL)
             return fail(c, HANA_E_DEVICE, "hana_batch_finalize: the persistent raster's wait timed out");
         if (!(st[STATUS_FLAGS] & FLAG_CAPACITY)) {
@@ -1307,9 +1392,11 @@ static int batch_size_part(hana_ctx* c, hana_batch* b, hana_batch_part& part) {
                                              "(triangle, tile) pairs; split the batch");
             return HANA_OK;   // a polygon over POLY_MAX vertices is dropped at every run, like a per-call draw
         }
-        min_bins = st[STATUS_BINS_NEEDED] + st[STATUS_BINS_NEEDED] / 8 + 1024;
-        min_polys = st[STATUS_POLYS] + st[STATUS_POLYS] / 8 + 1024;
-        min_tris = st[STATUS_TRIS] + st[STATUS_TRIS] / 8 + 1024;
+        min_bins = st[STATUS_NEED_BINS] + st[STATUS_NEED_BINS] / 8 + 1024;
+        min_polys = st[STATUS_NEED_POLYS] + st[STATUS_NEED_POLYS] / 8 + 1024;
+        Needs need;
+        need.take(st);
+        if ((st[STATUS_FLAGS] & FLAG_CHUNK_OVERFLOW) && (r = grow_chunks(c, A, need))) return r;
     }
     return fail(c, HANA_E_OVERFLOW, "hana_batch_finalize: capacity not reached");
 }

@@ -89,7 +89,7 @@ namespace {
 
 // Device footprint charged to a request: its targets and the per-pass
 // workspace (per vertex: position, varyings, outcode; per face: bins, clip
-// queue and pool, triangle list).
+// queue and pool).
 int64_t request_bytes(const hana_request& r, int sw, int sh) {
     int64_t V = r.mesh->V, F = r.mesh->F;
     int passes = r.enable_shadow ? 2 : 1;

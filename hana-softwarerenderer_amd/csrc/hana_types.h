@@ -48,6 +48,11 @@ static_assert(HANA_SMALL_PIX >= 1 && HANA_SMALL_PIX <= 32, "small-triangle candi
 #endif
 constexpr int VPT = HANA_VPT;              // vertices per thread in k_vertex
 constexpr int FPT = HANA_FPT;              // faces per thread in k_setup
+#ifndef HANA_FRONT_FPT
+#define HANA_FRONT_FPT 1
+#endif
+constexpr int FRONT_FPT = HANA_FRONT_FPT;  // faces per thread in k_front
+constexpr int FRONT_VPT = 1;               // vertices per thread in k_front
 // Vertices the device keeps of a clipped polygon: a convex polygon gains at
 // most one vertex per plane (3 + 7), rounding in the inside tests can add a
 // few more; one lane of a 16-lane clip group holds each.
@@ -111,41 +116,57 @@ struct PassDesc {
     uint64_t* stats;             // 5 counters (hana_pass_stats order), or null
     // first block of this pass in each kernel's grid / first global tile
     int32_t vblock0, fblock0, tile0, tblock0;
+    int32_t index;               // of this pass in its sequence (its list of wide triangles)
+    int32_t pad_;
 };
 
 // Buffers shared by every pass of one launch sequence.
+//
+// The (triangle, tile) pairs of a sequence are held as chunks: the entries of
+// one set-up workgroup's triangles that touch one tile, contiguous in `bins`.
+// Each tile has chunk_cap places for its chunks' descriptors, filled in the
+// order the workgroups reach it.  A pair outside any workgroup's table (a
+// clipped fan triangle, a table overflow) is a descriptor that holds its entry
+// itself (CHUNK_INLINE).  So one pass over the triangles bins them, without
+// counts, a scan or a second pass, and a raster workgroup reads its tile's
+// descriptors with one coalesced load.  Descriptors past a tile's places go to
+// one list of the sequence, which the raster workgroups of such tiles search,
+// so that meshes crowded into few tiles of a large target need no places for
+// them in every tile.  A triangle over more than WIDE_TILES tiles goes to its
+// pass's list instead, which every tile of the pass tests.
 struct Workspace {
-    uint32_t* tile_count;        // per global tile
-    uint32_t* tile_offset;       // exclusive scan of tile_count (+ total at [ntiles])
-    uint32_t* tile_cursor;
-    uint32_t* bins;              // triangle entries grouped by tile
+    uint2* chunks;               // per tile, chunk_cap: first bin entry and entries, or entry and CHUNK_INLINE
+    uint32_t chunk_cap;
+    uint32_t* bins;              // triangle entries: face id and its FACE_* bits, or CLIPPED_BIT | polygon << 4 | fan
+    uint4* over;                 // descriptors past their tile's places: tile, then as in chunks
+    uint32_t over_cap;
+    uint32_t wide_cap;
+    uint2* wide;                 // per pass, wide_cap: box of tiles (wide_box) and bin entry
     float4* pool_vr;             // clipped polygons: POLY_MAX vertices each
     float* pool_vs;              //   ... POLY_VARY varyings per vertex
     int32_t* pool_face;          //   face (within its pass) of each polygon
-    int32_t* pool_pass;          //   pass of each polygon
-    int32_t* pool_n;             //   vertex count of each polygon
     uint64_t* clip_queue;        // faces failing the trivial accept: pass << 32 | face
-    uint4* tris;                 // every triangle with tiles: bin entry, pass, first tile, last tile;
-                                 //   BLOCK*FPT per k_setup workgroup, then the clipped fan triangles
-    uint32_t* seg_count;         // records in each k_setup workgroup's segment
-    uint2* seg_tiles;            // per segment, seg_stride entries: (tile, pairs) of its triangles
-                                 //   over at most WIDE_TILES tiles, counted in k_setup's LDS table
-    uint16_t* seg_wide;          // per segment, BLOCK*FPT entries: its triangles over more tiles
-    uint32_t* seg_info;          // per segment: listed tiles | wide triangles << 16
-    uint32_t seg_stride;
-    uint64_t* scan_part;         // per scan chunk: sum of its tile counts
+    // counters of this sequence, all zero when its first triangle is set up:
+    // the SEQ_* words, then a count of wide triangles per pass, then a count
+    // of chunks per tile
+    uint32_t* seq;
+    uint32_t* wide_count;
+    uint32_t* tile_chunks;
+    // words the sequence's first kernel zeroes: the counters themselves where a
+    // launch precedes set-up, else those of the workspace's other counter set
+    uint32_t* zero;
+    uint32_t zero_n;
     uint32_t* status;            // see STATUS_*
-    uint32_t* status_out;        // or null: host-mapped copy of the status words, written by the scan
-    int32_t ntiles;
+    uint32_t* status_out;        // or null: host-mapped copy of the status words, written by the raster
     uint32_t bin_cap;
+    uint32_t seg_region;         // bin entries that belong to one set-up workgroup each; the rest is shared
     uint32_t poly_cap;
     uint32_t clipq_cap;
-    uint32_t tris_cap;
-    uint32_t seg_region;         // records reserved for the setup segments
     // queue of the persistent raster (k_raster_q): its items are the tiles of
     // every pass in global tile order (shadow passes first, then main passes
     // that sample no map drawn here, then those that do)
-    uint32_t* qstate;            // [0] next item, [1] group-0 tiles finished and published
+    // (its state: seq[SEQ_QUEUE] the next item, seq[SEQ_QUEUE_DONE] the
+    // group-0 tiles finished and published)
     uint32_t q_items;            // tiles of all passes
     uint32_t q_g0;               // tiles of group-0 passes
     uint32_t q_dep_from;         // first item of a pass that samples a map drawn by group 0
@@ -158,29 +179,49 @@ struct Workspace {
     // b + that)
     const uint2* tile_pass[2];
 };
+// The tables of a sequence of at most FRONT_PASSES passes, as launch arguments.
+constexpr int FRONT_PASSES = 2;
+struct FrontTables {
+    PassDesc d[FRONT_PASSES];
+    DevUniforms u[FRONT_PASSES];
+};
+
 constexpr int TILE_PASS_SHIFT = 6;
 constexpr uint32_t TILE_PASS_PURE = 0x80000000u;
 
-// the tile scan: SCAN_CHUNK tile counters per workgroup of SCAN_THREADS
-constexpr int SCAN_THREADS = 256;
-constexpr int SCAN_PER_THREAD = 16;
-constexpr int SCAN_CHUNK = SCAN_THREADS * SCAN_PER_THREAD;
+constexpr uint32_t SEG_PAIRS = 2;          // bin entries of a set-up workgroup, per face
+constexpr uint32_t CHUNK_INLINE = 0x80000000u;
+constexpr uint32_t CHUNK_SLACK = 16;       // places per tile beyond a reported need
+// Triangles over more than WIDE_TILES tiles are listed once per pass, up to
+// Workspace::wide_cap of them (WIDE_MAX at first); later ones take a descriptor
+// in each of their tiles.
+constexpr int WIDE_TILES = 16;
+#ifndef HANA_WIDE_MAX
+#define HANA_WIDE_MAX 512
+#endif
+constexpr uint32_t WIDE_MAX = HANA_WIDE_MAX;
+constexpr uint32_t OVER_MIN = 1024;        // Workspace::over_cap at first
 
-// status words.  The first STATUS_SEQ_WORDS belong to one launch sequence
-// (zeroed by its first kernel): polygons allocated, faces queued for
-// clipping, clipped fan triangles listed, bin entries needed, and the flags
-// this sequence raised.  The others stay set across sequences until the host
-// reads them at a sync point: the flags of every sequence and the largest
-// needs seen, so that calls need not wait for one another.
-enum { STATUS_POLYS = 0, STATUS_CLIPQ = 1, STATUS_TRIS = 2, STATUS_BINS_NEEDED = 3, STATUS_SEQ_FLAGS = 4,
-       STATUS_SEQ_WORDS = 5, STATUS_FLAGS = 5, STATUS_NEED_BINS = 6, STATUS_NEED_POLYS = 7, STATUS_NEED_TRIS = 8,
-       STATUS_WORDS = 9 };
+// counter words of one sequence: polygons allocated, faces queued for
+// clipping, the flags it raised, the descriptors past their tiles' places and
+// the most chunks of one such tile, the persistent raster's queue, and (64-bit
+// each) the pairs outside the set-up workgroups' own entries and the pairs of
+// the listed wide triangles
+enum { SEQ_POLYS = 0, SEQ_CLIPQ = 1, SEQ_FLAGS = 2, SEQ_OVER = 3, SEQ_PAIRS = 4, SEQ_WIDE_PAIRS = 6,
+       SEQ_QUEUE = 8, SEQ_QUEUE_DONE = 9, SEQ_MAX_CHUNKS = 10, SEQ_WORDS = 16 };
+// status words: set across sequences until the host reads them at a sync
+// point, so that calls need not wait for one another: the flags of every
+// sequence and the largest needs seen: of places for descriptors, in units of
+// 1024 over all tiles of the sequence; of the list behind them; of wide
+// triangles in one pass.
+enum { STATUS_FLAGS = 0, STATUS_NEED_BINS = 1, STATUS_NEED_POLYS = 2, STATUS_NEED_CHUNKS = 3, STATUS_NEED_OVER = 4,
+       STATUS_NEED_WIDE = 5, STATUS_WORDS = 6 };
 enum { FLAG_BIN_OVERFLOW = 1, FLAG_POLY_OVERFLOW = 2, FLAG_POLY_TOO_LARGE = 4, FLAG_CLIPQ_OVERFLOW = 8,
-       FLAG_TRIS_OVERFLOW = 16, FLAG_PAIR_LIMIT = 32, FLAG_QUEUE_STALL = 64 };
+       FLAG_CHUNK_OVERFLOW = 16, FLAG_PAIR_LIMIT = 32, FLAG_QUEUE_STALL = 64 };
 // A workspace capacity ran out: the sequence is incomplete, its rasters write
 // nothing, and the host grows the workspace and renders it again.
-constexpr uint32_t FLAG_CAPACITY = FLAG_BIN_OVERFLOW | FLAG_POLY_OVERFLOW | FLAG_CLIPQ_OVERFLOW | FLAG_TRIS_OVERFLOW;
-// Flags of a sequence whose binning and rasters do nothing.
+constexpr uint32_t FLAG_CAPACITY = FLAG_BIN_OVERFLOW | FLAG_POLY_OVERFLOW | FLAG_CLIPQ_OVERFLOW | FLAG_CHUNK_OVERFLOW;
+// Flags of a sequence whose rasters do nothing.
 constexpr uint32_t FLAG_NO_RASTER = FLAG_CAPACITY | FLAG_PAIR_LIMIT;
 // (triangle, tile) pairs one launch sequence may hold: bin positions are
 // 32-bit.  A sequence with more sets FLAG_PAIR_LIMIT and rasterises nothing.

@@ -150,8 +150,8 @@ int hana_gpu_replay_count(hana_ctx* ctx, int64_t* out);
 
 /* Per-stage kernel timing with HIP events recorded around each launch
  * (benchmarking; while it is on, draws use one stream and do not overlap).  Stages: 0 vertex, 1 set-up (cull,
- * bounds, tile counts), 2 clipping, 3 tile scan, 4 binning, 5 (unused, no
- * launches), 6 raster of the first dependency group (shadow passes), 7 raster
+ * bounds, binning; of smaller sequences also vertices and clipping, in the
+ * same launch), 2 clipping, 3-5 (unused, no launches), 6 raster of the first dependency group (shadow passes), 7 raster
  * of the second group (main passes).  Reading returns the milliseconds and
  * launch counts accumulated since the last read. */
 #define HANA_TIMING_STAGES 8
