@@ -722,6 +722,33 @@ int check_status(hana_ctx* c) {
     return HANA_OK;
 }
 
+// The tuning of a per-call sequence.  Until the caller sets one, sequences of
+// few large triangles take 32x32 tiles: a raster workgroup's fixed part (the
+// tile's counters, its pass's wide triangles, a handful of dependent loads)
+// then serves four times the pixels.  Where the targets have so many tiles
+// that the workgroups run in several rounds, that is what they spend their
+// time on; with fewer tiles the larger ones leave CUs idle, with smaller
+// triangles their lanes.  Measured with 16x16 and 32x32 tiles, us per frame:
+// 3840x2160 of 1,000 faces 77 and 47, of 20,000 81 and 48, of 100,000 (83
+// pixels each) 78 and 63; 1920x1080 of 5,000 faces 27 and 21, of 20,000 (104)
+// 26 and 24, with a frame-sized shadow map 48 and 56, of 100,000 32 and 43;
+// 1280x720 of 1,000 faces 15 and 18.  The last condition holds where no scene
+// has more pairs of a triangle (at most 8 of a face) and a 16x16 tile than bin
+// positions reach, so that the rule decides nothing on what is refused.
+// Statistics count 16x16 tiles.
+static Tuning call_tuning(const hana_ctx* c, const std::vector<PassSpec>& specs) {
+    Tuning t = c->tuning;
+    if (!t.set && !c->stats_enabled) {
+        int64_t px = 0, faces = 0;
+        for (const PassSpec& s : specs) {
+            px += (int64_t)s.target->w * s.target->h;
+            faces += s.mesh->F;
+        }
+        if (px >= 8000 * 256 && px >= 128 * faces && px * faces < (int64_t(1) << 37)) t.tile_shift = 5;
+    }
+    return t;
+}
+
 // Renders a list of passes (per-call path).  Consecutive calls rotate over
 // the context's slots, each a stream with its own workspace: the geometry
 // stages of a call run while earlier calls rasterise, and its raster waits
@@ -739,7 +766,8 @@ int run_passes(hana_ctx* c, std::vector<PassSpec> specs) {
         if (!drawn && std::find(sampled.begin(), sampled.end(), s.shadow) == sampled.end()) sampled.push_back(s.shadow);
     }
     Plan pl;
-    if ((r = build_plan(c, std::move(specs), pl, c->tuning))) return r;
+    const Tuning tuning = call_tuning(c, specs);
+    if ((r = build_plan(c, std::move(specs), pl, tuning))) return r;
     bool rotate = c->pipelined && !c->timing && !c->stats_enabled;
     // Large sequences rotate over two slots: with a third in flight, the 2.6 M
     // faces of a 1.3 M-triangle frame with its shadow pass ran 1.2 % slower,
@@ -817,6 +845,7 @@ int tuning_from(hana_ctx* c, const hana_tuning* t, Tuning& out) {
     out.raster_wgs_per_cu = t->raster_wgs_per_cu;
     out.raster_waves = t->raster_waves ? t->raster_waves : 4;
     out.parts = t->parts;
+    out.set = true;
     return HANA_OK;
 }
 

@@ -217,7 +217,8 @@ int hana_render_frame_noalloc(hana_ctx* ctx, const hana_frame_desc* f);
  * raster workgroup, 2 or 4 waves (two waves fit twice the tiles on a CU).
  * parts: the concurrent parts a batch is split into (1-4; ignored for
  * per-call draws).  Results are identical under every tuning.  Default: 16,
- * 0, 4 parts, 4 waves. */
+ * 0, 4 parts, 4 waves; until a tuning is set, per-call draws of few large
+ * triangles on large targets take 32x32 tiles. */
 typedef struct hana_tuning {
     int32_t tile_size;
     int32_t raster_wgs_per_cu;

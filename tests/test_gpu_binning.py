@@ -49,6 +49,10 @@ CASES = {
     "crowded-list": (60_000, (2048, 1024), (100, 400), 0.01),
     "crowded-places": (120_000, (2048, 1024), (100, 400), 0.01),
     "crowded-large": (140_000, (4096, 4096), (100, 400), 0.01),
+    # 32x32 tiles from 8,000 16x16 tiles and 128 pixels per face on
+    "tiles-16": (16_257, (1930, 1078), (4, 30), 1.0),
+    "tiles-32": (16_253, (1930, 1078), (4, 30), 1.0),
+    "tiles-32-clipped": (3000, (2049, 1025), (30, 90), 1.5),
 }
 
 
