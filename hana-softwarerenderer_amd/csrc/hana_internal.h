@@ -130,6 +130,8 @@ constexpr int kRing = 32;
 // calls kept for replay; past this many a call first checks the status of
 // those before it (a sync)
 constexpr size_t kMaxLoggedCalls = 1024;
+// a piece of a result staged in pinned memory; two are in flight
+constexpr size_t kStagePiece = size_t(8) << 20;
 // streams (each with a workspace) that consecutive per-call draws rotate over
 #ifndef HANA_DRAW_SLOTS
 #define HANA_DRAW_SLOTS 4
@@ -195,6 +197,15 @@ struct hana_ctx {
     bool pipelined = true;
     // device staging for hana_target_present
     hana::rt::DevBuf present;
+    // pinned staging of results for pageable memory (up to 2 kStagePiece)
+    char* stage_host = nullptr;
+    char* stage_dev = nullptr;
+    size_t stage_cap = 0;
+    // bands of two planes stored there (k_read_back): flags behind the staging's
+    // stage_cap bytes, the kernel's counters, the last launch's number
+    hana::rt::DevBuf stage_count;
+    uint32_t stage_epoch = 0;
+    hipEvent_t stage_done[2] = {nullptr, nullptr};
     // optional per-stage timing
     bool timing = false;
     std::vector<hipEvent_t> ev_pool;

@@ -1820,6 +1820,40 @@ __global__ void k_present(const uint32_t* __restrict__ src, uint32_t* __restrict
     }
 }
 
+// The word of the read-back image at i: k_present's, or the plane's own.
+__device__ __forceinline__ uint32_t read_back_word(const uint32_t* src, uint32_t i, uint32_t w, uint32_t h, bool flip) {
+    if (!flip) return gld(src + i);
+    uint32_t r = i / w, v = gld(src + (size_t)(h - 1u - r) * w + (i - r * w));
+    return ((v & 0xFFu) << 16) | (v & 0xFF00FF00u) | ((v >> 16) & 0xFFu);
+}
+
+// A plane written to host memory by the kernel itself, READ_WGS workgroups per
+// band, and a flag in host memory as each band is complete: the host copies it
+// on to the caller while the next ones come.  Bound by the link (2.4 MB in
+// about 50 us), of which 16-byte stores keep enough in flight.
+__global__ void k_read_back(const uint32_t* __restrict__ src, uint32_t* __restrict__ dst, uint32_t w, uint32_t h, int flip,
+                            uint32_t band, uint32_t wgs, uint32_t* done, uint32_t* flags, uint32_t epoch) {
+    const uint32_t n = w * h, b = blockIdx.x / wgs, first = b * band, end = min(n, first + band);
+    for (uint32_t i = first + ((blockIdx.x - b * wgs) * BLOCK + threadIdx.x) * 4u; i < end; i += wgs * BLOCK * 4u) {
+        uint32_t v[4];
+        for (uint32_t k = 0; k < 4u; k++) v[k] = i + k < end ? read_back_word(src, i + k, w, h, flip != 0) : 0u;
+        if (i + 4u <= end) *reinterpret_cast<uint4*>(dst + i) = make_uint4(v[0], v[1], v[2], v[3]);
+        else
+            for (uint32_t k = 0; i + k < end; k++) dst[i + k] = v[k];
+    }
+    if (gridDim.x == wgs) return;   // one band: the host waits for the launch
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        // one fence for the workgroup (one a thread took 15 us more at 360 KB);
+        // a band's workgroups count up over the launches
+        __threadfence_system();
+        if ((gadd(done + b, 1u) + 1u) % wgs == 0u) {
+            __threadfence_system();
+            __hip_atomic_store(flags + b, epoch, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
+    }
+}
+
 // ---------------------------------------------------------------------------
 // launch wrappers
 // ---------------------------------------------------------------------------
@@ -1896,6 +1930,17 @@ hipError_t launch_raster_queue(const PassDesc* d_passes, int npasses, const Work
         if (two) hipLaunchKernelGGL((k_raster_q<4, 128>), dim3(workgroups), dim3(128), 0, s, d_passes, npasses, ws);
         else hipLaunchKernelGGL((k_raster_q<4, 256>), dim3(workgroups), dim3(256), 0, s, d_passes, npasses, ws);
     }
+    return hipGetLastError();
+}
+hipError_t launch_read_back(const uint32_t* src, uint32_t* dst, int w, int h, bool flip, uint32_t band, uint32_t* done,
+                            uint32_t* flags, uint32_t epoch, hipStream_t s) {
+    const uint32_t bands = ((uint32_t)w * (uint32_t)h + band - 1u) / band;
+    if (bands == 0) return hipSuccess;
+    if (bands > READ_BANDS || band % 4u) return hipErrorInvalidValue;
+    // a single band has as many workgroups as it fills once
+    const uint32_t wgs = bands > 1 ? READ_WGS : ((uint32_t)w * (uint32_t)h + 4 * BLOCK - 1) / (4 * BLOCK);
+    hipLaunchKernelGGL(k_read_back, dim3(bands * wgs), dim3(BLOCK), 0, s, src, dst, (uint32_t)w, (uint32_t)h, flip ? 1 : 0,
+                       band, wgs, done, flags, epoch);
     return hipGetLastError();
 }
 hipError_t launch_present(const uint32_t* src, uint32_t* dst, int w, int h, hipStream_t s) {

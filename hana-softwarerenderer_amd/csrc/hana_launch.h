@@ -21,6 +21,11 @@ hipError_t launch_raster(const PassDesc* d_passes, int npasses, const Workspace&
 hipError_t launch_raster_queue(const PassDesc* d_passes, int npasses, const Workspace& ws, int workgroups,
                                hipStream_t s);
 hipError_t launch_fill32(uint32_t* dst, uint32_t value, size_t n, hipStream_t s);
+// One plane of w x h words into host-mapped memory, as k_present does (flip) or
+// as it is, in bands of `band` words; band i stored, flags[i] becomes epoch.
+// done: READ_BANDS device words, zero before the first launch.
+hipError_t launch_read_back(const uint32_t* src, uint32_t* dst, int w, int h, bool flip, uint32_t band, uint32_t* done,
+                            uint32_t* flags, uint32_t epoch, hipStream_t s);
 hipError_t launch_present(const uint32_t* src, uint32_t* dst, int w, int h, hipStream_t s);
 
 }  // namespace hana

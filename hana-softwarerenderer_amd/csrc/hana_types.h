@@ -179,6 +179,10 @@ struct Workspace {
     // b + that)
     const uint2* tile_pass[2];
 };
+// A plane on its way to host memory in bands (k_read_back).
+constexpr int READ_BANDS = 8;              // of a plane
+constexpr uint32_t READ_WGS = 32;          // workgroups per band
+constexpr uint32_t READ_BAND_MIN = 1u << 17;   // words of a band, at least
 // The tables of a sequence of at most FRONT_PASSES passes, as launch arguments.
 constexpr int FRONT_PASSES = 2;
 struct FrontTables {
