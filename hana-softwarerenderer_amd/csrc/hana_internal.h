@@ -99,7 +99,7 @@ struct Plan {
     int total_tiles = 0;
     bool small_tris = true;   // every pass has at most 4 target pixels per face
     int tile_shift = TILE_SHIFT_DEFAULT;
-    int raster_waves = 4;
+    int raster_waves[2] = {4, 4};   // per raster group (the persistent raster: the first)
     int raster_wgs = 0;       // workgroups of the persistent raster (0: one per tile and group)
     bool front = false;       // geometry in one launch (k_front)
     bool args = false;        // ... which brings the tables as arguments (no upload, no pass lookup)

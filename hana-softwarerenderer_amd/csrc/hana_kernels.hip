@@ -1906,10 +1906,10 @@ static void raster_launch(const PassDesc* d_passes, int npasses, const Workspace
     if (group) hipLaunchKernelGGL((k_raster<TS, 1, RB>), dim3(blocks), dim3(RB), 0, s, d_passes, npasses, ws);
     else hipLaunchKernelGGL((k_raster<TS, 0, RB>), dim3(blocks), dim3(RB), 0, s, d_passes, npasses, ws);
 }
-hipError_t launch_raster(const PassDesc* d_passes, int npasses, const Workspace& ws, int blocks, int group,
+hipError_t launch_raster(const PassDesc* d_passes, int npasses, const Workspace& ws, int blocks, int group, int waves,
                          hipStream_t s) {
     if (blocks <= 0) return hipSuccess;
-    bool two = ws.raster_waves == 2;
+    bool two = waves == 2;
     if (ws.tile_shift == 5) {
         if (two) raster_launch<5, 128>(d_passes, npasses, ws, blocks, group, s);
         else raster_launch<5, 256>(d_passes, npasses, ws, blocks, group, s);
@@ -1920,9 +1920,9 @@ hipError_t launch_raster(const PassDesc* d_passes, int npasses, const Workspace&
     return hipGetLastError();
 }
 hipError_t launch_raster_queue(const PassDesc* d_passes, int npasses, const Workspace& ws, int workgroups,
-                               hipStream_t s) {
+                               int waves, hipStream_t s) {
     if (workgroups <= 0 || ws.q_items == 0) return hipSuccess;
-    bool two = ws.raster_waves == 2;
+    bool two = waves == 2;
     if (ws.tile_shift == 5) {
         if (two) hipLaunchKernelGGL((k_raster_q<5, 128>), dim3(workgroups), dim3(128), 0, s, d_passes, npasses, ws);
         else hipLaunchKernelGGL((k_raster_q<5, 256>), dim3(workgroups), dim3(256), 0, s, d_passes, npasses, ws);

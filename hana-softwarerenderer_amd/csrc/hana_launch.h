@@ -14,12 +14,12 @@ hipError_t launch_clip(const PassDesc* d_passes, const Workspace& ws, hipStream_
 // device memory already) come with it and are stored at d_passes and d_unis
 hipError_t launch_front(const FrontTables* tables, PassDesc* d_passes, DevUniforms* d_unis, int npasses, const Workspace& ws,
                         int fblocks, int vblocks, hipStream_t s);
-// one workgroup per tile of dependency group `group` (ws.tile_shift selects the tile size)
-hipError_t launch_raster(const PassDesc* d_passes, int npasses, const Workspace& ws, int blocks, int group,
+// one workgroup of `waves` (2 or 4) waves per tile of dependency group `group` (ws.tile_shift selects the tile size)
+hipError_t launch_raster(const PassDesc* d_passes, int npasses, const Workspace& ws, int blocks, int group, int waves,
                          hipStream_t s);
 // the persistent raster over every pass of the sequence: `workgroups` workgroups take tiles from a queue
 hipError_t launch_raster_queue(const PassDesc* d_passes, int npasses, const Workspace& ws, int workgroups,
-                               hipStream_t s);
+                               int waves, hipStream_t s);
 hipError_t launch_fill32(uint32_t* dst, uint32_t value, size_t n, hipStream_t s);
 // One plane of w x h words into host-mapped memory, as k_present does (flip) or
 // as it is, in bands of `band` words; band i stored, flags[i] becomes epoch.

@@ -250,7 +250,6 @@ extern "C" int hana_render_frame_noalloc(hana_ctx* c, const hana_frame_desc* f) 
     ws.q_g0 = (uint32_t)tb[0];
     ws.q_dep_from = n == 2 ? (uint32_t)descs[1].tile0 : (uint32_t)tile0;
     ws.tile_shift = tshift;
-    ws.raster_waves = c->tuning.raster_waves;
     for (int i = 0; i < n; i++) {
         descs[i].vr = vr + voff[i];
         descs[i].vs = vs + vsoff[i];
@@ -277,11 +276,12 @@ extern "C" int hana_render_frame_noalloc(hana_ctx* c, const hana_frame_desc* f) 
     NA_TRY(launch_setup(d_desc, n, ws, fb, small_tris, s));
     NA_TRY(launch_clip(d_desc, ws, s));
     if (c->tuning.raster_wgs_per_cu > 0) {
-        NA_TRY(launch_raster_queue(d_desc, n, ws, c->tuning.raster_wgs_per_cu * c->num_cus, s));
+        NA_TRY(launch_raster_queue(d_desc, n, ws, c->tuning.raster_wgs_per_cu * c->num_cus,
+                                   c->tuning.raster_waves, s));
     } else {
         for (int g = 0; g < 2; g++)
             if (group_count[g])
-                NA_TRY(launch_raster(d_desc + group_first[g], group_count[g], ws, tb[g], g, s));
+                NA_TRY(launch_raster(d_desc + group_first[g], group_count[g], ws, tb[g], g, c->tuning.raster_waves, s));
     }
     NA_TRY(hipEventRecord(c->slot_done[0], s));
 #undef NA_TRY

@@ -225,7 +225,28 @@ int build_plan(hana_ctx* c, std::vector<PassSpec> specs, Plan& pl, const Tuning&
     pl.total_f = fo;
     pl.total_tiles = tile0;
     pl.tile_shift = tshift;
-    pl.raster_waves = tu.raster_waves;
+    // Waves per raster workgroup.  Until the caller sets a tuning, a group of
+    // many 16x16 tiles, so that their workgroups run in several rounds, takes
+    // two: a workgroup's life is mostly waits (for its pass, its tile's chunks,
+    // entries, indices and vertices, each behind the one before), and 13 of 2
+    // waves fit a CU where 8 of 4 do.  With fewer tiles, or with smaller
+    // triangles, more of which keep four waves busy, four are faster.  4 and 2
+    // waves, us per frame (frame-sized shadow map): 3840x2160 of 100,000 faces
+    // 129 and 98, of 1,000,000 (8 pixels each) 155 and 137; 2560x1440 of
+    // 300,000 (12) 80 and 73, of 1,000,000 (3.7) 98 and 109; 1920x1080 (8,160
+    // tiles) of 300,000 (7) 61 and 67; 1366x768 of 100,000 35 and 44.  A batch of
+    // 64 scenes of 1,000-200,000 faces, 128^2-1024^2, 421 and, in the parts that
+    // this takes, 412.
+    for (int g = 0; g < 2; g++) {
+        int64_t px = 0, faces = 0;
+        for (const PassSpec& s : specs)
+            if (s.group == g) {
+                px += (int64_t)s.target->w * s.target->h;
+                faces += s.mesh->F;
+            }
+        const bool two = !tu.set && tu.raster_wgs_per_cu == 0 && tshift == 4 && tb[g] >= 10000 && px >= 4 * faces;
+        pl.raster_waves[g] = two ? 2 : tu.raster_waves;
+    }
     pl.raster_wgs = tu.raster_wgs_per_cu > 0 ? tu.raster_wgs_per_cu * c->num_cus : 0;
     pl.q_g0 = (uint32_t)tb[0];
     pl.q_dep_from = pl.q_dep_from < (uint32_t)n ? (uint32_t)pl.descs[pl.q_dep_from].tile0 : (uint32_t)tile0;
@@ -399,7 +420,6 @@ int bind_plan(hana_ctx* c, Plan& pl, Arena& A, uint32_t min_bins, uint32_t min_p
     ws.q_g0 = pl.q_g0;
     ws.q_dep_from = pl.q_dep_from;
     ws.tile_shift = pl.tile_shift;
-    ws.raster_waves = pl.raster_waves;
     for (int g = 0; g < 2; g++)
         ws.tile_pass[g] = pl.group_count[g] > 0 && !pl.args
                               ? reinterpret_cast<const uint2*>(A.tables.as<char>() + pl.tp_off) + pl.tp_first[g]
@@ -501,14 +521,15 @@ int enqueue_raster(hana_ctx* c, const Plan& pl, const Arena& A, hipStream_t s, b
     const PassDesc* d = A.tables.as<PassDesc>();
     if (pl.raster_wgs > 0) {
         StageTimer t(c, 6, timed, s);
-        HIP_TRY(c, launch_raster_queue(d, (int)pl.descs.size(), pl.ws, pl.raster_wgs, s));
+        HIP_TRY(c, launch_raster_queue(d, (int)pl.descs.size(), pl.ws, pl.raster_wgs, pl.raster_waves[0], s));
         t.done(s);
         return HANA_OK;
     }
     for (int g = 0; g < 2; g++)
         if (pl.group_count[g]) {
             StageTimer t(c, 6 + g, timed, s);
-            HIP_TRY(c, launch_raster(d + pl.group_first[g], pl.group_count[g], pl.ws, pl.group_blocks[g], g, s));
+            HIP_TRY(c, launch_raster(d + pl.group_first[g], pl.group_count[g], pl.ws, pl.group_blocks[g], g,
+                                    pl.raster_waves[g], s));
             t.done(s);
         }
     return HANA_OK;
@@ -1803,6 +1824,7 @@ int hana_batch_autotune(hana_ctx* c, hana_batch* b, int use_graph, int reps, han
     if ((r = batch_check_new(c, b, "hana_batch_autotune"))) return r;
     if ((r = check_status(c)) || (r = join(c))) return r;
     Tuning best = b->tuning;
+    best.set = true;   // what is tried is what runs
     double best_ms = 0.0;
     auto measure = [&](const Tuning& t, double* ms) {
         b->tuning = t;

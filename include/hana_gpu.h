@@ -218,7 +218,8 @@ int hana_render_frame_noalloc(hana_ctx* ctx, const hana_frame_desc* f);
  * parts: the concurrent parts a batch is split into (1-4; ignored for
  * per-call draws).  Results are identical under every tuning.  Default: 16,
  * 0, 4 parts, 4 waves; until a tuning is set, per-call draws of few large
- * triangles on large targets take 32x32 tiles. */
+ * triangles on large targets take 32x32 tiles, and the rasters of many tiles
+ * with triangles that are not small 2 waves. */
 typedef struct hana_tuning {
     int32_t tile_size;
     int32_t raster_wgs_per_cu;

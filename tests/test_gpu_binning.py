@@ -53,6 +53,11 @@ CASES = {
     "tiles-16": (16_257, (1930, 1078), (4, 30), 1.0),
     "tiles-32": (16_253, (1930, 1078), (4, 30), 1.0),
     "tiles-32-clipped": (3000, (2049, 1025), (30, 90), 1.5),
+    # two waves per raster workgroup from 10,000 16x16 tiles and 4 pixels per face on
+    "waves-4-tiles": (30_000, (1584, 1600), (4, 30), 1.0),
+    "waves-2": (30_000, (1599, 1600), (4, 30), 1.0),
+    "waves-2-clipped": (200_000, (1600, 1600), (2, 9), 1.3),
+    "waves-4-faces": (640_001, (1600, 1600), (1, 4), 1.0),
 }
 
 
