@@ -137,8 +137,12 @@ constexpr size_t kStagePiece = size_t(8) << 20;
 #define HANA_DRAW_SLOTS 4
 #endif
 constexpr int kDrawSlots = HANA_DRAW_SLOTS;
-// launch sequences of at least this many faces use two of the slots
+// launch sequences of at least this many faces that draw into the target of the
+// call before take turns with it on two of the slots
 constexpr size_t kLargeSequenceFaces = size_t(1) << 19;
+// launch sequences of at least this many faces use two of the slots, whose
+// workspaces are 2 GB and more
+constexpr size_t kHugeSequenceFaces = size_t(1) << 24;
 // launch sequences of at most this many faces run their geometry in one launch
 #ifndef HANA_FRONT_FACES
 #define HANA_FRONT_FACES (1 << 18)
@@ -194,6 +198,7 @@ struct hana_ctx {
     // it touches one of them
     std::vector<hana_target*> pend[hana::rt::kDrawSlots][hana::rt::kDrawSlots];
     int next_slot = 0;
+    int last_slot = -1;          // of the last per-call draw
     bool pipelined = true;
     // device staging for hana_target_present
     hana::rt::DevBuf present;

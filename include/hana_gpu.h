@@ -25,8 +25,10 @@
  * A context owns four HIP streams, each with its own workspace, and every
  * device object created on it; calls on one context must be externally
  * synchronised.  Work is enqueued asynchronously: consecutive draws rotate
- * over the streams (over two of them for draws of 2^19 faces or more) so that
- * a draw's geometry stages overlap the rasters of the draws before it.  A
+ * over the streams (over two of them for draws of 2^24 faces or more, or of
+ * 2^19 into the target of the draw before; draws of up to 2^15 faces follow
+ * their target's last one on its stream) so that a draw's geometry stages
+ * overlap the rasters of the draws before it.  A
  * raster waits for every earlier draw that draws or samples one of its
  * targets or shadow maps, so each target sees the draws in call order; draws
  * on disjoint targets may run concurrently.  hana_target_read(_winner),
