@@ -496,7 +496,7 @@ def bench_c3(ctx, args, scenes, cpu):
     eager = Batch(ctx)
     for d in devs:
         eager.add(d.desc())
-    eager.set_tuning(chosen["tile_size"], chosen["raster_wgs_per_cu"], chosen["parts"])
+    eager.set_tuning(chosen["tile_size"], chosen["raster_wgs_per_cu"], chosen["parts"], chosen["raster_waves"])
     eager.finalize(use_graph=False)
     eager.run()
     stage_ms, launches = timed_stages(ctx, eager.run, reps)

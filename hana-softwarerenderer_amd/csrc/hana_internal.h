@@ -59,6 +59,7 @@ struct Tuning {
     int raster_wgs_per_cu = 0;            // 0: one raster workgroup per tile; else a persistent raster
     int raster_waves = 4;                  // waves per raster workgroup (2 or 4)
     int parts = 4;                         // concurrent parts of a batch
+    bool auto_waves = true;                // raster_waves, or 2 where build_plan finds them better
     bool set = false;                      // by the caller
 };
 

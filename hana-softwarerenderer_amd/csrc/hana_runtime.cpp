@@ -225,9 +225,8 @@ int build_plan(hana_ctx* c, std::vector<PassSpec> specs, Plan& pl, const Tuning&
     pl.total_f = fo;
     pl.total_tiles = tile0;
     pl.tile_shift = tshift;
-    // Waves per raster workgroup.  Until the caller sets a tuning, a group of
-    // many 16x16 tiles, so that their workgroups run in several rounds, takes
-    // two: a workgroup's life is mostly waits (for its pass, its tile's chunks,
+    // Waves per raster workgroup.  Until the caller sets them, a group of many
+    // 16x16 tiles, so that their workgroups run in several rounds, takes two: a workgroup's life is mostly waits (for its pass, its tile's chunks,
     // entries, indices and vertices, each behind the one before), and 13 of 2
     // waves fit a CU where 8 of 4 do.  With fewer tiles, or with smaller
     // triangles, more of which keep four waves busy, four are faster.  4 and 2
@@ -244,7 +243,7 @@ int build_plan(hana_ctx* c, std::vector<PassSpec> specs, Plan& pl, const Tuning&
                 px += (int64_t)s.target->w * s.target->h;
                 faces += s.mesh->F;
             }
-        const bool two = !tu.set && tu.raster_wgs_per_cu == 0 && tshift == 4 && tb[g] >= 10000 && px >= 4 * faces;
+        const bool two = tu.auto_waves && tu.raster_wgs_per_cu == 0 && tshift == 4 && tb[g] >= 10000 && px >= 4 * faces;
         pl.raster_waves[g] = two ? 2 : tu.raster_waves;
     }
     pl.raster_wgs = tu.raster_wgs_per_cu > 0 ? tu.raster_wgs_per_cu * c->num_cus : 0;
@@ -871,6 +870,7 @@ int tuning_from(hana_ctx* c, const hana_tuning* t, Tuning& out) {
     out.raster_wgs_per_cu = t->raster_wgs_per_cu;
     out.raster_waves = t->raster_waves ? t->raster_waves : 4;
     out.parts = t->parts;
+    out.auto_waves = t->raster_waves == 0;
     out.set = true;
     return HANA_OK;
 }
@@ -1827,7 +1827,6 @@ int hana_batch_autotune(hana_ctx* c, hana_batch* b, int use_graph, int reps, han
     if ((r = batch_check_new(c, b, "hana_batch_autotune"))) return r;
     if ((r = check_status(c)) || (r = join(c))) return r;
     Tuning best = b->tuning;
-    best.set = true;   // what is tried is what runs
     double best_ms = 0.0;
     auto measure = [&](const Tuning& t, double* ms) {
         b->tuning = t;
@@ -1848,8 +1847,10 @@ int hana_batch_autotune(hana_ctx* c, hana_batch* b, int use_graph, int reps, han
             const int curs[4] = {base.tile_shift, base.raster_wgs_per_cu, base.raster_waves, base.parts};
             int& field = *fields[dim];
             const int cur = curs[dim];
-            if (vals[i] == cur) continue;
+            const bool waves_dim = dim == 2;
+            if (vals[i] == cur && !(waves_dim && base.auto_waves)) continue;
             field = vals[i];
+            if (waves_dim) t.auto_waves = false;
             double ms = 0.0;
             if ((r = measure(t, &ms))) return r;
             if (ms < best_ms * (1.0 - kAutotuneMargin)) {

@@ -220,13 +220,13 @@ int hana_render_frame_noalloc(hana_ctx* ctx, const hana_frame_desc* f);
  * parts: the concurrent parts a batch is split into (1-4; ignored for
  * per-call draws).  Results are identical under every tuning.  Default: 16,
  * 0, 4 parts, 4 waves; until a tuning is set, per-call draws of few large
- * triangles on large targets take 32x32 tiles, and the rasters of many tiles
- * with triangles that are not small 2 waves. */
+ * triangles on large targets take 32x32 tiles.  Until they are set, or set to 0,
+ * the waves are 2 for rasters of many tiles with triangles that are not small. */
 typedef struct hana_tuning {
     int32_t tile_size;
     int32_t raster_wgs_per_cu;
     int32_t parts;
-    int32_t raster_waves;           /* waves per raster workgroup: 2 or 4 (0: 4) */
+    int32_t raster_waves;           /* waves per raster workgroup: 2 or 4 (0: chosen per raster) */
     double ms;                      /* hana_batch_autotune: measured run time of the choice */
 } hana_tuning;
 /* Tuning of the context's per-call draws (hana_draw, hana_render_frame). */
