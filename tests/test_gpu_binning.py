@@ -1,6 +1,8 @@
 """The GPU's binning at the sizes where its paths change, against the oracle:
 depth and the winning face of every pixel bit-exact, colour as in
 test_gpu_parity."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -92,3 +94,23 @@ def test_calls_on_one_target_keep_order(ctx, oracle, faces):
     assert_depth_exact(dep, o_big.depth, "target")
     assert_color_ok(col, o_big.color, "target")
     assert_depth_exact(ctx.read(smap, 160, 120)[1], o_smap.depth, "shadow map")
+
+
+@pytest.mark.parametrize("name", ["crowded-places", "wide-700", "front-scattered", "front-clipped"])
+def test_binning_in_fixed_scratch(ctx, oracle, name):
+    """The frame without allocation bins into a workspace of fixed size, with
+    every wide triangle listed and its own list behind the tiles' places."""
+    from hana_amd.gpu import build_uniforms
+    n, (w, h), px, spread = CASES[name]
+    scene = soup_scene(n, w, h, px[0], px[1], seed=700 + n)
+    scene.mesh.pos[:, :2] *= np.float32(spread)
+    target = ctx.target(w, h)
+    desc = ctx.frame_desc(ctx.mesh(scene.mesh), scene.shader, False, build_uniforms(scene), target, None,
+                          ctx.texture(scene.diffuse), ctx.texture(scene.normal))
+    ctx.sync()
+    ctx.check(ctx.lib.hana_render_frame_noalloc(ctx.h, C.byref(desc)), "noalloc")
+    col, dep = ctx.read(target, w, h)
+    ref = HostTarget(w, h)
+    oracle.draw(scene.mesh, scene.shader, oracle.build_uniforms(scene), ref, scene.diffuse, scene.normal)
+    assert_depth_exact(dep, ref.depth, name)
+    assert_color_ok(col, ref.color, name)
