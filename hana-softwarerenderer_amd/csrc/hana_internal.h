@@ -60,6 +60,7 @@ struct Tuning {
     int raster_waves = 4;                  // waves per raster workgroup (2 or 4)
     int parts = 4;                         // concurrent parts of a batch
     bool auto_waves = true;                // raster_waves, or 2 where build_plan finds them better
+    bool auto_parts = true;                // parts by the batch's tiles (batch_prepare)
     bool set = false;                      // by the caller
 };
 

@@ -871,6 +871,7 @@ int tuning_from(hana_ctx* c, const hana_tuning* t, Tuning& out) {
     out.raster_waves = t->raster_waves ? t->raster_waves : 4;
     out.parts = t->parts;
     out.auto_waves = t->raster_waves == 0;
+    out.auto_parts = false;
     out.set = true;
     return HANA_OK;
 }
@@ -1514,9 +1515,9 @@ static std::vector<double> frame_weights(const hana_batch* b) {
 
 // The end frame of each part when the frames, in order, are split into up to
 // b->tuning.parts parts of about equal estimated work w (one value per frame),
-// at most one part per frame.  Four parts measured best on 256 mixed scenes
-// (2.10 ms per batch, against 2.20 for two and 2.3-2.4 for six or eight): a
-// process gets four hardware queues, and more streams than that share them.
+// at most one part per frame.  Not more than four: six or eight were slower on
+// 256 mixed scenes, since a process gets four hardware queues, and more streams
+// than that share them.
 static std::vector<size_t> split_ends(const hana_batch* b, const std::vector<double>& w) {
     size_t nf = b->frame_first.size();
     size_t np = std::min(nf, std::min((size_t)b->tuning.parts, kMaxBatchParts));
@@ -1639,7 +1640,7 @@ static void batch_drop_graph(hana_batch* b) {
 }
 
 // Splits, sizes and (with use_graph) captures the batch for b->tuning.
-static int batch_prepare(hana_ctx* c, hana_batch* b, bool use_graph) {
+static int batch_prepare_parts(hana_ctx* c, hana_batch* b, bool use_graph) {
     int r;
     batch_drop_graph(b);
     std::vector<double> w = frame_weights(b);
@@ -1716,6 +1717,30 @@ static int batch_prepare(hana_ctx* c, hana_batch* b, bool use_graph) {
         HIP_TRY(c, hipGraphInstantiate(&b->exec, b->graph, nullptr, nullptr, 0));
     }
     return HANA_OK;
+}
+
+// The parts of a batch until the caller sets them, by its 16x16 tiles.  Each part
+// adds its launches to the graph, and with few tiles those are what a batch
+// takes; with many, more parts fill each other's tails.  1, 2 and 4 parts, us a
+// batch: 1,276 tiles 64, 75 and 98; 11,396 tiles 98, 108 and 113, of larger
+// meshes 113, 113 and 119; 16,973 tiles 143, 145 and 164; 22,464 tiles 166, 168
+// and 163; 23,208 tiles 215, 188 and 191; 33,414 tiles 221, 210 and 218; 93,766
+// tiles 430, 399 and 414; 390,000 tiles 1,282, 1,221 and 1,192.
+static int parts_for(const hana_batch* b) {
+    int64_t tiles = 0;
+    for (const PassSpec& s : b->specs) tiles += (int64_t)((s.target->w + 15) / 16) * ((s.target->h + 15) / 16);
+    return tiles <= 17000 ? 1 : (tiles <= 200000 ? 2 : 4);
+}
+
+static int batch_prepare(hana_ctx* c, hana_batch* b, bool use_graph) {
+    if (b->tuning.auto_parts) b->tuning.parts = parts_for(b);
+    int r = batch_prepare_parts(c, b, use_graph);
+    if (r == HANA_E_NOMEM && b->tuning.auto_parts && b->tuning.parts < 4) {
+        // more pairs than a part of this size may hold, or a workspace too large
+        b->tuning.parts = 4;
+        r = batch_prepare_parts(c, b, use_graph);
+    }
+    return r;
 }
 
 static int batch_check_new(hana_ctx* c, hana_batch* b, const char* what) {
@@ -1834,6 +1859,7 @@ int hana_batch_autotune(hana_ctx* c, hana_batch* b, int use_graph, int reps, han
         return e ? e : batch_time(c, b, reps, ms);
     };
     if ((r = measure(best, &best_ms))) return r;
+    best.parts = b->tuning.parts;
     const int shifts[] = {4, 5}, wgs[] = {0, 2, 4, 8}, waves[] = {4, 2}, parts[] = {1, 2, 4};
     const int* dims[4] = {shifts, wgs, waves, parts};
     const int counts[4] = {2, 4, 2, 3};
@@ -1851,6 +1877,7 @@ int hana_batch_autotune(hana_ctx* c, hana_batch* b, int use_graph, int reps, han
             if (vals[i] == cur && !(waves_dim && base.auto_waves)) continue;
             field = vals[i];
             if (waves_dim) t.auto_waves = false;
+            if (dim == 3) t.auto_parts = false;
             double ms = 0.0;
             if ((r = measure(t, &ms))) return r;
             if (ms < best_ms * (1.0 - kAutotuneMargin)) {

@@ -221,7 +221,9 @@ int hana_render_frame_noalloc(hana_ctx* ctx, const hana_frame_desc* f);
  * per-call draws).  Results are identical under every tuning.  Default: 16,
  * 0, 4 parts, 4 waves; until a tuning is set, per-call draws of few large
  * triangles on large targets take 32x32 tiles.  Until they are set, or set to 0,
- * the waves are 2 for rasters of many tiles with triangles that are not small. */
+ * the waves are 2 for rasters of many tiles with triangles that are not small.
+ * Until a batch's tuning is set it has 1 part up to 17,000 16x16 tiles, 2 up to
+ * 200,000. */
 typedef struct hana_tuning {
     int32_t tile_size;
     int32_t raster_wgs_per_cu;
