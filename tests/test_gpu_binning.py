@@ -114,3 +114,26 @@ def test_binning_in_fixed_scratch(ctx, oracle, name):
     oracle.draw(scene.mesh, scene.shader, oracle.build_uniforms(scene), ref, scene.diffuse, scene.normal)
     assert_depth_exact(dep, ref.depth, name)
     assert_color_ok(col, ref.color, name)
+
+
+@pytest.mark.parametrize("edge,parts", [(1040, 1), (1056, 2), (3568, 2), (3584, 4)])
+def test_batch_parts_by_tiles(ctx, edge, parts):
+    """Four frames of edge x edge: one part up to 17,000 16x16 tiles, two up to
+    200,000, four beyond; each with the images of the frames drawn one by one."""
+    from hana_amd.gpu import Batch, build_uniforms
+    batch, frames = Batch(ctx), []
+    for k in range(4):
+        s = soup_scene(200 + 100 * k, edge, edge, 10, 60, seed=800 + k)
+        u, mesh = build_uniforms(s), ctx.mesh(s.mesh)
+        tex = (ctx.texture(s.diffuse), ctx.texture(s.normal))
+        t, single = ctx.target(edge, edge), ctx.target(edge, edge)
+        batch.add(ctx.frame_desc(mesh, s.shader, False, u, t, None, *tex))
+        ctx.draw(mesh, s.shader, u, single, *tex)
+        frames.append((t, single))
+    batch.finalize(use_graph=True)
+    assert batch.tuning()["parts"] == parts
+    batch.run()
+    for t, single in frames:
+        got, want = ctx.read(t, edge, edge), ctx.read(single, edge, edge)
+        assert np.array_equal(got[0], want[0]) and got[1].tobytes() == want[1].tobytes()
+    batch.close()
