@@ -154,6 +154,10 @@ constexpr size_t kHugeSequenceFaces = size_t(1) << 24;
 #define HANA_FRONT_FACES (1 << 18)
 #endif
 constexpr size_t kFrontFaces = HANA_FRONT_FACES;
+// the same for a part of a batch, whose launches no other call's fill up: in
+// three launches and in one, a part of 296,000 faces 113 and 105 us a batch, two
+// parts of 801,000 together 189 and 190, of 1,036,000 146 and 154
+constexpr size_t kBatchFrontFaces = size_t(3) << 17;
 // sequences of at most this many faces draw on the slot that last drew into
 // their target: 16 small models into one target took 299 us over all slots,
 // whose waits for one another cost the host 14 us a call, and take 183

@@ -131,7 +131,7 @@ int materialize_clear(hana_ctx* c, hana_target* t, hipStream_t s) {
 // drawn by the first group come last: the persistent raster's queue holds the
 // tiles in pass order, so every shadow tile precedes the tiles that wait for
 // them.  Every per-pass slice is 1024-vertex aligned.
-int build_plan(hana_ctx* c, std::vector<PassSpec> specs, Plan& pl, const Tuning& tu) {
+int build_plan(hana_ctx* c, std::vector<PassSpec> specs, Plan& pl, const Tuning& tu, size_t front_faces) {
     {
         std::vector<std::pair<int, size_t>> key(specs.size());
         for (size_t i = 0; i < specs.size(); i++) {
@@ -159,7 +159,7 @@ int build_plan(hana_ctx* c, std::vector<PassSpec> specs, Plan& pl, const Tuning&
     int n = (int)specs.size();
     size_t faces = 0;
     for (const PassSpec& s : specs) faces += (size_t)s.mesh->F;
-    pl.front = faces <= kFrontFaces;
+    pl.front = faces <= front_faces;
     pl.args = pl.front && n <= FRONT_PASSES;
     const size_t vchunk = (size_t)BLOCK * (pl.front ? FRONT_VPT : VPT), fchunk = (size_t)BLOCK * (pl.front ? FRONT_FPT : FPT);
     pl.descs.resize(n);
@@ -789,7 +789,7 @@ int run_passes(hana_ctx* c, std::vector<PassSpec> specs) {
     }
     Plan pl;
     const Tuning tuning = call_tuning(c, specs);
-    if ((r = build_plan(c, std::move(specs), pl, tuning))) return r;
+    if ((r = build_plan(c, std::move(specs), pl, tuning, kFrontFaces))) return r;
     bool rotate = c->pipelined && !c->timing && !c->stats_enabled;
     // Large sequences into one target rotate over two slots: their rasters wait
     // for each other, and with a third in flight the 2.6 M faces of a 1.3 M-
@@ -1594,7 +1594,7 @@ static int batch_enqueue(hana_ctx* c, hana_batch* b, bool timed) {
 // Sizes a part's workspace exactly with trial runs.
 static int batch_size_part(hana_ctx* c, hana_batch* b, hana_batch_part& part) {
     int r;
-    if ((r = build_plan(c, part.specs, part.plan, b->tuning))) return r;
+    if ((r = build_plan(c, part.specs, part.plan, b->tuning, kBatchFrontFaces))) return r;
     uint32_t min_bins = 0, min_polys = 0;
     Arena& A = *part.arena;
     for (int attempt = 0; attempt < 3; attempt++) {

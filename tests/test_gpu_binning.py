@@ -137,3 +137,22 @@ def test_batch_parts_by_tiles(ctx, edge, parts):
         got, want = ctx.read(t, edge, edge), ctx.read(single, edge, edge)
         assert np.array_equal(got[0], want[0]) and got[1].tobytes() == want[1].tobytes()
     batch.close()
+
+
+@pytest.mark.parametrize("faces", [3 << 17, (3 << 17) + 1])
+def test_batch_part_at_the_one_launch_limit(ctx, faces):
+    """A batch's part of up to 3 x 2^17 faces runs its geometry in one launch,
+    a larger one in three: both render what the single draw does."""
+    from hana_amd.gpu import Batch, build_uniforms
+    s = soup_scene(faces, 640, 480, 1, 4, seed=900)
+    s.mesh.pos[:, :2] *= np.float32(1.2)
+    u, mesh, tex = build_uniforms(s), ctx.mesh(s.mesh), (ctx.texture(s.diffuse), ctx.texture(s.normal))
+    t, single = ctx.target(640, 480), ctx.target(640, 480)
+    batch = Batch(ctx)
+    batch.add(ctx.frame_desc(mesh, s.shader, False, u, t, None, *tex))
+    batch.finalize(use_graph=True)
+    ctx.draw(mesh, s.shader, u, single, *tex)
+    batch.run()
+    got, want = ctx.read(t, 640, 480), ctx.read(single, 640, 480)
+    assert np.array_equal(got[0], want[0]) and got[1].tobytes() == want[1].tobytes()
+    batch.close()
