@@ -419,6 +419,7 @@ constexpr int CLIP_THREADS = 512;
 #define HANA_CLIP_GRID 2048
 #endif
 constexpr int CLIP_GRID = HANA_CLIP_GRID;
+constexpr int COUNT_CLIP_GRID = 256;
 constexpr int CLIP_FACES = CLIP_THREADS / CLIP_GROUP;   // faces per workgroup and round
 constexpr int CLIP_NF = 4 + POLY_VARY;
 static_assert(POLY_MAX <= CLIP_GROUP, "one lane per polygon vertex");
@@ -796,17 +797,19 @@ __device__ __forceinline__ bool dies_at_first_crossed_plane(uint32_t c0, uint32_
 }
 
 // FPT faces per lane.  Trivially accepted faces are set up from the shared
-// post-transform vertices and binned; faces that clipping would remove are
-// dropped; the others are queued for k_clip with one global atomic per
-// workgroup.
-// Six waves per SIMD: the gathers of all FPT faces in flight take about 80
-// VGPRs; at 64 (eight waves) the compiler serialises them and the kernel is
-// slower, at 97 (five) it is slower too.
-template <int BITS, int TS>
-__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(6))) void k_setup(const PassDesc* __restrict__ passes, int npasses, Workspace ws) {
-    __shared__ SegLds<BITS, BLOCK, BLOCK * FPT> L;
-    __shared__ uint32_t s_nq, s_qbase;
-    if (threadIdx.x == 0) s_nq = 0;
+// post-transform vertices and listed, then binned by bin(pass); faces that
+// clipping would remove are dropped; the others are queued for k_clip with one
+// global atomic per workgroup.
+template <int BITS>
+struct SetupLds {
+    SegLds<BITS, BLOCK, BLOCK * FPT> seg;
+    uint32_t nq, qbase;
+};
+template <int BITS, int TS, class Bin>
+__device__ __forceinline__ void setup_block(SetupLds<BITS>& S, const PassDesc* passes, int npasses, const Workspace& ws, bool stats,
+                                            const Bin& bin) {
+    SegLds<BITS, BLOCK, BLOCK * FPT>& L = S.seg;
+    if (threadIdx.x == 0) S.nq = 0;
     int pass = find_pass<1>(passes, npasses, blockIdx.x);
     const PassDesc& P = passes[pass];
     int base = (blockIdx.x - P.fblock0) * BLOCK * FPT;
@@ -857,9 +860,9 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(6))) void
             bool clipq = clipped && !dies_at_first_crossed_plane(codes[k][0], codes[k][1], codes[k][2]);
             if (clipped && !clipq) gst(P.poly_of_face + f, -1);
             // faces to clip take the list's places from its end: a face is either
-            uint32_t q = wave_reserve_lds(&s_nq, clipq);
+            uint32_t q = wave_reserve_lds(&S.nq, clipq);
             if (clipq) L.entry[BLOCK * FPT - 1 - q] = (uint32_t)f;
-            if (P.stats) {
+            if (stats && P.stats) {
                 uint64_t nv = __popcll(__ballot(valid[k])), nc = __popcll(__ballot(clipped));
                 if (__lane_id() == 0) {
                     stat_add(P, ST_FACES, nv);
@@ -873,15 +876,26 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(6))) void
         }
     }
     lds_barrier();
-    if (threadIdx.x == 0) s_qbase = s_nq ? atomicAdd(&ws.seq[SEQ_CLIPQ], s_nq) : 0u;
-    const uint32_t own = blockIdx.x * (SEG_PAIRS * BLOCK * FPT);
-    bin_segment<false>(L, [&](uint32_t) -> const PassDesc& { return P; }, ws, own, own + SEG_PAIRS * BLOCK * FPT);
+    if (threadIdx.x == 0) S.qbase = S.nq ? atomicAdd(&ws.seq[SEQ_CLIPQ], S.nq) : 0u;
+    bin(P);
     __syncthreads();
-    for (uint32_t i = threadIdx.x; i < s_nq; i += BLOCK) {
-        uint32_t q = s_qbase + i;
+    for (uint32_t i = threadIdx.x; i < S.nq; i += BLOCK) {
+        uint32_t q = S.qbase + i;
         if (q < ws.clipq_cap) gst(ws.clip_queue + q, ((uint64_t)(uint32_t)pass << 32) | L.entry[BLOCK * FPT - 1 - i]);
         else raise_flag(ws, FLAG_CLIPQ_OVERFLOW);
     }
+}
+
+// Six waves per SIMD: the gathers of all FPT faces in flight take about 80
+// VGPRs; at 64 (eight waves) the compiler serialises them and the kernel is
+// slower, at 97 (five) it is slower too.
+template <int BITS, int TS>
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(6))) void k_setup(const PassDesc* __restrict__ passes, int npasses, Workspace ws) {
+    __shared__ SetupLds<BITS> S;
+    setup_block<BITS, TS>(S, passes, npasses, ws, true, [&](const PassDesc& P) {
+        const uint32_t own = blockIdx.x * (SEG_PAIRS * BLOCK * FPT);
+        bin_segment<false>(S.seg, [&](uint32_t) -> const PassDesc& { return P; }, ws, own, own + SEG_PAIRS * BLOCK * FPT);
+    });
 }
 
 // The LDS of a clipping round of FACES faces.
@@ -908,7 +922,7 @@ struct ClipLds {
 // round.
 template <int TS, int FACES, class Seg, class Listed>
 __device__ __forceinline__ void clip_round(ClipLds<FACES>& L, Seg& B, SegSums& sums, const PassDesc& P, Uniforms u, const Workspace& ws,
-                                           bool have, int f, const Listed& listed) {
+                                           bool have, int f, bool stats, const Listed& listed) {
     const int tid = threadIdx.x, lane = tid & 63, g = tid / CLIP_GROUP, li = tid % CLIP_GROUP;
     const uint64_t gmask = 0xFFFFull << (lane & ~(CLIP_GROUP - 1));
     if (tid == 0) L.npoly = 0;
@@ -990,7 +1004,7 @@ __device__ __forceinline__ void clip_round(ClipLds<FACES>& L, Seg& B, SegSums& s
     if (have && li == 0) {
         if (keep) {
             gst(ws.pool_face + pid, f);
-            stat_add(P, ST_POLYS, 1);
+            if (stats) stat_add(P, ST_POLYS, 1);
         }
         gst(P.poly_of_face + f, keep ? (int)pid : -1);
     }
@@ -1000,30 +1014,252 @@ __device__ __forceinline__ void clip_round(ClipLds<FACES>& L, Seg& B, SegSums& s
 }
 
 // Clips the queued faces, CLIP_FACES per workgroup and round, grid-stride over
-// the queue.
-template <int TS>
-__global__ __launch_bounds__(CLIP_THREADS) void k_clip(const PassDesc* __restrict__ passes, Workspace ws) {
-    constexpr int FANS = CLIP_FACES * (POLY_MAX - 2);
-    __shared__ ClipLds<CLIP_FACES> L;
-    __shared__ SegLds<10, CLIP_THREADS, FANS> B;
-    __shared__ int fan_pass[FANS];
+// the queue; a round's fan triangles are then binned by bin(pass_of).
+struct QueueLds {
+    static constexpr int FANS = CLIP_FACES * (POLY_MAX - 2);
+    ClipLds<CLIP_FACES> clip;
+    SegLds<10, CLIP_THREADS, FANS> seg;
+    int fan_pass[FANS];
+};
+template <int TS, class Bin>
+__device__ __forceinline__ void clip_queue(QueueLds& Q, const PassDesc* passes, const Workspace& ws, bool stats, const Bin& bin) {
     uint32_t count = min(ws.seq[SEQ_CLIPQ], ws.clipq_cap);
     for (uint32_t base = blockIdx.x * CLIP_FACES; base < count; base += gridDim.x * CLIP_FACES) {
-        seg_clear(B);
+        seg_clear(Q.seg);
         SegSums sums;
         uint32_t q = base + threadIdx.x / CLIP_GROUP;
         bool have = q < count;
         uint64_t e = have ? gld(ws.clip_queue + q) : 0ull;
         const int pass = (int)(e >> 32);
         const PassDesc& P = passes[pass];
-        clip_round<TS, CLIP_FACES>(L, B, sums, P, uniforms_of(P.u), ws, have, (int)(uint32_t)e,
-                                   [&](uint32_t at) { fan_pass[at] = pass; });
+        clip_round<TS, CLIP_FACES>(Q.clip, Q.seg, sums, P, uniforms_of(P.u), ws, have, (int)(uint32_t)e, stats,
+                                   [&](uint32_t at) { Q.fan_pass[at] = pass; });
         lds_barrier();
-        bin_segment<false>(B, [&](uint32_t i) -> const PassDesc& { return passes[fan_pass[i]]; }, ws, 0u, 0u);
+        bin([&](uint32_t i) -> const PassDesc& { return passes[Q.fan_pass[i]]; });
         __syncthreads();
     }
 }
+template <int TS>
+__global__ __launch_bounds__(CLIP_THREADS) void k_clip(const PassDesc* __restrict__ passes, Workspace ws) {
+    __shared__ QueueLds Q;
+    clip_queue<TS>(Q, passes, ws, true, [&](const auto& pass_of) { bin_segment<false>(Q.seg, pass_of, ws, 0u, 0u); });
+}
 
+// ---------------------------------------------------------------------------
+// counted binning: exact whatever the order and the sizes of the triangles
+// ---------------------------------------------------------------------------
+
+// How many descriptors the chunked binning takes depends on the order of the
+// faces and on the order in which workgroups and lanes arrive.  Counted binning
+// takes one bin entry per (triangle, tile) pair and nothing else: set-up and
+// clipping run once to count every tile's pairs, a scan gives each tile its
+// range of the bins, and they run again to place them (the pool's polygons are
+// made anew, in whatever order the second run takes them).  The raster gets a
+// tile's range as its one chunk.  It costs a second set-up, so it is the way
+// out where the chunks do not fit.
+struct Counted {
+    uint32_t* pairs;         // per global tile, zero at first
+    uint32_t* next;          // per global tile: where its next pair goes
+    const uint32_t* first;   // or null: counters of the chunked binning before; only where that did not fit anything runs
+    uint32_t region;         //   its Workspace::seg_region
+    uint32_t place;          // the second run
+};
+
+// Whether the chunked binning whose counters are given ran out of descriptors
+// or bins, and of nothing else.
+__device__ __forceinline__ bool chunks_ran_out(const uint32_t* seq, uint32_t region, const Workspace& ws) {
+    const uint64_t pairs = ((uint64_t)seq[SEQ_PAIRS] | ((uint64_t)seq[SEQ_PAIRS + 1] << 32)) + region;
+    const uint64_t wide = (uint64_t)seq[SEQ_WIDE_PAIRS] | ((uint64_t)seq[SEQ_WIDE_PAIRS + 1] << 32);
+    return !(seq[SEQ_FLAGS] & FLAG_NO_RASTER) && pairs + wide <= MAX_PAIRS && (pairs > ws.bin_cap || seq[SEQ_OVER] > ws.over_cap);
+}
+__device__ __forceinline__ bool counted_runs(const Workspace& ws, const Counted& q) {
+    if (q.place) return ws.seq[SEQ_COUNTED] != 0u;
+    return !q.first || chunks_ran_out(q.first, q.region, ws);
+}
+
+// The counters of the chunked binning, for the raster: what it asked for is
+// met.  (Its own kernels' conditions no longer read them.)
+__device__ __forceinline__ void counters_met(const Workspace& ws, const Counted& q) {
+    uint32_t* seq = const_cast<uint32_t*>(q.first);
+    const uint64_t pairs = (uint64_t)ws.seq[SEQ_PAIRS] | ((uint64_t)ws.seq[SEQ_PAIRS + 1] << 32);
+    const uint64_t past = pairs > q.region ? pairs - q.region : 0u;
+    seq[SEQ_PAIRS] = (uint32_t)past;
+    seq[SEQ_PAIRS + 1] = (uint32_t)(past >> 32);
+    seq[SEQ_OVER] = 0u;
+    seq[SEQ_MAX_CHUNKS] = 0u;
+}
+
+// A triangle over more than WIDE_TILES tiles: listed if the pass's list holds
+// them all (wide_cap > 0), else counted or placed by the whole wave in each of
+// its tiles.  Past the pair limit, where nothing is rasterised, counting stops.
+__device__ __forceinline__ void count_wide(const PassDesc& P, const Workspace& ws, const Counted& q, bool wide, const TileSpan& s) {
+    if (!__ballot(wide)) return;
+    uint32_t n = 0;
+    bool each = false;
+    if (wide) {
+        n = (uint32_t)s.nx() * (uint32_t)s.ny();
+        if (ws.wide_cap) {
+            if (q.place) {
+                uint32_t idx = gadd(ws.wide_count + P.index, 1u);
+                if (idx < ws.wide_cap)
+                    gst2(ws.wide + (size_t)P.index * ws.wide_cap + idx,
+                         make_uint2(wide_box(wide_shift(P), s.x0(), s.y0(), s.x0() + s.nx() - 1, s.y0() + s.ny() - 1), s.entry));
+            }
+        } else {
+            each = q.place || seq_add64(ws, SEQ_PAIRS, n) + n <= MAX_PAIRS;
+        }
+    }
+    uint64_t mask = __ballot(each);
+    int tile0 = P.tile0, tiles_x = P.tiles_x;
+    while (mask) {
+        int src = __ffsll((unsigned long long)mask) - 1;
+        mask &= mask - 1;
+        int wn = __shfl((int)n, src), wnx = __shfl(s.nx(), src), wx0 = __shfl(s.x0(), src), wy0 = __shfl(s.y0(), src);
+        int wt0 = __shfl(tile0, src), wtx = __shfl(tiles_x, src);
+        uint32_t we = __shfl(s.entry, src);
+        for (int k = __lane_id(); k < wn; k += 64) {
+            uint32_t gt = (uint32_t)(wt0 + (wy0 + k / wnx) * wtx + wx0 + k % wnx);
+            if (q.place) {
+                uint32_t pos = gadd(q.next + gt, 1u);
+                if (pos < ws.bin_cap) gst(ws.bins + pos, we);
+            } else {
+                gadd(q.pairs + gt, 1u);
+            }
+        }
+    }
+}
+
+// Counts or places the pairs of the listed triangles: per tile in the LDS
+// table, with one global atomic per distinct tile, or where the table has no
+// slot left for the tile with one per pair.
+template <int BITS, int THREADS, int CAP, class PassOf>
+__device__ __forceinline__ void count_segment(SegLds<BITS, THREADS, CAP>& L, const PassOf& pass_of, const Workspace& ws, const Counted& q) {
+    const int tid = threadIdx.x;
+    const uint32_t n = L.n;
+    if (!n) return;
+    uint32_t* const at_tile = q.place ? q.next : q.pairs;
+    uint32_t mine = 0;
+    for (uint32_t i0 = 0; i0 < n; i0 += THREADS) {   // uniform
+        const uint32_t i = i0 + (uint32_t)tid;
+        const bool have = i < n;
+        TileSpan t{0u, 0u, 0u};
+        if (have) t = TileSpan{L.entry[i], L.t0[i], L.t1[i]};
+        const PassDesc& P = pass_of(have ? i : 0u);
+        const int nx = t.nx(), nt = nx * t.ny();
+        const bool wide = have && nt > WIDE_TILES;
+        count_wide(P, ws, q, wide, t);
+        if (have && !q.place && P.stats) stat_add(P, ST_ENTRIES, (uint64_t)nt);
+        if (!have || wide) continue;
+        mine += (uint32_t)nt;
+        for (int k = 0; k < nt; k++) {
+            const uint32_t gt = (uint32_t)(P.tile0 + (t.y0() + k / nx) * P.tiles_x + t.x0() + k % nx);
+            const int sl = bin_slot<BITS>(L.keys, gt, true);
+            if (sl >= 0) {
+                atomicAdd(&L.cnt[sl], 1u);
+            } else {
+                const uint32_t pos = gadd(at_tile + gt, 1u);
+                if (q.place && pos < ws.bin_cap) gst(ws.bins + pos, t.entry);
+            }
+        }
+    }
+    if (!q.place) {
+        const uint32_t sum = wave_scan(mine);
+        if (__lane_id() == 63 && sum) seq_add64(ws, SEQ_PAIRS, sum);
+    }
+    lds_barrier();
+    for (int sl = tid; sl < (1 << BITS); sl += THREADS)
+        if (const uint32_t c = L.cnt[sl]) L.cnt[sl] = gadd(at_tile + L.keys[sl], c);
+    lds_barrier();
+    if (!q.place) return;
+    for (uint32_t i = (uint32_t)tid; i < n; i += THREADS) {
+        const TileSpan t{L.entry[i], L.t0[i], L.t1[i]};
+        const int nx = t.nx(), nt = nx * t.ny();
+        if (nt > WIDE_TILES) continue;
+        const PassDesc& P = pass_of(i);
+        for (int k = 0; k < nt; k++) {
+            const uint32_t gt = (uint32_t)(P.tile0 + (t.y0() + k / nx) * P.tiles_x + t.x0() + k % nx);
+            const int sl = bin_slot<BITS>(L.keys, gt, false);
+            if (sl < 0) continue;   // placed above: a tile that found no slot never does
+            const uint32_t pos = atomicAdd(&L.cnt[sl], 1u);
+            if (pos < ws.bin_cap) gst(ws.bins + pos, t.entry);
+        }
+    }
+}
+
+template <int TS>
+__global__ __launch_bounds__(BLOCK) void k_setup_counted(const PassDesc* __restrict__ passes, int npasses, Workspace ws, Counted q) {
+    __shared__ SetupLds<10> S;
+    if (!counted_runs(ws, q)) return;
+    setup_block<10, TS>(S, passes, npasses, ws, !q.place, [&](const PassDesc& P) {
+        count_segment(S.seg, [&](uint32_t) -> const PassDesc& { return P; }, ws, q);
+    });
+}
+template <int TS>
+__global__ __launch_bounds__(CLIP_THREADS) void k_clip_counted(const PassDesc* __restrict__ passes, Workspace ws, Counted q) {
+    __shared__ QueueLds Q;
+    if (!counted_runs(ws, q)) return;
+    if (q.place && q.first && blockIdx.x == 0 && threadIdx.x == 0) counters_met(ws, q);
+    clip_queue<TS>(Q, passes, ws, !q.place, [&](const auto& pass_of) { count_segment(Q.seg, pass_of, ws, q); });
+}
+
+// Gives every tile its range of the bins, one workgroup per SCAN_TILES tiles
+// (each sums the counts before its own), and the raster that range as the
+// tile's chunks; then the counters are as before the first run, for the second
+// one.  Where the pairs do not fit the second run does not take place.
+constexpr int SCAN_THREADS = 1024, SCAN_TILES = 4 * SCAN_THREADS;
+constexpr uint32_t CHUNK_MAX = 1u << 30;   // entries of a chunk
+__device__ __forceinline__ uint32_t scan_sum(uint32_t* sh, uint32_t v, uint32_t* before) {
+    const int w = threadIdx.x >> 6;
+    const uint32_t incl = wave_scan(v);
+    if (__lane_id() == 63) sh[w] = incl;
+    __syncthreads();
+    uint32_t all = 0, lower = 0;
+    for (int k = 0; k < SCAN_THREADS / 64; k++) {
+        if (k < w) lower += sh[k];
+        all += sh[k];
+    }
+    __syncthreads();
+    if (before) *before = lower + incl - v;
+    return all;
+}
+__global__ __launch_bounds__(SCAN_THREADS) void k_count_scan(Workspace ws, Counted q) {
+    __shared__ uint32_t sh[SCAN_THREADS / 64];
+    if (!counted_runs(ws, q)) return;
+    const uint64_t pairs = (uint64_t)ws.seq[SEQ_PAIRS] | ((uint64_t)ws.seq[SEQ_PAIRS + 1] << 32);
+    if ((ws.seq[SEQ_FLAGS] & FLAG_NO_RASTER) || pairs > ws.bin_cap) return;   // uniform
+    const uint32_t n = ws.q_items, first = blockIdx.x * (uint32_t)SCAN_TILES;
+    uint32_t v = 0;
+    for (uint32_t t = threadIdx.x; t < first; t += SCAN_THREADS) v += gld(q.pairs + t);
+    uint32_t at = scan_sum(sh, v, nullptr);
+    const uint32_t t0 = first + threadIdx.x * 4u;
+    uint32_t c[4];
+    v = 0;
+    for (uint32_t k = 0; k < 4u; k++) {
+        c[k] = t0 + k < n ? gld(q.pairs + t0 + k) : 0u;
+        v += c[k];
+    }
+    uint32_t before;
+    scan_sum(sh, v, &before);
+    at += before;
+    for (uint32_t k = 0; k < 4u && t0 + k < n; k++) {
+        const uint32_t t = t0 + k;
+        gst(q.next + t, at);
+        uint32_t chunks = 0;
+        for (uint32_t left = c[k]; left && chunks < ws.chunk_cap; chunks++) {
+            const uint32_t m = min(left, CHUNK_MAX);
+            gst2(ws.chunks + ((size_t)t * ws.chunk_cap + chunks), make_uint2(at + (c[k] - left), m));
+            left -= m;
+        }
+        gst(ws.tile_chunks + t, chunks);
+        at += c[k];
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        ws.seq[SEQ_COUNTED] = 1u;
+        ws.seq[SEQ_POLYS] = 0u;
+        ws.seq[SEQ_CLIPQ] = 0u;
+        for (uint32_t* w = ws.wide_count; w < ws.tile_chunks; w++) *w = 0u;
+    }
+}
 // The geometry of a whole sequence in one launch.  Workgroups below nfb take
 // FRONT_FPT faces per lane: they run the vertex program on the faces' own
 // corners instead of waiting for the vertices of a launch before (each vertex
@@ -1130,7 +1366,7 @@ __global__ __launch_bounds__(BLOCK) void k_front(FrontTables tables, PassDesc* _
         while (q0 < nq && L.n <= BLOCK * FRONT_FPT) {   // uniform
             uint32_t q = q0 + threadIdx.x / CLIP_GROUP;
             bool have = q < nq;
-            clip_round<TS, FACES>(C, L, sums, P, *up, ws, have, have ? (int)s_queue[q] : 0, [](uint32_t) {});
+            clip_round<TS, FACES>(C, L, sums, P, *up, ws, have, have ? (int)s_queue[q] : 0, true, [](uint32_t) {});
             q0 += FACES;
         }
         seg_sums(L, sums);
@@ -1883,6 +2119,26 @@ hipError_t launch_clip(const PassDesc* d_passes, const Workspace& ws, hipStream_
     if (ws.tile_shift == 5) hipLaunchKernelGGL(k_clip<5>, dim3(CLIP_GRID), dim3(CLIP_THREADS), 0, s, d_passes, ws);
     else hipLaunchKernelGGL(k_clip<4>, dim3(CLIP_GRID), dim3(CLIP_THREADS), 0, s, d_passes, ws);
     return hipGetLastError();
+}
+hipError_t launch_counted(const PassDesc* d_passes, int npasses, const Workspace& ws, const CountedBins& b, int blocks, hipStream_t s) {
+    Counted q{b.pairs, b.next, b.first, b.region, 0u};
+    const int scan = (int)((ws.q_items + SCAN_TILES - 1) / SCAN_TILES);
+    for (q.place = 0; q.place < 2u; q.place++) {
+        hipError_t e;
+        if (q.place) {
+            hipLaunchKernelGGL(k_count_scan, dim3(std::max(scan, 1)), dim3(SCAN_THREADS), 0, s, ws, Counted{b.pairs, b.next, b.first, b.region, 0u});
+            if ((e = hipGetLastError()) != hipSuccess) return e;
+        }
+        if (blocks > 0) {
+            if (ws.tile_shift == 5) hipLaunchKernelGGL(k_setup_counted<5>, dim3(blocks), dim3(BLOCK), 0, s, d_passes, npasses, ws, q);
+            else hipLaunchKernelGGL(k_setup_counted<4>, dim3(blocks), dim3(BLOCK), 0, s, d_passes, npasses, ws, q);
+            if ((e = hipGetLastError()) != hipSuccess) return e;
+        }
+        if (ws.tile_shift == 5) hipLaunchKernelGGL(k_clip_counted<5>, dim3(COUNT_CLIP_GRID), dim3(CLIP_THREADS), 0, s, d_passes, ws, q);
+        else hipLaunchKernelGGL(k_clip_counted<4>, dim3(COUNT_CLIP_GRID), dim3(CLIP_THREADS), 0, s, d_passes, ws, q);
+        if ((e = hipGetLastError()) != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
 hipError_t launch_front(const FrontTables* tables, PassDesc* d_passes, DevUniforms* d_unis, int npasses, const Workspace& ws,
                         int fblocks, int vblocks, hipStream_t s) {

@@ -10,6 +10,16 @@ hipError_t launch_vertex(const PassDesc* d_passes, int npasses, const Workspace&
 hipError_t launch_setup(const PassDesc* d_passes, int npasses, const Workspace& ws, int blocks, bool small_tris,
                         hipStream_t s);
 hipError_t launch_clip(const PassDesc* d_passes, const Workspace& ws, hipStream_t s);
+// Set-up and clipping twice, to count and then to place every pair (after the
+// vertices).  With `first`, the counters of a chunked binning before, all of it
+// runs only where that one ran out of descriptors or bins.
+struct CountedBins {
+    uint32_t* pairs;         // per tile, zero
+    uint32_t* next;          // per tile
+    uint32_t* first;
+    uint32_t region;         // the chunked binning's Workspace::seg_region
+};
+hipError_t launch_counted(const PassDesc* d_passes, int npasses, const Workspace& ws, const CountedBins& b, int blocks, hipStream_t s);
 // vertex, set-up and clipping in one launch; `tables` (or null: they are in
 // device memory already) come with it and are stored at d_passes and d_unis
 hipError_t launch_front(const FrontTables* tables, PassDesc* d_passes, DevUniforms* d_unis, int npasses, const Workspace& ws,

@@ -160,9 +160,11 @@ extern "C" int hana_render_frame_noalloc(hana_ctx* c, const hana_frame_desc* f) 
     // on it whatever the layout below needs: 12 bytes per tile, the vertices'
     // and faces' arrays, 28 KiB (24 in passes of small triangles) per 1,024
     // faces, the clip pool and, at least, four bin entries per face and two
-    // per tile.
+    // per tile.  Such a frame may have as many (triangle, tile) pairs as words
+    // are left then, whatever the order of its faces.
     const size_t ntiles = (size_t)std::max(tile0, 1), segs = std::max<size_t>(fb, 1);
     const uint64_t poly_cap = std::min<uint64_t>(tf / 256 + 1024, POOL_CAP_MAX);
+    size_t nominal_bins;
     {
         Carver nom{nullptr, 0, kNoAllocScratchBytes};
         nom.take<char>(2 * 264);
@@ -189,6 +191,7 @@ extern "C" int hana_render_frame_noalloc(hana_ctx* c, const hana_frame_desc* f) 
             return fail(c, HANA_E_NOMEM,
                         "hana_render_frame_noalloc: the frame needs more workspace than the " +
                             std::to_string(kNoAllocScratchBytes >> 20) + " MiB no-alloc scratch holds; use hana_render_frame");
+        nominal_bins = words;
     }
 
     // the workspace, carved from the scratch array
@@ -197,40 +200,41 @@ extern "C" int hana_render_frame_noalloc(hana_ctx* c, const hana_frame_desc* f) 
     DevUniforms* d_uni = cv.take<DevUniforms>(2);
     Workspace ws{};
     ws.status = cv.take<uint32_t>(STATUS_WORDS);
-    const size_t counters = (size_t)SEQ_WORDS + 4 + ((ntiles + 3) & ~(size_t)3);
+    // counters of the chunked binning, then of the counted one (launch_counted):
+    // its own and its pairs per tile
+    const size_t tile_words = (ntiles + 3) & ~(size_t)3, chunked = (size_t)SEQ_WORDS + 4 + tile_words;
+    const size_t counters = chunked + SEQ_WORDS + tile_words;
     ws.seq = cv.take<uint32_t>(counters);
+    uint32_t* const next = cv.take<uint32_t>(ntiles);
     float4* vr = cv.take<float4>(tv);
     float* vs = cv.take<float>(tvs);
     uint8_t* code = cv.take<uint8_t>(tv);
     int32_t* pof = cv.take<int32_t>(tf);
-    // every wide triangle is listed: a descriptor in each of its tiles would
-    // take more than the bin entry there that the nominal size counts
-    const size_t wide_cap = (size_t)f->mesh->F + 8 * poly_cap;
+    // every wide triangle is listed: they take no bin entries
+    const size_t wide_cap = (size_t)f->mesh->F + (POLY_MAX - 2) * poly_cap;
     ws.wide = cv.take<uint2>(wide_cap * n);
     ws.clip_queue = cv.take<uint64_t>(std::max<size_t>(tf, 1024));
     ws.pool_vr = cv.take<float4>(POLY_MAX * poly_cap);
     ws.pool_vs = cv.take<float>(POLY_MAX * POLY_VARY * poly_cap);
     ws.pool_face = cv.take<int32_t>(poly_cap);
-    // of what is left, the set-up workgroups' own bin entries and beside them
-    // as many as the nominal size counts (narrow triangles have at most 16
-    // each), then of the spare words half for the tiles' chunk descriptors, or
-    // a quarter where that is more than an allocated workspace starts with
-    // (bind_plan), and a quarter for the list behind them
+    // What is left goes to the tiles' chunk descriptors and the bins.  Chunked
+    // binning may run out of either, by the order of the faces; counted binning
+    // then needs an entry per pair of the narrow triangles, at most 16 each.  Of
+    // the words beyond those the descriptors take half, or a quarter where that
+    // is more than an allocated workspace starts with (bind_plan), but one a tile.
     const uint64_t seg_region = (uint64_t)fb * SEG_PAIRS * BLOCK * FPT;
-    const size_t min_bins = (size_t)seg_region + std::min(16 * tf, 4 * tf + 2 * ((size_t)tile0 + 1)) + 64;
+    const size_t tris = tf + (POLY_MAX - 2) * std::min<size_t>(poly_cap, tf);
     size_t left = cv.fits() ? (kNoAllocScratchBytes - cv.off) / sizeof(uint32_t) : 0;
     left = left > 256 ? left - 256 : 0;
+    const size_t min_bins = std::max<size_t>(seg_region + tf + 64, std::min(WIDE_TILES * tris, nominal_bins));
     const size_t spare = left > min_bins ? left - min_bins : 0;
     const size_t per_face = tf / ntiles + 1;
     const size_t want_cap = std::max<size_t>(std::min<size_t>(8 * per_face, std::max<size_t>(512, 2 * per_face)), 64) + CHUNK_SLACK;
     size_t cap = std::min(spare / 4 / ntiles, std::max(want_cap, spare / 8 / ntiles));
     if (cap >= 8) cap = 4 * (cap / 4 - 1 + (cap / 4 & 1));   // an odd number of 32-byte groups
     cap = std::max<size_t>(cap, 1);
-    const size_t over_cap = spare > 2 * cap * ntiles ? std::min(spare / 4, spare - 2 * cap * ntiles) / 4 : 0;
     ws.chunks = cv.take<uint2>(cap * ntiles);
     ws.chunk_cap = (uint32_t)cap;
-    ws.over = cv.take<uint4>(over_cap);
-    ws.over_cap = (uint32_t)over_cap;
     ws.wide_cap = (uint32_t)wide_cap;
     left = cv.fits() ? (kNoAllocScratchBytes - cv.off) / sizeof(uint32_t) : 0;
     const size_t bins_cap = std::min<size_t>(left, MAX_PAIRS);
@@ -250,6 +254,10 @@ extern "C" int hana_render_frame_noalloc(hana_ctx* c, const hana_frame_desc* f) 
     ws.q_g0 = (uint32_t)tb[0];
     ws.q_dep_from = n == 2 ? (uint32_t)descs[1].tile0 : (uint32_t)tile0;
     ws.tile_shift = tshift;
+    Workspace counted = ws;
+    counted.seq = ws.seq + chunked;
+    counted.seg_region = 0;
+    const CountedBins bins{counted.seq + SEQ_WORDS, next, ws.seq, (uint32_t)seg_region};
     for (int i = 0; i < n; i++) {
         descs[i].vr = vr + voff[i];
         descs[i].vs = vs + vsoff[i];
@@ -275,6 +283,7 @@ extern "C" int hana_render_frame_noalloc(hana_ctx* c, const hana_frame_desc* f) 
     NA_TRY(launch_vertex(d_desc, n, ws, vb, s));
     NA_TRY(launch_setup(d_desc, n, ws, fb, small_tris, s));
     NA_TRY(launch_clip(d_desc, ws, s));
+    NA_TRY(launch_counted(d_desc, n, counted, bins, fb, s));
     if (c->tuning.raster_wgs_per_cu > 0) {
         NA_TRY(launch_raster_queue(d_desc, n, ws, c->tuning.raster_wgs_per_cu * c->num_cus,
                                    c->tuning.raster_waves, s));

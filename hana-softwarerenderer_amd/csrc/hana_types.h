@@ -209,9 +209,10 @@ constexpr uint32_t OVER_MIN = 1024;        // Workspace::over_cap at first
 // clipping, the flags it raised, the descriptors past their tiles' places and
 // the most chunks of one such tile, the persistent raster's queue, and (64-bit
 // each) the pairs outside the set-up workgroups' own entries and the pairs of
-// the listed wide triangles
+// the listed wide triangles; of counted binning, all pairs in the first of them,
+// and whether they fit
 enum { SEQ_POLYS = 0, SEQ_CLIPQ = 1, SEQ_FLAGS = 2, SEQ_OVER = 3, SEQ_PAIRS = 4, SEQ_WIDE_PAIRS = 6,
-       SEQ_QUEUE = 8, SEQ_QUEUE_DONE = 9, SEQ_MAX_CHUNKS = 10, SEQ_WORDS = 16 };
+       SEQ_QUEUE = 8, SEQ_QUEUE_DONE = 9, SEQ_MAX_CHUNKS = 10, SEQ_COUNTED = 11, SEQ_WORDS = 16 };
 // status words: set across sequences until the host reads them at a sync
 // point, so that calls need not wait for one another: the flags of every
 // sequence and the largest needs seen: of places for descriptors, in units of
