@@ -79,7 +79,7 @@ struct Arena {
     int counters_next = 0;
     uint32_t bin_cap = 0, poly_cap = 0, clipq_cap = 0;
     uint64_t chunk_slots = 0;   // descriptors the chunks buffer holds
-    uint32_t over_cap = 0, wide_cap = WIDE_MAX;
+    uint32_t over_cap = 0;
 };
 
 struct Plan {
@@ -104,7 +104,8 @@ struct Plan {
     int raster_waves[2] = {4, 4};   // per raster group (the persistent raster: the first)
     int raster_wgs = 0;       // workgroups of the persistent raster (0: one per tile and group)
     bool front = false;       // geometry in one launch (k_front)
-    bool args = false;        // ... which brings the tables as arguments (no upload, no pass lookup)
+    bool counted = false;     // counted binning (launch_counted) instead of chunks
+    bool args = false;        // front, and the launch brings the tables as arguments (no upload, no pass lookup)
     uint32_t q_g0 = 0, q_dep_from = 0;
     Workspace ws{};
 };
@@ -232,6 +233,10 @@ struct hana_ctx {
     std::vector<hana::rt::LoggedCall> log;
     bool replay_overflow = true;
     int64_t replays = 0;   // status checks that rendered the logged calls again
+    // per-call sequences of at least these faces and tiles bin by counting: the
+    // least of those whose descriptors the workspaces do not grow to
+    size_t counted_faces = ~size_t(0), counted_tiles = ~size_t(0);
+    bool count_next = false;   // without replay_overflow: so does the next one, which renders a failed one again
     // hana_render_frame_noalloc: the device address of this GPU's scratch
     // array, host-mapped status words of its sequences, whether one ran
     // since the last status check, and the draw slots that must wait for it

@@ -1399,11 +1399,10 @@ __device__ __forceinline__ bool sequence_fits(const Workspace& ws, bool publish)
             atomicMax(&ws.status[STATUS_NEED_BINS], (uint32_t)pairs);
             if (f & FLAG_CHUNK_OVERFLOW) {
                 uint64_t slots = ((uint64_t)ws.seq[SEQ_MAX_CHUNKS] + CHUNK_SLACK) * ws.q_items >> 10;
-                uint32_t wide = 0u;
-                for (const uint32_t* w = ws.wide_count; w < ws.tile_chunks; w++) wide = max(wide, *w);
                 atomicMax(&ws.status[STATUS_NEED_CHUNKS], (uint32_t)(slots < 0xFFFFFFFFu ? slots + 1u : slots));
                 atomicMax(&ws.status[STATUS_NEED_OVER], q[SEQ_OVER]);
-                atomicMax(&ws.status[STATUS_NEED_WIDE], wide);
+                atomicMax(&ws.status[STATUS_OVER_FACES], ~ws.faces);
+                atomicMax(&ws.status[STATUS_OVER_TILES], ~ws.q_items);
             }
         }
         atomicMax(&ws.status[STATUS_NEED_POLYS], q[SEQ_POLYS]);

@@ -246,6 +246,7 @@ extern "C" int hana_render_frame_noalloc(hana_ctx* c, const hana_frame_desc* f) 
     ws.zero = ws.seq;
     ws.zero_n = (uint32_t)counters;
     ws.bin_cap = (uint32_t)bins_cap;
+    ws.faces = (uint32_t)tf;
     ws.seg_region = (uint32_t)seg_region;
     ws.poly_cap = (uint32_t)poly_cap;
     ws.clipq_cap = (uint32_t)std::max<size_t>(tf, 1024);

@@ -131,7 +131,7 @@ int materialize_clear(hana_ctx* c, hana_target* t, hipStream_t s) {
 // drawn by the first group come last: the persistent raster's queue holds the
 // tiles in pass order, so every shadow tile precedes the tiles that wait for
 // them.  Every per-pass slice is 1024-vertex aligned.
-int build_plan(hana_ctx* c, std::vector<PassSpec> specs, Plan& pl, const Tuning& tu, size_t front_faces) {
+int build_plan(hana_ctx* c, std::vector<PassSpec> specs, Plan& pl, const Tuning& tu, size_t front_faces, bool counted) {
     {
         std::vector<std::pair<int, size_t>> key(specs.size());
         for (size_t i = 0; i < specs.size(); i++) {
@@ -159,7 +159,8 @@ int build_plan(hana_ctx* c, std::vector<PassSpec> specs, Plan& pl, const Tuning&
     int n = (int)specs.size();
     size_t faces = 0;
     for (const PassSpec& s : specs) faces += (size_t)s.mesh->F;
-    pl.front = faces <= front_faces;
+    pl.counted = counted;
+    pl.front = !counted && faces <= front_faces;
     pl.args = pl.front && n <= FRONT_PASSES;
     const size_t vchunk = (size_t)BLOCK * (pl.front ? FRONT_VPT : VPT), fchunk = (size_t)BLOCK * (pl.front ? FRONT_FPT : FPT);
     pl.descs.resize(n);
@@ -282,9 +283,10 @@ int build_plan(hana_ctx* c, std::vector<PassSpec> specs, Plan& pl, const Tuning&
 }
 
 // Words of a sequence's counters: the SEQ_* words, the passes' wide triangles,
-// the tiles' chunks.
+// the tiles' chunks; with counted binning, also the tiles' pairs and next places.
+static size_t tile_words(const Plan& pl) { return ((size_t)pl.total_tiles + 3) & ~(size_t)3; }
 static size_t counter_words(const Plan& pl) {
-    return (size_t)SEQ_WORDS + ((pl.descs.size() + 3) & ~(size_t)3) + (((size_t)pl.total_tiles + 3) & ~(size_t)3);
+    return (size_t)SEQ_WORDS + ((pl.descs.size() + 3) & ~(size_t)3) + (pl.counted ? 3 : 1) * tile_words(pl);
 }
 
 // Points the plan's workspace at counter set k of the arena.
@@ -329,7 +331,7 @@ int bind_plan(hana_ctx* c, Plan& pl, Arena& A, uint32_t min_bins, uint32_t min_p
     size_t nt = (size_t)pl.total_tiles + 1;
     // (triangle, tile) entries: most triangles touch one tile and about half
     // are culled; the raster reports the exact need if this is exceeded
-    const uint64_t seg_region = (uint64_t)pl.fblocks * SEG_PAIRS * BLOCK * (pl.front ? FRONT_FPT : FPT);
+    const uint64_t seg_region = pl.counted ? 0 : (uint64_t)pl.fblocks * SEG_PAIRS * BLOCK * (pl.front ? FRONT_FPT : FPT);
     uint64_t want_bins = std::max<uint64_t>({(uint64_t)min_bins, (uint64_t)4 * pl.total_f + 2 * nt, 1u << 22,
                                              seg_region + (uint64_t)pl.total_f + 4096});
     if (seg_region + 4096 > MAX_PAIRS) return fail(c, HANA_E_NOMEM, "launch sequence too large (triangle list)");
@@ -345,6 +347,7 @@ int bind_plan(hana_ctx* c, Plan& pl, Arena& A, uint32_t min_bins, uint32_t min_p
     const uint64_t tiles = (uint64_t)std::max(pl.total_tiles, 1), per_face = pl.total_f / tiles + 1;
     uint64_t want_cap = std::min<uint64_t>(8 * per_face, std::max<uint64_t>(512, 2 * per_face));
     want_cap = std::max<uint64_t>(want_cap, tiles > (1u << 20) ? 16 : 64) + CHUNK_SLACK;
+    if (pl.counted) want_cap = 32;   // a tile's range of the bins
     uint64_t want_slots = tiles * want_cap;
     if (want_slots > A.chunk_slots) {
         if ((r = ensure(c, A.chunks, sizeof(uint2) * want_slots))) return r;
@@ -352,7 +355,7 @@ int bind_plan(hana_ctx* c, Plan& pl, Arena& A, uint32_t min_bins, uint32_t min_p
     }
     A.over_cap = std::max(A.over_cap, OVER_MIN);
     if ((r = ensure(c, A.over, sizeof(uint4) * A.over_cap))) return r;
-    if ((r = ensure(c, A.wide, sizeof(uint2) * A.wide_cap * std::max(n, 1)))) return r;
+    if ((r = ensure(c, A.wide, sizeof(uint2) * WIDE_MAX * std::max(n, 1)))) return r;
     uint64_t want_polys = std::max<uint64_t>({(uint64_t)min_polys, pl.total_f / 16 + 4096});
     want_polys = std::min<uint64_t>(want_polys, POOL_CAP_MAX);
     if (want_polys > A.poly_cap) {
@@ -399,7 +402,7 @@ int bind_plan(hana_ctx* c, Plan& pl, Arena& A, uint32_t min_bins, uint32_t min_p
     ws.over = A.over.as<uint4>();
     ws.over_cap = A.over_cap;
     ws.wide = A.wide.as<uint2>();
-    ws.wide_cap = A.wide_cap;
+    ws.wide_cap = pl.counted ? 0 : WIDE_MAX;
     ws.pool_vr = A.pool_vr.as<float4>();
     ws.pool_vs = A.pool_vs.as<float>();
     ws.pool_face = A.pool_face.as<int32_t>();
@@ -413,6 +416,7 @@ int bind_plan(hana_ctx* c, Plan& pl, Arena& A, uint32_t min_bins, uint32_t min_p
     ws.status = A.status.as<uint32_t>();
     ws.status_out = nullptr;
     ws.bin_cap = A.bin_cap;
+    ws.faces = (uint32_t)std::min<size_t>(pl.total_f, 0xFFFFFFFFu);
     ws.seg_region = (uint32_t)seg_region;
     ws.poly_cap = A.poly_cap;
     ws.q_items = (uint32_t)pl.total_tiles;
@@ -473,7 +477,7 @@ struct StageTimer {
 
 // The geometry stages: vertex, set-up with binning, clipping; or all of them
 // in one launch (timed as set-up), before which a sequence that zeroes its own
-// counters does so.
+// counters does so; or vertex and counted binning (also timed as set-up).
 int enqueue_geometry(hana_ctx* c, const Plan& pl, const Arena& A, hipStream_t s, bool timed) {
     PassDesc* d = A.tables.as<PassDesc>();
     int n = (int)pl.descs.size();
@@ -500,6 +504,13 @@ int enqueue_geometry(hana_ctx* c, const Plan& pl, const Arena& A, hipStream_t s,
         StageTimer t(c, 0, timed, s);
         HIP_TRY(c, launch_vertex(d, n, pl.ws, pl.vblocks, s));
         t.done(s);
+    }
+    if (pl.counted) {
+        StageTimer t(c, 1, timed, s);
+        uint32_t* const pairs = pl.ws.tile_chunks + tile_words(pl);
+        HIP_TRY(c, launch_counted(d, n, pl.ws, {pairs, pairs + tile_words(pl), nullptr, 0}, pl.fblocks, s));
+        t.done(s);
+        return HANA_OK;
     }
     {
         StageTimer t(c, 1, timed, s);
@@ -584,23 +595,25 @@ struct Needs {
     }
 };
 
-// Grows an arena's chunk descriptors to the needs of an overflow.  The list
-// behind the tiles' places holds all that came after those; the places grow to
-// the fullest tile's need where that is up to 2^25 over all tiles (256 MB),
-// else, for few crowded tiles of large targets, by as many as came after.
-// More than 2^26 of them are wide triangles in each of their tiles: those are
-// then listed once each.
+// Whether an arena's chunk descriptors grow to the needs of an overflow: up to
+// 2^26 past the tiles' places, and any number that the tiles take in places.
+// Sequences that need more bin by counting.
+static uint64_t full_places(const Needs& need) { return (uint64_t)need.w[STATUS_NEED_CHUNKS] * 1024 / 4 * 5; }
+static bool chunks_grow(const Needs& need) {
+    return need.w[STATUS_NEED_OVER] <= (1u << 26) || full_places(need) <= (1u << 25);
+}
+
+// Grows them.  The list behind the tiles' places holds all that came after
+// those; the places grow to the fullest tile's need where that is up to 2^25
+// over all tiles (256 MB), else, for few crowded tiles of large targets, by as
+// many as came after.
 static int grow_chunks(hana_ctx* c, Arena& A, const Needs& need) {
     int r;
-    const uint64_t past = need.w[STATUS_NEED_OVER], full = (uint64_t)need.w[STATUS_NEED_CHUNKS] * 1024 / 4 * 5;
-    if (past > (1u << 26)) {
-        A.wide_cap = std::max(A.wide_cap, need.w[STATUS_NEED_WIDE]);   // bind_plan allocates
-    } else {
-        const uint64_t want = full <= (1u << 25) ? std::max(full, A.chunk_slots) : A.chunk_slots + past / 4 * 5;
-        if ((r = ensure(c, A.chunks, sizeof(uint2) * want))) return r;
-        A.chunk_slots = want;
-        A.over_cap = std::max<uint32_t>(A.over_cap, (uint32_t)(past / 4 * 5 + OVER_MIN));
-    }
+    const uint64_t past = need.w[STATUS_NEED_OVER], full = full_places(need);
+    const uint64_t want = full <= (1u << 25) ? std::max(full, A.chunk_slots) : A.chunk_slots + past / 4 * 5;
+    if ((r = ensure(c, A.chunks, sizeof(uint2) * want))) return r;
+    A.chunk_slots = want;
+    A.over_cap = std::max<uint32_t>(A.over_cap, (uint32_t)(std::min<uint64_t>(past, 1u << 26) / 4 * 5 + OVER_MIN));
     return HANA_OK;
 }
 
@@ -616,7 +629,7 @@ static int grow_arena(hana_ctx* c, Arena& A, const Needs& need) {
         if (r) return r;
         A.bin_cap = (uint32_t)want;
     }
-    if (flags & FLAG_CHUNK_OVERFLOW) {
+    if ((flags & FLAG_CHUNK_OVERFLOW) && chunks_grow(need)) {
         int r = grow_chunks(c, A, need);
         if (r) return r;
     }
@@ -632,10 +645,30 @@ static int grow_arena(hana_ctx* c, Arena& A, const Needs& need) {
     return HANA_OK;
 }
 
+// Whether a per-call sequence of this size bins by counting.
+static bool bins_by_counting(const hana_ctx* c, size_t faces, size_t tiles) {
+    return c->count_next || (faces >= c->counted_faces && tiles >= c->counted_tiles);
+}
+
 // Renders a logged call again on the context stream with slot 0's workspace
 // (every stream is idle: the status check has waited for them).
-static int replay_call(hana_ctx* c, LoggedCall& L) {
+static int replay_call(hana_ctx* c, LoggedCall& L, bool counted) {
     int r;
+    if (counted && !L.pl.counted) {
+        // laid out anew, with the clears that the call took
+        Tuning t;
+        t.tile_shift = L.pl.tile_shift;
+        if (c->num_cus > 0) t.raster_wgs_per_cu = L.pl.raster_wgs / c->num_cus;
+        Plan pl;
+        if ((r = build_plan(c, L.pl.specs, pl, t, 0, true))) return r;
+        for (size_t i = 0; i < pl.descs.size(); i++) {
+            const PassDesc& d = L.pl.descs[i];
+            pl.descs[i].clear = d.clear;
+            pl.descs[i].clear_rgba = d.clear_rgba;
+            pl.descs[i].clear_depth = d.clear_depth;
+        }
+        L.pl = std::move(pl);
+    }
     Plan& pl = L.pl;
     Arena& A = slot_arena(c, 0);
     if ((r = bind_plan(c, pl, A, 0, 0, false, c->stream))) return r;
@@ -661,7 +694,10 @@ static int replay_call(hana_ctx* c, LoggedCall& L) {
 //   largest need seen and the calls since the last check are rendered again
 //   in call order; a draw over the same state twice leaves it as drawn once
 //   (the depth test keeps the last of the fragments at the minimum depth), so
-//   the targets end as the calls in order leave them.  With replay_overflow
+//   the targets end as the calls in order leave them.  What the chunked binning
+//   needs varies with the order in which workgroups arrive, so the second time
+//   they bin by counting, whose needs are exact; so do, from then on, sequences
+//   like one whose descriptors no workspace grows to.  With replay_overflow
 //   off, the caller is asked to render again (HANA_E_OVERFLOW).
 // - More (triangle, tile) pairs than 32-bit bins reach: that sequence was not
 //   rasterised (HANA_E_NOMEM).
@@ -700,10 +736,14 @@ int check_status(hana_ctx* c) {
                     c->status_pending = false;
                     return r;
                 }
-        if (cap && c->replay_overflow && attempt < 3) {
+        if ((cap & FLAG_CHUNK_OVERFLOW) && !chunks_grow(need)) {
+            c->counted_faces = std::min<size_t>(c->counted_faces, ~need.w[STATUS_OVER_FACES]);
+            c->counted_tiles = std::min<size_t>(c->counted_tiles, ~need.w[STATUS_OVER_TILES]);
+        }
+        if (cap && c->replay_overflow && attempt < 4) {
             c->replays++;
             for (LoggedCall& L : c->log)
-                if ((r = replay_call(c, L))) {
+                if ((r = replay_call(c, L, attempt > 0 || bins_by_counting(c, L.pl.total_f, L.pl.total_tiles)))) {
                     c->log.clear();
                     c->status_pending = false;
                     return r;
@@ -712,9 +752,10 @@ int check_status(hana_ctx* c) {
         }
         c->log.clear();
         c->status_pending = false;
+        c->count_next = cap && !c->replay_overflow;
         if (cap)
             return fail(c, HANA_E_OVERFLOW,
-                        c->replay_overflow ? "workspace capacity still exceeded after growing it three times"
+                        c->replay_overflow ? "workspace capacity still exceeded after growing it four times"
                                            : "bin or clip-pool capacity exceeded since the last sync; buffers were "
                                              "grown, render those frames again");
         break;
@@ -789,7 +830,13 @@ int run_passes(hana_ctx* c, std::vector<PassSpec> specs) {
     }
     Plan pl;
     const Tuning tuning = call_tuning(c, specs);
-    if ((r = build_plan(c, std::move(specs), pl, tuning, kFrontFaces))) return r;
+    size_t faces = 0, tiles = 0;
+    for (const PassSpec& s : specs) {
+        const int edge = tile_edge(tuning.tile_shift);
+        faces += (size_t)s.mesh->F;
+        tiles += (size_t)((s.target->w + edge - 1) / edge) * ((s.target->h + edge - 1) / edge);
+    }
+    if ((r = build_plan(c, std::move(specs), pl, tuning, kFrontFaces, bins_by_counting(c, faces, tiles)))) return r;
     bool rotate = c->pipelined && !c->timing && !c->stats_enabled;
     // Large sequences into one target rotate over two slots: their rasters wait
     // for each other, and with a third in flight the 2.6 M faces of a 1.3 M-
@@ -955,7 +1002,6 @@ static void free_arena(Arena& a) {
     a.bin_cap = a.poly_cap = a.clipq_cap = 0;
     a.chunk_slots = 0;
     a.over_cap = 0;
-    a.wide_cap = WIDE_MAX;
     a.counters_used[0] = a.counters_used[1] = 0;
 }
 
@@ -1594,10 +1640,13 @@ static int batch_enqueue(hana_ctx* c, hana_batch* b, bool timed) {
 // Sizes a part's workspace exactly with trial runs.
 static int batch_size_part(hana_ctx* c, hana_batch* b, hana_batch_part& part) {
     int r;
-    if ((r = build_plan(c, part.specs, part.plan, b->tuning, kBatchFrontFaces))) return r;
     uint32_t min_bins = 0, min_polys = 0;
+    bool counted = false;
     Arena& A = *part.arena;
-    for (int attempt = 0; attempt < 3; attempt++) {
+    for (int attempt = 0; attempt < 6; attempt++) {
+        if ((attempt == 0 || counted != part.plan.counted) &&
+            (r = build_plan(c, part.specs, part.plan, b->tuning, kBatchFrontFaces, counted)))
+            return r;
         if ((r = bind_plan(c, part.plan, A, min_bins, min_polys, false, c->stream))) return r;
         batch_clear_flags(part);
         HIP_TRY(c, hipMemcpy(A.tables.p, part.plan.descs.data(), sizeof(PassDesc) * part.plan.descs.size(),
@@ -1627,7 +1676,10 @@ static int batch_size_part(hana_ctx* c, hana_batch* b, hana_batch_part& part) {
         min_polys = st[STATUS_NEED_POLYS] + st[STATUS_NEED_POLYS] / 8 + 1024;
         Needs need;
         need.take(st);
-        if ((st[STATUS_FLAGS] & FLAG_CHUNK_OVERFLOW) && (r = grow_chunks(c, A, need))) return r;
+        // as in check_status: by counting where the descriptors do not grow that
+        // far, or when growing them was not enough
+        if (attempt >= 2 || ((st[STATUS_FLAGS] & FLAG_CHUNK_OVERFLOW) && !chunks_grow(need))) counted = true;
+        else if ((st[STATUS_FLAGS] & FLAG_CHUNK_OVERFLOW) && (r = grow_chunks(c, A, need))) return r;
     }
     return fail(c, HANA_E_OVERFLOW, "hana_batch_finalize: capacity not reached");
 }

@@ -159,6 +159,7 @@ struct Workspace {
     uint32_t* status;            // see STATUS_*
     uint32_t* status_out;        // or null: host-mapped copy of the status words, written by the raster
     uint32_t bin_cap;
+    uint32_t faces;              // of all passes
     uint32_t seg_region;         // bin entries that belong to one set-up workgroup each; the rest is shared
     uint32_t poly_cap;
     uint32_t clipq_cap;
@@ -196,8 +197,8 @@ constexpr uint32_t SEG_PAIRS = 2;          // bin entries of a set-up workgroup,
 constexpr uint32_t CHUNK_INLINE = 0x80000000u;
 constexpr uint32_t CHUNK_SLACK = 16;       // places per tile beyond a reported need
 // Triangles over more than WIDE_TILES tiles are listed once per pass, up to
-// Workspace::wide_cap of them (WIDE_MAX at first); later ones take a descriptor
-// in each of their tiles.
+// Workspace::wide_cap of them (WIDE_MAX, or none or all with counted binning);
+// later ones take a descriptor in each of their tiles.
 constexpr int WIDE_TILES = 16;
 #ifndef HANA_WIDE_MAX
 #define HANA_WIDE_MAX 512
@@ -216,10 +217,11 @@ enum { SEQ_POLYS = 0, SEQ_CLIPQ = 1, SEQ_FLAGS = 2, SEQ_OVER = 3, SEQ_PAIRS = 4,
 // status words: set across sequences until the host reads them at a sync
 // point, so that calls need not wait for one another: the flags of every
 // sequence and the largest needs seen: of places for descriptors, in units of
-// 1024 over all tiles of the sequence; of the list behind them; of wide
-// triangles in one pass.
+// 1024 over all tiles of the sequence; of the list behind them; and the
+// complements of the faces and tiles of the smallest sequences that ran out of
+// descriptors.
 enum { STATUS_FLAGS = 0, STATUS_NEED_BINS = 1, STATUS_NEED_POLYS = 2, STATUS_NEED_CHUNKS = 3, STATUS_NEED_OVER = 4,
-       STATUS_NEED_WIDE = 5, STATUS_WORDS = 6 };
+       STATUS_OVER_FACES = 5, STATUS_OVER_TILES = 6, STATUS_WORDS = 7 };
 enum { FLAG_BIN_OVERFLOW = 1, FLAG_POLY_OVERFLOW = 2, FLAG_POLY_TOO_LARGE = 4, FLAG_CLIPQ_OVERFLOW = 8,
        FLAG_CHUNK_OVERFLOW = 16, FLAG_PAIR_LIMIT = 32, FLAG_QUEUE_STALL = 64 };
 // A workspace capacity ran out: the sequence is incomplete, its rasters write

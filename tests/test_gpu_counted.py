@@ -9,7 +9,8 @@ import pytest
 from hana_amd import scenegen as sg
 from parity import assert_color_ok, assert_depth_exact
 from pyoracle import CPURenderer, HostTarget
-from test_gpu_parity import soup_scene
+from test_gpu_parity import soup_scene, straddling_scene
+from test_gpu_serve import collect
 
 pytestmark = pytest.mark.gpu
 
@@ -19,9 +20,9 @@ def oracle():
     return CPURenderer("oracle")
 
 
-def layered_scene(layers, nx, ny, width, height, seed, kind=sg.TEXTURE, fill=0.98, order="random"):
+def layered_scene(layers, nx, ny, width, height, seed, kind=sg.TEXTURE, fill=0.98, jitter=0.3):
     """Planes of nx x ny quads that fill the view from (0, 0, 2), one behind the
-    other, jittered, with their faces in random order or row by row."""
+    other, jittered, with their faces in random order."""
     rng = np.random.default_rng(seed)
     gx, gy = np.meshgrid(np.linspace(-1, 1, nx + 1), np.linspace(-1, 1, ny + 1))
     q = np.arange((nx + 1) * (ny + 1), dtype=np.int32).reshape(ny + 1, nx + 1)
@@ -30,13 +31,12 @@ def layered_scene(layers, nx, ny, width, height, seed, kind=sg.TEXTURE, fill=0.9
     for k in range(layers):
         z = 0.5 - k / layers
         half = (2.0 - z) * np.tan(np.radians(30.0)) * fill
-        jit = rng.uniform(-0.3, 0.3, (2,) + gx.shape)
+        jit = rng.uniform(-jitter, jitter, (2,) + gx.shape)
         pos.append(np.stack([(gx + jit[0] * 2 / nx * (np.abs(gx) < 1)) * half * width / height,
                              (gy + jit[1] * 2 / ny * (np.abs(gy) < 1)) * half, np.full_like(gx, z)], -1).reshape(-1, 3))
         idx.append(quad + k * q.size)
     pos, idx = np.concatenate(pos).astype(np.float32), np.concatenate(idx)
-    if order == "random":
-        idx = idx[rng.permutation(len(idx))]
+    idx = idx[rng.permutation(len(idx))]
     nrm = np.zeros_like(pos)
     nrm[:, 2] = 1.0
     uv = np.tile(np.stack([(gx + 1) / 2, (gy + 1) / 2], -1).reshape(-1, 2), (layers, 1))
@@ -90,3 +90,75 @@ def test_noalloc_whatever_the_order(oracle, name, tile, wgs):
             ref = oracle_image(oracle, s)
             assert_depth_exact(dep, ref.depth, s.name)
             assert_color_ok(col, ref.color, s.name)
+
+
+def test_more_descriptors_than_a_workspace_grows_to():
+    """7.5 million triangles in random order, of 9 to 16 tiles each: 95 million
+    descriptors, where a workspace has places for 16 million.  The draw gives the
+    image that its faces give in eight draws, in their order; so does a batch,
+    and neither needs rendering again from then on."""
+    from hana_amd.gpu import Batch, Context, build_uniforms
+    scene = layered_scene(3720, 42, 24, 1920, 1080, 11, fill=1.008, jitter=0.0)
+    mesh = scene.mesh
+    with Context(0) as ctx:
+        u = build_uniforms(scene)
+        tex = (ctx.texture(scene.diffuse), ctx.texture(scene.normal))
+        whole, parts, batched = (ctx.target(1920, 1080) for _ in range(3))
+        m = ctx.mesh(mesh)
+        ctx.draw(m, scene.shader, u, whole, *tex)
+        got = [ctx.read(whole, 1920, 1080)]
+        replays = ctx.replay_count()
+        for k in range(2):
+            ctx.clear(whole)
+            ctx.draw(m, scene.shader, u, whole, *tex)
+            got.append(ctx.read(whole, 1920, 1080))
+        assert ctx.replay_count() == replays
+        batch = Batch(ctx)
+        batch.add(ctx.frame_desc(m, scene.shader, False, u, batched, None, *tex))
+        batch.finalize(use_graph=True)
+        batch.run()
+        batch.run()
+        got.append(ctx.read(batched, 1920, 1080))
+        batch.close()
+    with Context(0) as ctx:
+        tex = (ctx.texture(scene.diffuse), ctx.texture(scene.normal))
+        parts = ctx.target(1920, 1080)
+        for f in np.array_split(mesh.idx, 8):
+            ctx.draw(ctx.mesh(sg.Mesh(mesh.pos, mesh.nrm, mesh.uv, np.ascontiguousarray(f))), scene.shader, u, parts, *tex)
+            ctx.sync()
+        col, dep = ctx.read(parts, 1920, 1080)
+    assert (dep < 1e30).mean() > 0.99
+    for c, d in got:
+        assert d.tobytes() == dep.tobytes() and np.array_equal(c, col)
+
+
+def test_counted_beside_an_overflow(oracle):
+    """A server's batch that outgrew its lane's workspace is launched again with
+    counted binning: frames of few and of many faces, of odd sizes, clipped, with
+    triangles of one tile and of hundreds, with and without shadow maps."""
+    from hana_amd.gpu import Context, Server
+    scenes = [straddling_scene()]
+    for k, (w, h, n) in enumerate([(65, 47, 1), (333, 217, 255), (1, 1, 40), (700, 900, 1025), (1930, 1078, 5000),
+                                   (97, 61, 20_000), (640, 480, 700)]):
+        s = soup_scene(n, w, h, *((100, 400) if n == 700 else (2, 90)), 60 + n)
+        s.mesh.pos[:, :2] *= np.float32(1.2)
+        s.shadow = k % 2 == 0
+        scenes.append(s)
+    first = soup_scene(1000, 3840, 2160, 2, 30, 3)
+    with Context(0) as ctx:
+        objects = [(ctx.mesh(s.mesh), ctx.texture(s.diffuse), ctx.texture(s.normal)) for s in [first] + scenes]
+        # the first has a batch's pixels by itself; the others arrive while the
+        # lane is busy with it, and are taken together
+        server = Server(ctx, lanes=1, max_batch_frames=16, max_batch_pixels=8_000_000, return_depth=True)
+        for k, (s, (m, d, n)) in enumerate(zip([first] + scenes, objects)):
+            server.submit(m, s.shader, s.shadow, s.width, s.height, s.cam_pos, s.light_pos, d, n, tag=k)
+        res = collect(server, 1 + len(scenes))
+        st = server.stats()
+        server.close()
+    assert st["retries"] >= 1 and max(v[2] for v in res.values()) == len(scenes)
+    for k, s in enumerate(scenes):
+        status, img, _, dep = res[1 + k]
+        ref, _, _ = oracle.render_frame(s)
+        assert status == 0, s.name
+        assert_depth_exact(dep, ref.depth, s.name)
+        assert_color_ok(img, ref.color, s.name)
