@@ -476,17 +476,12 @@ __device__ __forceinline__ void lds_barrier() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-// Stores descriptor idx of tile gt: past the tile's places, in the list of the
-// sequence; past that it is lost, the sequence rasterises nothing and the host
-// renders it again with more of both.
+// Stores descriptor idx of tile gt.  Past the tile's places it is lost, and the
+// sequence rasterises nothing: the host renders it again with more of them, or
+// by counting.
 __device__ __forceinline__ void put_chunk(const Workspace& ws, uint32_t gt, uint32_t idx, uint2 d) {
-    if (idx < ws.chunk_cap) {
-        gst2(ws.chunks + ((size_t)gt * ws.chunk_cap + idx), d);
-        return;
-    }
-    atomicMax(&ws.seq[SEQ_MAX_CHUNKS], idx + 1u);
-    uint32_t o = atomicAdd(&ws.seq[SEQ_OVER], 1u);
-    if (o < ws.over_cap) ws.over[o] = make_uint4(gt, d.x, d.y, 0u);
+    if (idx < ws.chunk_cap) gst2(ws.chunks + ((size_t)gt * ws.chunk_cap + idx), d);
+    else atomicMax(&ws.seq[SEQ_MAX_CHUNKS], idx + 1u);
 }
 
 // The tiles of a triangle to be binned: bin entry, first and last tile.
@@ -1070,7 +1065,7 @@ struct Counted {
 __device__ __forceinline__ bool chunks_ran_out(const uint32_t* seq, uint32_t region, const Workspace& ws) {
     const uint64_t pairs = ((uint64_t)seq[SEQ_PAIRS] | ((uint64_t)seq[SEQ_PAIRS + 1] << 32)) + region;
     const uint64_t wide = (uint64_t)seq[SEQ_WIDE_PAIRS] | ((uint64_t)seq[SEQ_WIDE_PAIRS + 1] << 32);
-    return !(seq[SEQ_FLAGS] & FLAG_NO_RASTER) && pairs + wide <= MAX_PAIRS && (pairs > ws.bin_cap || seq[SEQ_OVER] > ws.over_cap);
+    return !(seq[SEQ_FLAGS] & FLAG_NO_RASTER) && pairs + wide <= MAX_PAIRS && (pairs > ws.bin_cap || seq[SEQ_MAX_CHUNKS]);
 }
 __device__ __forceinline__ bool counted_runs(const Workspace& ws, const Counted& q) {
     if (q.place) return ws.seq[SEQ_COUNTED] != 0u;
@@ -1085,7 +1080,6 @@ __device__ __forceinline__ void counters_met(const Workspace& ws, const Counted&
     const uint64_t past = pairs > q.region ? pairs - q.region : 0u;
     seq[SEQ_PAIRS] = (uint32_t)past;
     seq[SEQ_PAIRS + 1] = (uint32_t)(past >> 32);
-    seq[SEQ_OVER] = 0u;
     seq[SEQ_MAX_CHUNKS] = 0u;
 }
 
@@ -1392,15 +1386,14 @@ __device__ __forceinline__ bool sequence_fits(const Workspace& ws, bool publish)
         f |= FLAG_PAIR_LIMIT;
     } else {
         if (pairs > ws.bin_cap) f |= FLAG_BIN_OVERFLOW;
-        if (q[SEQ_OVER] > ws.over_cap) f |= FLAG_CHUNK_OVERFLOW;
+        if (q[SEQ_MAX_CHUNKS]) f |= FLAG_CHUNK_OVERFLOW;
     }
     if (publish) {
         if (!(f & FLAG_PAIR_LIMIT)) {
             atomicMax(&ws.status[STATUS_NEED_BINS], (uint32_t)pairs);
             if (f & FLAG_CHUNK_OVERFLOW) {
-                uint64_t slots = ((uint64_t)ws.seq[SEQ_MAX_CHUNKS] + CHUNK_SLACK) * ws.q_items >> 10;
+                uint64_t slots = ((uint64_t)q[SEQ_MAX_CHUNKS] + CHUNK_SLACK) * ws.q_items >> 10;
                 atomicMax(&ws.status[STATUS_NEED_CHUNKS], (uint32_t)(slots < 0xFFFFFFFFu ? slots + 1u : slots));
-                atomicMax(&ws.status[STATUS_NEED_OVER], q[SEQ_OVER]);
                 atomicMax(&ws.status[STATUS_OVER_FACES], ~ws.faces);
                 atomicMax(&ws.status[STATUS_OVER_TILES], ~ws.q_items);
             }
@@ -1537,7 +1530,6 @@ struct TileBin {
     const uint2* chunks;
     const uint2* wide;      // boxes and entries
     int nchunks, nwide;
-    int end;                // of the steps over the chunks: nchunks, or past whole 64s of them the list of the sequence
     uint32_t tx, ty;        // the tile in the boxes' units
 };
 __device__ __forceinline__ bool wide_hits(const TileBin& B, uint32_t box) {
@@ -1577,23 +1569,14 @@ __device__ __forceinline__ uint32_t list_wide(TileLds<TS, RB>& L, const TileBin&
 // Every wave prefix-sums the descriptors, 64 at a time, one a lane, and copies
 // its share of the chunks, 4, 16 or 64 lanes to a chunk by their mean length,
 // so that no barrier stands between the descriptors and the entries' loads.
-// Where the tile's places were too few, the list of the sequence follows, with
-// the other tiles' descriptors counted as empty.  Returns the number of all
-// entries; a barrier must follow.
+// Returns the number of all entries; a barrier must follow.
 template <int TS, int RB>
-__device__ __forceinline__ uint32_t list_chunks(TileLds<TS, RB>& L, const TileBin& B, const Workspace& ws, int gt,
-                                                uint32_t w0, uint32_t base) {
+__device__ __forceinline__ uint32_t list_chunks(TileLds<TS, RB>& L, const TileBin& B, const Workspace& ws, uint32_t w0,
+                                                uint32_t base) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    for (int g0 = 0; g0 < B.end; g0 += 64) {   // uniform
-        int nc = min(B.nchunks - g0, 64);
-        uint2 d;
-        if (__builtin_expect(nc > 0, 1)) {
-            d = gld2(B.chunks + g0 + min(lane, nc - 1));
-        } else {
-            nc = min(B.end - g0, 64);
-            const uint4 e = ws.over[g0 - ((B.nchunks + 63) & ~63) + min(lane, nc - 1)];
-            d = make_uint2(e.y, e.x == (uint32_t)gt ? e.z : 0u);
-        }
+    for (int g0 = 0; g0 < B.nchunks; g0 += 64) {   // uniform
+        const int nc = min(B.nchunks - g0, 64);
+        uint2 d = gld2(B.chunks + g0 + min(lane, nc - 1));
         if (lane >= nc) d.y = 0u;
         const uint32_t n = (d.y & CHUNK_INLINE) ? 1u : d.y;
         const uint32_t incl = wave_scan(n), total = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
@@ -1824,11 +1807,9 @@ __device__ void raster_tile(TileLds<TS, RB>& L, const PassDesc& P, const Workspa
     int tid = threadIdx.x;
     int W = P.width, H = P.height;
     const int ws_shift = wide_shift(P);
-    TileBin B{ws.chunks + (size_t)gt * ws.chunk_cap, ws.wide + (size_t)P.index * ws.wide_cap,
-              (int)min(nchunks, ws.chunk_cap), (int)min(nwide, ws.wide_cap), 0, (uint32_t)(tx >> ws_shift),
+    const TileBin B{ws.chunks + (size_t)gt * ws.chunk_cap, ws.wide + (size_t)P.index * ws.wide_cap,
+              (int)min(nchunks, ws.chunk_cap), (int)min(nwide, ws.wide_cap), (uint32_t)(tx >> ws_shift),
               (uint32_t)(ty >> ws_shift)};
-    B.end = B.nchunks;
-    if (__builtin_expect(nchunks > ws.chunk_cap, 0)) B.end = ((B.nchunks + 63) & ~63) + (int)min(seq_count(ws.seq, SEQ_OVER), ws.over_cap);
 
     // One copy of the code for every list of a long bin and for the second
     // sweep after NaN fragments.  Every wave reads a round's entries ahead of
@@ -1864,7 +1845,7 @@ __device__ void raster_tile(TileLds<TS, RB>& L, const PassDesc& P, const Workspa
             if (tid < 12) (&L.cnt[0][0])[tid] = 0;
             if (tid == 0) L.nan_seen = 0;
         }
-        const uint32_t n = list_chunks<TS, RB>(L, B, ws, gt, w0, nw);
+        const uint32_t n = list_chunks<TS, RB>(L, B, ws, w0, nw);
         first = false;
         __syncthreads();
         set = sweep<TS, RB>(L, P, min(n - w0, TILE_LIST), xb, yb, second, set);

@@ -353,8 +353,6 @@ int bind_plan(hana_ctx* c, Plan& pl, Arena& A, uint32_t min_bins, uint32_t min_p
         if ((r = ensure(c, A.chunks, sizeof(uint2) * want_slots))) return r;
         A.chunk_slots = want_slots;
     }
-    A.over_cap = std::max(A.over_cap, OVER_MIN);
-    if ((r = ensure(c, A.over, sizeof(uint4) * A.over_cap))) return r;
     if ((r = ensure(c, A.wide, sizeof(uint2) * WIDE_MAX * std::max(n, 1)))) return r;
     uint64_t want_polys = std::max<uint64_t>({(uint64_t)min_polys, pl.total_f / 16 + 4096});
     want_polys = std::min<uint64_t>(want_polys, POOL_CAP_MAX);
@@ -399,8 +397,6 @@ int bind_plan(hana_ctx* c, Plan& pl, Arena& A, uint32_t min_bins, uint32_t min_p
     // number of them so that the tiles' first groups spread over the caches
     uint64_t groups = std::min<uint64_t>(A.chunk_slots / tiles / 4, 1u << 28);
     ws.chunk_cap = (uint32_t)(4 * (groups - 1 + (groups & 1)));
-    ws.over = A.over.as<uint4>();
-    ws.over_cap = A.over_cap;
     ws.wide = A.wide.as<uint2>();
     ws.wide_cap = pl.counted ? 0 : WIDE_MAX;
     ws.pool_vr = A.pool_vr.as<float4>();
@@ -595,26 +591,15 @@ struct Needs {
     }
 };
 
-// Whether an arena's chunk descriptors grow to the needs of an overflow: up to
-// 2^26 past the tiles' places, and any number that the tiles take in places.
-// Sequences that need more bin by counting.
+// The places for chunk descriptors that an overflow asks for: those of its
+// fullest tile, and a quarter more, in all tiles.
 static uint64_t full_places(const Needs& need) { return (uint64_t)need.w[STATUS_NEED_CHUNKS] * 1024 / 4 * 5; }
-static bool chunks_grow(const Needs& need) {
-    return need.w[STATUS_NEED_OVER] <= (1u << 26) || full_places(need) <= (1u << 25);
-}
-
-// Grows them.  The list behind the tiles' places holds all that came after
-// those; the places grow to the fullest tile's need where that is up to 2^25
-// over all tiles (256 MB), else, for few crowded tiles of large targets, by as
-// many as came after.
+static bool chunks_grow(const Needs& need) { return full_places(need) <= kGrownChunks; }
 static int grow_chunks(hana_ctx* c, Arena& A, const Needs& need) {
-    int r;
-    const uint64_t past = need.w[STATUS_NEED_OVER], full = full_places(need);
-    const uint64_t want = full <= (1u << 25) ? std::max(full, A.chunk_slots) : A.chunk_slots + past / 4 * 5;
-    if ((r = ensure(c, A.chunks, sizeof(uint2) * want))) return r;
-    A.chunk_slots = want;
-    A.over_cap = std::max<uint32_t>(A.over_cap, (uint32_t)(std::min<uint64_t>(past, 1u << 26) / 4 * 5 + OVER_MIN));
-    return HANA_OK;
+    const uint64_t want = std::max(full_places(need), A.chunk_slots);
+    int r = ensure(c, A.chunks, sizeof(uint2) * want);
+    if (!r) A.chunk_slots = want;
+    return r;
 }
 
 // Grows an arena's bins, chunk descriptors and clip pool to the needs reported
@@ -991,7 +976,7 @@ int create_context(int device, int nslots, hana_ctx** out) {
 extern "C" {
 
 static void free_arena(Arena& a) {
-    DevBuf* bufs[] = {&a.tables, &a.vr, &a.vs, &a.code, &a.pof, &a.bins, &a.chunks, &a.over, &a.wide, &a.pool_vr,
+    DevBuf* bufs[] = {&a.tables, &a.vr, &a.vs, &a.code, &a.pof, &a.bins, &a.chunks, &a.wide, &a.pool_vr,
                       &a.pool_vs, &a.pool_face, &a.clip_queue, &a.status, &a.stats, &a.counters[0], &a.counters[1]};
     for (DevBuf* b : bufs)
         if (b->p) {
@@ -1001,7 +986,6 @@ static void free_arena(Arena& a) {
         }
     a.bin_cap = a.poly_cap = a.clipq_cap = 0;
     a.chunk_slots = 0;
-    a.over_cap = 0;
     a.counters_used[0] = a.counters_used[1] = 0;
 }
 

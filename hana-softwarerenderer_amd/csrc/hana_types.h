@@ -129,17 +129,14 @@ struct PassDesc {
 // clipped fan triangle, a table overflow) is a descriptor that holds its entry
 // itself (CHUNK_INLINE).  So one pass over the triangles bins them, without
 // counts, a scan or a second pass, and a raster workgroup reads its tile's
-// descriptors with one coalesced load.  Descriptors past a tile's places go to
-// one list of the sequence, which the raster workgroups of such tiles search,
-// so that meshes crowded into few tiles of a large target need no places for
-// them in every tile.  A triangle over more than WIDE_TILES tiles goes to its
-// pass's list instead, which every tile of the pass tests.
+// descriptors with one coalesced load.  A triangle over more than WIDE_TILES
+// tiles goes to its pass's list instead, which every tile of the pass tests.
+// Where a tile has no place left the sequence is binned by counting
+// (launch_counted), with the range of its pairs as each tile's one chunk.
 struct Workspace {
     uint2* chunks;               // per tile, chunk_cap: first bin entry and entries, or entry and CHUNK_INLINE
     uint32_t chunk_cap;
     uint32_t* bins;              // triangle entries: face id and its FACE_* bits, or CLIPPED_BIT | polygon << 4 | fan
-    uint4* over;                 // descriptors past their tile's places: tile, then as in chunks
-    uint32_t over_cap;
     uint32_t wide_cap;
     uint2* wide;                 // per pass, wide_cap: box of tiles (wide_box) and bin entry
     float4* pool_vr;             // clipped polygons: POLY_MAX vertices each
@@ -204,24 +201,22 @@ constexpr int WIDE_TILES = 16;
 #define HANA_WIDE_MAX 512
 #endif
 constexpr uint32_t WIDE_MAX = HANA_WIDE_MAX;
-constexpr uint32_t OVER_MIN = 1024;        // Workspace::over_cap at first
 
 // counter words of one sequence: polygons allocated, faces queued for
-// clipping, the flags it raised, the descriptors past their tiles' places and
-// the most chunks of one such tile, the persistent raster's queue, and (64-bit
+// clipping, the flags it raised, the most chunks of a tile with more than its
+// places, the persistent raster's queue, and (64-bit
 // each) the pairs outside the set-up workgroups' own entries and the pairs of
 // the listed wide triangles; of counted binning, all pairs in the first of them,
 // and whether they fit
-enum { SEQ_POLYS = 0, SEQ_CLIPQ = 1, SEQ_FLAGS = 2, SEQ_OVER = 3, SEQ_PAIRS = 4, SEQ_WIDE_PAIRS = 6,
-       SEQ_QUEUE = 8, SEQ_QUEUE_DONE = 9, SEQ_MAX_CHUNKS = 10, SEQ_COUNTED = 11, SEQ_WORDS = 16 };
+enum { SEQ_POLYS = 0, SEQ_CLIPQ = 1, SEQ_FLAGS = 2, SEQ_MAX_CHUNKS = 3, SEQ_PAIRS = 4, SEQ_WIDE_PAIRS = 6,
+       SEQ_QUEUE = 8, SEQ_QUEUE_DONE = 9, SEQ_COUNTED = 10, SEQ_WORDS = 16 };
 // status words: set across sequences until the host reads them at a sync
 // point, so that calls need not wait for one another: the flags of every
 // sequence and the largest needs seen: of places for descriptors, in units of
-// 1024 over all tiles of the sequence; of the list behind them; and the
-// complements of the faces and tiles of the smallest sequences that ran out of
+// 1024 over all tiles of the sequence; and the complements of the faces and tiles of the smallest sequences that ran out of
 // descriptors.
-enum { STATUS_FLAGS = 0, STATUS_NEED_BINS = 1, STATUS_NEED_POLYS = 2, STATUS_NEED_CHUNKS = 3, STATUS_NEED_OVER = 4,
-       STATUS_OVER_FACES = 5, STATUS_OVER_TILES = 6, STATUS_WORDS = 7 };
+enum { STATUS_FLAGS = 0, STATUS_NEED_BINS = 1, STATUS_NEED_POLYS = 2, STATUS_NEED_CHUNKS = 3, STATUS_OVER_FACES = 4,
+       STATUS_OVER_TILES = 5, STATUS_WORDS = 6 };
 enum { FLAG_BIN_OVERFLOW = 1, FLAG_POLY_OVERFLOW = 2, FLAG_POLY_TOO_LARGE = 4, FLAG_CLIPQ_OVERFLOW = 8,
        FLAG_CHUNK_OVERFLOW = 16, FLAG_PAIR_LIMIT = 32, FLAG_QUEUE_STALL = 64 };
 // A workspace capacity ran out: the sequence is incomplete, its rasters write

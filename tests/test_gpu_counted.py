@@ -2,6 +2,7 @@
 by how they crowd: counted binning renders them, against the oracle (depth
 bit-exact, colour as in test_gpu_parity)."""
 import ctypes as C
+import time
 
 import numpy as np
 import pytest
@@ -92,9 +93,9 @@ def test_noalloc_whatever_the_order(oracle, name, tile, wgs):
             assert_color_ok(col, ref.color, s.name)
 
 
-def test_more_descriptors_than_a_workspace_grows_to():
+def test_many_more_descriptors_than_places():
     """7.5 million triangles in random order, of 9 to 16 tiles each: 95 million
-    descriptors, where a workspace has places for 16 million.  The draw gives the
+    descriptors, where a workspace has places for 16 million at first.  The draw gives the
     image that its faces give in eight draws, in their order; so does a batch,
     and neither needs rendering again from then on."""
     from hana_amd.gpu import Batch, Context, build_uniforms
@@ -130,6 +131,62 @@ def test_more_descriptors_than_a_workspace_grows_to():
     assert (dep < 1e30).mean() > 0.99
     for c, d in got:
         assert d.tobytes() == dep.tobytes() and np.array_equal(c, col)
+
+
+def test_more_descriptors_than_a_workspace_grows_to(oracle):
+    """A quarter of a million triangles on a few dozen of 262,144 tiles: each of
+    those has a descriptor of nearly every set-up workgroup, and as many places in
+    every tile are more than a workspace grows to.  One overflow, then counted
+    binning in each draw, whose shadow pass is binned so too; and in a batch."""
+    from hana_amd.gpu import Batch, Context, build_uniforms
+    scene = soup_scene(250_000, 8192, 8192, 100, 400, 13)
+    scene.mesh.pos[:, :2] *= np.float32(0.01)
+    ref = oracle_image(oracle, scene)
+    with Context(0) as ctx:
+        u, mesh = build_uniforms(scene), ctx.mesh(scene.mesh)
+        tex = (ctx.texture(scene.diffuse), ctx.texture(scene.normal))
+        t, frame, smap, batched = (ctx.target(8192, 8192) for _ in range(4))
+        for k in range(2):
+            ctx.clear(t)
+            ctx.draw(mesh, scene.shader, u, t, *tex)
+            col, dep = ctx.read(t, 8192, 8192)
+            assert ctx.replay_count() == 1
+            assert_depth_exact(dep, ref.depth, scene.name)
+            assert_color_ok(col, ref.color, scene.name)
+        ctx.render_frame(mesh, scene.shader, True, u, frame, smap, *tex)
+        assert np.array_equal(ctx.read(frame, 8192, 8192)[1], dep)
+        batch = Batch(ctx)
+        batch.add(ctx.frame_desc(mesh, scene.shader, False, u, batched, None, *tex))
+        batch.finalize(use_graph=True)
+        for k in range(2):
+            batch.run()
+        got = ctx.read(batched, 8192, 8192)
+        assert got[1].tobytes() == dep.tobytes() and np.array_equal(got[0], col)
+        batch.close()
+
+
+def test_scattered_faces_take_no_longer_than_a_scan_of_their_entries():
+    """Three million faces that crowd into a thousand tiles of a 4K target, in
+    random order and row by row: a tile reads its own entries only, so the order
+    costs a few times as much at most."""
+    from hana_amd.gpu import Context, build_uniforms
+    scene = layered_scene(1, 1500, 1000, 3840, 2160, 14, fill=0.17, jitter=10.0)
+    order = np.lexsort((np.arange(len(scene.mesh.idx)), scene.mesh.idx.min(1)))
+    rows = sg.Mesh(scene.mesh.pos, scene.mesh.nrm, scene.mesh.uv, np.ascontiguousarray(scene.mesh.idx[order]))
+    took = []
+    with Context(0) as ctx:
+        u, tex = build_uniforms(scene), (ctx.texture(scene.diffuse), ctx.texture(scene.normal))
+        t = ctx.target(3840, 2160)
+        for m in (ctx.mesh(rows), ctx.mesh(scene.mesh)):
+            best = 1e9
+            for k in range(6):
+                t0 = time.perf_counter()
+                ctx.clear(t)
+                ctx.draw(m, scene.shader, u, t, *tex)
+                ctx.sync()
+                best = min(best, time.perf_counter() - t0)
+            took.append(best)
+    assert took[1] < 8 * took[0], took
 
 
 def test_counted_beside_an_overflow(oracle):
