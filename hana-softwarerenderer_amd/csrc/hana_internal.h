@@ -235,6 +235,9 @@ struct hana_ctx {
     // that finds a capacity overflow grows the workspaces and renders them
     // again (replay_overflow), else reports HANA_E_OVERFLOW
     std::vector<hana::rt::LoggedCall> log;
+    // batches run since the last status check and before those calls, by their
+    // last runs: a run some part of which outgrew its workspace is run again
+    std::vector<hana_batch*> batches;
     bool replay_overflow = true;
     int64_t replays = 0;   // status checks that rendered the logged calls again
     // per-call sequences of at least these faces and tiles bin by counting: the
@@ -262,6 +265,7 @@ struct hana_batch_part {
     hana::rt::Plan plan;
     hana::rt::Arena* arena = nullptr;   // the batch's arena of the same index
     size_t f0 = 0, f1 = 0;               // its frames [f0, f1) of the batch
+    bool counted = false;                // outgrew its workspace after it was sized: bins by counting
 };
 
 struct hana_batch {
@@ -278,6 +282,9 @@ struct hana_batch {
     hipEvent_t fork = nullptr;
     std::vector<hipEvent_t> joined;    // one per part after the first
     std::vector<hipStream_t> extra;    // streams of the parts beyond the context's draw slots
+    // the parts' status words (STATUS_WORDS each), pinned, and their device address
+    uint32_t* status_host = nullptr;
+    uint32_t* status_dev = nullptr;
 };
 
 namespace hana {

@@ -27,6 +27,12 @@
 using namespace hana;
 using namespace hana::rt;
 
+extern "C" {
+static uint32_t batch_take_flags(hana_ctx* c, hana_batch* b, uint32_t* parts);
+static int batch_recount(hana_ctx* c, hana_batch* b, uint32_t parts);
+static int batch_launch(hana_ctx* c, hana_batch* b);
+}
+
 namespace hana {
 namespace rt {
 
@@ -684,14 +690,22 @@ static int replay_call(hana_ctx* c, LoggedCall& L, bool counted) {
 //   they bin by counting, whose needs are exact; so do, from then on, sequences
 //   like one whose descriptors no workspace grows to.  With replay_overflow
 //   off, the caller is asked to render again (HANA_E_OVERFLOW).
+// - The same in a part of a batch that was run since: the part is sized again, by
+//   counting, and the batches are run again in the order of their last runs, then
+//   the calls, all of which came after them (hana_batch_run).
 // - More (triangle, tile) pairs than 32-bit bins reach: that sequence was not
 //   rasterised (HANA_E_NOMEM).
 // - A clipped polygon with more than POLY_MAX vertices was dropped, the rest
 //   drawn (HANA_E_UNSUPPORTED).
 int check_status(hana_ctx* c) {
-    if (!c->status_pending && !c->noalloc_pending) return HANA_OK;
+    if (!c->status_pending && !c->noalloc_pending && c->batches.empty()) return HANA_OK;
     int r;
     uint32_t seen = 0;
+    auto forget = [&] {
+        c->log.clear();
+        c->batches.clear();
+        c->status_pending = false;
+    };
     for (int attempt = 0;; attempt++) {
         if ((r = sync_all(c))) return r;
         Needs need;
@@ -717,28 +731,49 @@ int check_status(hana_ctx* c) {
         if (cap)
             for (int k = 0; k < c->nslots; k++)
                 if ((r = grow_arena(c, slot_arena(c, k), need))) {
-                    c->log.clear();
-                    c->status_pending = false;
+                    forget();
                     return r;
                 }
+        bool rerun = false;
+        for (hana_batch* b : c->batches) {
+            uint32_t parts = 0;
+            const uint32_t f = batch_take_flags(c, b, &parts) & ~(uint32_t)FLAG_POLY_TOO_LARGE;
+            seen |= f;
+            if (!(f & FLAG_CAPACITY)) continue;
+            rerun = true;
+            if ((r = batch_recount(c, b, parts))) {
+                forget();
+                return r;
+            }
+        }
+        if (rerun && c->noalloc_pending) {
+            // the frame may have drawn over the batch's targets, and cannot be drawn again
+            forget();
+            return fail(c, HANA_E_OVERFLOW,
+                        "a batch outgrew its workspace and left targets as they were, and a no-alloc frame followed it; "
+                        "the workspace was grown, render both again");
+        }
         if ((cap & FLAG_CHUNK_OVERFLOW) && !chunks_grow(need)) {
             c->counted_faces = std::min<size_t>(c->counted_faces, ~need.w[STATUS_OVER_FACES]);
             c->counted_tiles = std::min<size_t>(c->counted_tiles, ~need.w[STATUS_OVER_TILES]);
         }
-        if (cap && c->replay_overflow && attempt < 4) {
+        if ((rerun || (cap && c->replay_overflow)) && attempt < 4) {
             c->replays++;
+            for (hana_batch* b : c->batches)
+                if (rerun && (r = batch_launch(c, b))) {
+                    forget();
+                    return r;
+                }
             for (LoggedCall& L : c->log)
                 if ((r = replay_call(c, L, attempt > 0 || bins_by_counting(c, L.pl.total_f, L.pl.total_tiles)))) {
-                    c->log.clear();
-                    c->status_pending = false;
+                    forget();
                     return r;
                 }
             continue;   // wait for the replay and check it
         }
-        c->log.clear();
-        c->status_pending = false;
+        forget();
         c->count_next = cap && !c->replay_overflow;
-        if (cap)
+        if (cap || rerun)
             return fail(c, HANA_E_OVERFLOW,
                         c->replay_overflow ? "workspace capacity still exceeded after growing it four times"
                                            : "bin or clip-pool capacity exceeded since the last sync; buffers were "
@@ -1311,6 +1346,9 @@ static bool flags_raised(hana_ctx* c) {
         const uint32_t* host = slot_status(c, k);
         if (host && *static_cast<const volatile uint32_t*>(host + STATUS_FLAGS)) return true;
     }
+    for (const hana_batch* b : c->batches)
+        for (size_t p = 0; p < b->parts.size(); p++)
+            if (*static_cast<const volatile uint32_t*>(b->status_host + STATUS_WORDS * p + STATUS_FLAGS) & FLAG_NO_RASTER) return true;
     return false;
 }
 
@@ -1621,17 +1659,73 @@ static int batch_enqueue(hana_ctx* c, hana_batch* b, bool timed) {
     return HANA_OK;
 }
 
-// Sizes a part's workspace exactly with trial runs.
+// Clears the parts' status words, once the batch's runs have ended; returns their
+// flags, and in `parts` the parts with one of a capacity.
+static uint32_t batch_take_flags(hana_ctx* c, hana_batch* b, uint32_t* parts) {
+    uint32_t all = 0;
+    for (size_t p = 0; p < b->parts.size(); p++) {
+        uint32_t* const host = b->status_host + STATUS_WORDS * p;
+        const uint32_t f = host[STATUS_FLAGS];
+        if (!f) continue;
+        all |= f;
+        if (f & FLAG_CAPACITY) *parts |= 1u << p;
+        (void)launch_fill32(b->arenas[p].status.as<uint32_t>(), 0u, STATUS_WORDS, c->stream);
+        std::memset(host, 0, sizeof(uint32_t) * STATUS_WORDS);
+    }
+    return all;
+}
+
+// Whether the workspace of a chunked part that was just run holds what another
+// run may need.  Which of the wide triangles a full list leaves out, which pairs
+// a full table leaves out and which fans are clipped together follow the order
+// in which workgroups and lanes arrive.  For the first there is a bound: every
+// listed triangle of a pass one more descriptor in a tile, and all their pairs.
+// For the others an eighth is added.  Grows what is too small (then true, and the
+// part is run again) or leaves the part to counted binning.
+static int batch_leave_room(hana_ctx* c, hana_batch_part& part, uint32_t* min_bins, bool* grown, bool* counted) {
+    const Plan& pl = part.plan;
+    Arena& A = *part.arena;
+    std::vector<uint32_t> n(counter_words(pl));
+    HIP_TRY(c, hipMemcpy(n.data(), pl.ws.seq, sizeof(uint32_t) * n.size(), hipMemcpyDeviceToHost));
+    auto pairs = [&](int w) { return (uint64_t)n[w] | (uint64_t)n[w + 1] << 32; };
+    const uint32_t *wide = n.data() + SEQ_WORDS, *chunks = n.data() + (pl.ws.tile_chunks - pl.ws.seq);
+    const bool left_out = *std::max_element(wide, wide + std::max<size_t>(pl.descs.size(), 1)) > pl.ws.wide_cap;
+    const uint64_t fullest = pl.total_tiles ? *std::max_element(chunks, chunks + pl.total_tiles) : 0;
+    const uint64_t places = fullest + fullest / 8 + CHUNK_SLACK + (left_out ? pl.ws.wide_cap : 0);
+    uint64_t shared = pairs(SEQ_PAIRS) + (left_out ? pairs(SEQ_WIDE_PAIRS) : 0);
+    shared += shared / 8 + 4096;
+    if (places > pl.ws.chunk_cap) {
+        const uint64_t slots = (places + places / 8 + 8) * (uint64_t)std::max(pl.total_tiles, 1);
+        if (slots > kGrownChunks) {
+            *counted = true;
+            return HANA_OK;
+        }
+        int r = ensure(c, A.chunks, sizeof(uint2) * slots);
+        if (r) return r;
+        A.chunk_slots = slots;
+        *grown = true;
+    }
+    if (pl.ws.seg_region + shared > pl.ws.bin_cap) {
+        if (pl.ws.seg_region + shared > MAX_PAIRS) *counted = true;
+        else *min_bins = (uint32_t)(pl.ws.seg_region + shared);
+        *grown = true;
+    }
+    return HANA_OK;
+}
+
+// Sizes a part's workspace with trial runs.
 static int batch_size_part(hana_ctx* c, hana_batch* b, hana_batch_part& part) {
     int r;
     uint32_t min_bins = 0, min_polys = 0;
-    bool counted = false;
+    bool counted = part.counted, roomy = false;
     Arena& A = *part.arena;
-    for (int attempt = 0; attempt < 6; attempt++) {
+    const size_t p = (size_t)(&part - b->parts.data());
+    for (int attempt = 0; attempt < 8; attempt++) {
         if ((attempt == 0 || counted != part.plan.counted) &&
             (r = build_plan(c, part.specs, part.plan, b->tuning, kBatchFrontFaces, counted)))
             return r;
         if ((r = bind_plan(c, part.plan, A, min_bins, min_polys, false, c->stream))) return r;
+        part.plan.ws.status_out = b->status_dev + STATUS_WORDS * p;
         batch_clear_flags(part);
         HIP_TRY(c, hipMemcpy(A.tables.p, part.plan.descs.data(), sizeof(PassDesc) * part.plan.descs.size(),
                              hipMemcpyHostToDevice));
@@ -1640,12 +1734,21 @@ static int batch_size_part(hana_ctx* c, hana_batch* b, hana_batch_part& part) {
         if (!part.plan.tile_pass.empty())
             HIP_TRY(c, hipMemcpy(A.tables.as<char>() + part.plan.tp_off, part.plan.tile_pass.data(),
                                  sizeof(uint2) * part.plan.tile_pass.size(), hipMemcpyHostToDevice));
-        // trial run: sizes the bins and the clip pool exactly
+        // trial run: what it needs, exactly or (chunks) as near as another's
         if ((r = enqueue_sequence(c, part.plan, A, c->stream))) return r;
         uint32_t st[STATUS_WORDS];
         HIP_TRY(c, hipMemcpyAsync(st, A.status.p, sizeof st, hipMemcpyDeviceToHost, c->stream));
         HIP_TRY(c, hipStreamSynchronize(c->stream));
-        batch_drop_pending(b);
+        std::memset(b->status_host + STATUS_WORDS * p, 0, sizeof st);
+        if (!(st[STATUS_FLAGS] & ~(uint32_t)FLAG_POLY_TOO_LARGE) && !counted && !roomy) {
+            roomy = true;   // once: it then has room for what this run needed and more
+            bool grown = false;
+            if ((r = batch_leave_room(c, part, &min_bins, &grown, &counted))) return r;
+            if (grown || counted) {
+                HIP_TRY(c, launch_fill32(A.status.as<uint32_t>(), 0u, STATUS_WORDS, c->stream));
+                continue;
+            }
+        }
         if (!st[STATUS_FLAGS]) return HANA_OK;
         HIP_TRY(c, launch_fill32(A.status.as<uint32_t>(), 0u, STATUS_WORDS, c->stream));
         if (st[STATUS_FLAGS] & FLAG_QUEUE_STALL)
@@ -1656,7 +1759,7 @@ static int batch_size_part(hana_ctx* c, hana_batch* b, hana_batch_part& part) {
                                              "(triangle, tile) pairs; split the batch");
             return HANA_OK;   // a polygon over POLY_MAX vertices is dropped at every run, like a per-call draw
         }
-        min_bins = st[STATUS_NEED_BINS] + st[STATUS_NEED_BINS] / 8 + 1024;
+        min_bins = std::max(min_bins, st[STATUS_NEED_BINS] + st[STATUS_NEED_BINS] / 8 + 1024);
         min_polys = st[STATUS_NEED_POLYS] + st[STATUS_NEED_POLYS] / 8 + 1024;
         Needs need;
         need.take(st);
@@ -1668,11 +1771,50 @@ static int batch_size_part(hana_ctx* c, hana_batch* b, hana_batch_part& part) {
     return fail(c, HANA_E_OVERFLOW, "hana_batch_finalize: capacity not reached");
 }
 
+// All of them, whose trial runs draw what was to be cleared.
+static int batch_size_parts(hana_ctx* c, hana_batch* b) {
+    int r = HANA_OK;
+    for (auto& part : b->parts)
+        if ((r = batch_size_part(c, b, part))) break;
+    batch_drop_pending(b);
+    return r;
+}
+
 static void batch_drop_graph(hana_batch* b) {
     if (b->exec) (void)hipGraphExecDestroy(b->exec);
     if (b->graph) (void)hipGraphDestroy(b->graph);
     b->exec = nullptr;
     b->graph = nullptr;
+}
+
+// Captures the sized parts (with use_graph).
+static int batch_capture(hana_ctx* c, hana_batch* b) {
+    batch_drop_graph(b);
+    if (b->use_graph) {
+        HIP_TRY(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
+        int er = batch_enqueue(c, b, false);
+        hipGraph_t g = nullptr;
+        hipError_t ec = hipStreamEndCapture(c->stream, &g);
+        if (er) {
+            if (g) (void)hipGraphDestroy(g);
+            return er;
+        }
+        if (ec != hipSuccess) return hip_fail(c, ec, "hipStreamEndCapture");
+        b->graph = g;
+        HIP_TRY(c, hipGraphInstantiate(&b->exec, b->graph, nullptr, nullptr, 0));
+    }
+    return HANA_OK;
+}
+
+// Sizes the given parts again, by counting.
+static int batch_recount(hana_ctx* c, hana_batch* b, uint32_t parts) {
+    int r;
+    for (size_t p = 0; p < b->parts.size(); p++) {
+        if (!(parts >> p & 1u)) continue;
+        b->parts[p].counted = true;
+        if ((r = batch_size_part(c, b, b->parts[p]))) return r;
+    }
+    return batch_capture(c, b);
 }
 
 // Splits, sizes and (with use_graph) captures the batch for b->tuning.
@@ -1681,8 +1823,7 @@ static int batch_prepare_parts(hana_ctx* c, hana_batch* b, bool use_graph) {
     batch_drop_graph(b);
     std::vector<double> w = frame_weights(b);
     batch_split(b, split_ends(b, w));
-    for (auto& part : b->parts)
-        if ((r = batch_size_part(c, b, part))) return r;
+    if ((r = batch_size_parts(c, b))) return r;
     if (b->parts.size() > 1) {
         // One rebalancing step.  The parts run concurrently and the batch ends
         // with its slowest one; with the first estimates the parts of 256
@@ -1723,8 +1864,7 @@ static int batch_prepare_parts(hana_ctx* c, hana_batch* b, bool use_graph) {
         for (auto& part : b->parts) before.push_back(part.f1);
         if (measured && ends != before) {
             batch_split(b, ends);
-            for (auto& part : b->parts)
-                if ((r = batch_size_part(c, b, part))) return r;
+            if ((r = batch_size_parts(c, b))) return r;
         }
     }
     if (b->parts.size() > 1 && !b->fork) HIP_TRY(c, hipEventCreateWithFlags(&b->fork, hipEventDisableTiming));
@@ -1739,20 +1879,7 @@ static int batch_prepare_parts(hana_ctx* c, hana_batch* b, bool use_graph) {
         b->extra.push_back(s);
     }
     b->use_graph = use_graph;
-    if (b->use_graph) {
-        HIP_TRY(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-        int er = batch_enqueue(c, b, false);
-        hipGraph_t g = nullptr;
-        hipError_t ec = hipStreamEndCapture(c->stream, &g);
-        if (er) {
-            if (g) (void)hipGraphDestroy(g);
-            return er;
-        }
-        if (ec != hipSuccess) return hip_fail(c, ec, "hipStreamEndCapture");
-        b->graph = g;
-        HIP_TRY(c, hipGraphInstantiate(&b->exec, b->graph, nullptr, nullptr, 0));
-    }
-    return HANA_OK;
+    return batch_capture(c, b);
 }
 
 // The parts of a batch until the caller sets them, by its 16x16 tiles.  Each part
@@ -1769,6 +1896,17 @@ static int parts_for(const hana_batch* b) {
 }
 
 static int batch_prepare(hana_ctx* c, hana_batch* b, bool use_graph) {
+    if (!b->status_host) {
+        const size_t bytes = sizeof(uint32_t) * STATUS_WORDS * kMaxBatchParts;
+        if (hipHostMalloc((void**)&b->status_host, bytes) != hipSuccess ||
+            hipHostGetDevicePointer((void**)&b->status_dev, b->status_host, 0) != hipSuccess) {
+            (void)hipGetLastError();
+            if (b->status_host) (void)hipHostFree(b->status_host);
+            b->status_host = nullptr;
+            return fail(c, HANA_E_NOMEM, "batch status words: pinned allocation failed");
+        }
+        std::memset(b->status_host, 0, bytes);
+    }
     if (b->tuning.auto_parts) b->tuning.parts = parts_for(b);
     int r = batch_prepare_parts(c, b, use_graph);
     if (r == HANA_E_NOMEM && b->tuning.auto_parts && b->tuning.parts < 4) {
@@ -1801,7 +1939,6 @@ int hana_batch_finalize(hana_ctx* c, hana_batch* b, int use_graph) {
 
 // One run of a prepared batch on the context stream.
 static int batch_launch(hana_ctx* c, hana_batch* b) {
-    batch_drop_pending(b);
     int r = join(c);
     if (r) return r;
     c->next_slot = 0;   // the next draw follows the sequence on the context stream
@@ -1829,6 +1966,7 @@ static int batch_time(hana_ctx* c, hana_batch* b, int reps, double* ms) {
         return fail(c, HANA_E_DEVICE, "hipEventCreate");
     }
     float t = 0.f;
+    batch_drop_pending(b);
     r = batch_launch(c, b);
     if (!r) r = sync_all(c);
     if (!r && hipEventRecord(e0, c->stream) != hipSuccess) r = fail(c, HANA_E_DEVICE, "hipEventRecord");
@@ -1890,9 +2028,15 @@ int hana_batch_autotune(hana_ctx* c, hana_batch* b, int use_graph, int reps, han
     Tuning best = b->tuning;
     double best_ms = 0.0;
     auto measure = [&](const Tuning& t, double* ms) {
-        b->tuning = t;
-        int e = batch_prepare(c, b, use_graph != 0);
-        return e ? e : batch_time(c, b, reps, ms);
+        for (int tries = 0; tries < 3; tries++) {
+            b->tuning = t;
+            int e = batch_prepare(c, b, use_graph != 0);
+            if (e || (e = batch_time(c, b, reps, ms))) return e;
+            uint32_t parts = 0;
+            if (!(batch_take_flags(c, b, &parts) & FLAG_NO_RASTER)) return (int)HANA_OK;
+            *ms = 1e30;   // frames were left out: no time of theirs
+        }
+        return (int)HANA_OK;
     };
     if ((r = measure(best, &best_ms))) return r;
     best.parts = b->tuning.parts;
@@ -1934,21 +2078,29 @@ int hana_batch_run(hana_ctx* c, hana_batch* b) {
     if (!c || !b || !b->finalized) return fail(c, HANA_E_INVALID, "hana_batch_run: batch not finalized");
     // per-call draws before the batch are complete (replayed if need be)
     // before the batch draws over their targets
-    int r = check_status(c);
-    if (r) return r;
+    int r;
+    if ((c->status_pending || c->noalloc_pending) && (r = check_status(c))) return r;
+    batch_drop_pending(b);
+    auto& runs = c->batches;
+    runs.erase(std::remove(runs.begin(), runs.end(), b), runs.end());
+    runs.push_back(b);
     return batch_launch(c, b);
 }
 
 int hana_batch_destroy(hana_ctx* c, hana_batch* b) {
     if (!c || !b) return HANA_E_INVALID;
+    // a run that outgrew the workspace is run again while it can be
+    const bool ran = std::find(c->batches.begin(), c->batches.end(), b) != c->batches.end();
+    const int st = ran ? check_status(c) : HANA_OK;
     (void)sync_all(c);
     batch_drop_graph(b);
+    if (b->status_host) (void)hipHostFree(b->status_host);
     for (auto& a : b->arenas) free_arena(a);
     if (b->fork) (void)hipEventDestroy(b->fork);
     for (hipEvent_t e : b->joined) (void)hipEventDestroy(e);
     for (hipStream_t s : b->extra) (void)hipStreamDestroy(s);
     delete b;
-    return HANA_OK;
+    return st;
 }
 
 }  // extern "C"

@@ -54,7 +54,7 @@ enum {
     HANA_E_INVALID = -1,     /* bad argument */
     HANA_E_DEVICE = -2,      /* HIP runtime error */
     HANA_E_NOMEM = -3,       /* device allocation failed or over budget */
-    HANA_E_OVERFLOW = -4,    /* internal capacity exceeded after three replays */
+    HANA_E_OVERFLOW = -4,    /* internal capacity exceeded after four replays */
     HANA_E_UNSUPPORTED = -5  /* a clipped polygon had more than 16 vertices: it was
                                 dropped, the rest drawn (the reference keeps 30) */
 };
@@ -238,7 +238,10 @@ int hana_gpu_set_tuning(hana_ctx* ctx, const hana_tuning* t);
  * The frames are split into up to four parts that run concurrently (branches
  * of the graph on the context's streams and the batch's own); they need
  * distinct targets and shadow maps.  hana_batch_run returns once the work is
- * enqueued; it first completes the per-call draws enqueued before it. */
+ * enqueued; it first completes the per-call draws enqueued before it.  A part
+ * whose run outgrows the workspace it was finalized with leaves its targets
+ * untouched; the next wait (as for draws) sizes it again and runs the batches
+ * since the previous wait again, and the draws after them. */
 int hana_batch_create(hana_ctx* ctx, hana_batch** out);
 int hana_batch_add_frame(hana_ctx* ctx, hana_batch* b, const hana_frame_desc* f);
 /* Tuning used by hana_batch_finalize (before it). */

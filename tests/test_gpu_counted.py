@@ -219,3 +219,108 @@ def test_counted_beside_an_overflow(oracle):
         assert status == 0, s.name
         assert_depth_exact(dep, ref.depth, s.name)
         assert_color_ok(img, ref.color, s.name)
+
+
+class MeshWords(C.Structure):
+    """How a mesh handle begins: its counts, then its arrays on the device."""
+    _fields_ = [("V", C.c_int32), ("F", C.c_int32), ("soa", C.c_void_p), ("idx", C.c_void_p)]
+
+
+def move_vertices(ctx, mesh, pos):
+    """Other positions for a resident mesh, as a program's own kernel would write them."""
+    words = MeshWords.from_address(mesh.value)
+    assert words.V == len(pos)
+    xyz = np.ascontiguousarray(pos.T, np.float32)
+    ctx.sync()
+    assert ctx.lib.hipMemcpy(C.c_void_p(words.soa), xyz.ctypes.data_as(C.c_void_p), C.c_size_t(xyz.nbytes), C.c_int(1)) == 0
+
+
+@pytest.mark.parametrize("parts,use_graph", [(1, True), (2, True), (3, False)])
+def test_batch_outgrows_the_workspace_it_was_sized_for(parts, use_graph):
+    """A part of a batch that needs more than its trial run did is run again,
+    with the images of single draws: after one run and after several, with a
+    draw or a clear of its targets behind it, and when it is destroyed."""
+    from hana_amd.gpu import Batch, Context, build_uniforms
+    scenes = [soup_scene(n, w, h, 100, 400, 70 + n) for n, w, h in ((900, 333, 217), (60_000, 2048, 1024), (300, 97, 61))]
+    tops = [soup_scene(50, s.width, s.height, 20, 60, 80 + k) for k, s in enumerate(scenes)]
+    spread = [s.mesh.pos.copy() for s in scenes]
+    for s, p in zip(scenes, spread):
+        p[:, :2] = s.mesh.pos.reshape(-1, 3, 3).mean(1, keepdims=True).repeat(3, 1).reshape(-1, 3)[:, :2]
+        p[:, :2] += (s.mesh.pos[:, :2] - p[:, :2]) * np.float32(0.02)      # small triangles all over the view
+        s.mesh.pos[:, :2] *= np.float32(0.03)                              # then in a few tiles
+    with Context(0) as ctx:
+        u = [build_uniforms(s) for s in scenes]
+        tex = [(ctx.texture(s.diffuse), ctx.texture(s.normal)) for s in scenes]
+        top = [ctx.mesh(s.mesh) for s in tops]
+        want, topped = [], []
+        for k, s in enumerate(scenes):
+            t = ctx.target(s.width, s.height)
+            ctx.draw(ctx.mesh(s.mesh), s.shader, u[k], t, *tex[k])
+            want.append(ctx.read(t, s.width, s.height))
+            ctx.draw(top[k], s.shader, u[k], t, *tex[k])
+            topped.append(ctx.read(t, s.width, s.height))
+
+        def same(targets, images, what):
+            for t, s, (col, dep) in zip(targets, scenes, images):
+                c, d = ctx.read(t, s.width, s.height)
+                assert d.tobytes() == dep.tobytes() and np.array_equal(c, col), what
+
+        for after in ("run", "runs", "draw", "clear", "destroy"):
+            meshes = [ctx.mesh(sg.Mesh(p, s.mesh.nrm, s.mesh.uv, s.mesh.idx)) for p, s in zip(spread, scenes)]
+            targets = [ctx.target(s.width, s.height) for s in scenes]
+            batch = Batch(ctx)
+            batch.set_tuning(16, 0, parts)
+            for k, s in enumerate(scenes):
+                batch.add(ctx.frame_desc(meshes[k], s.shader, False, u[k], targets[k], None, *tex[k]))
+            batch.finalize(use_graph=use_graph)
+            batch.run()
+            for m, s in zip(meshes, scenes):
+                move_vertices(ctx, m, s.mesh.pos)
+            before = ctx.replay_count()
+            for k in range(3 if after == "runs" else 1):
+                batch.run()
+            if after == "draw":
+                for k, s in enumerate(scenes):
+                    ctx.draw(top[k], s.shader, u[k], targets[k], *tex[k])
+            elif after == "clear":
+                ctx.clear(targets[1])
+                col, dep = ctx.read(targets[1], 2048, 1024)
+                assert (dep > 3e38).all() and not col[..., :3].any()
+                targets, full = [targets[0], targets[2]], targets
+            elif after == "destroy":
+                batch.close()
+            if after == "clear":
+                for t, k in zip(targets, (0, 2)):
+                    c, d = ctx.read(t, scenes[k].width, scenes[k].height)
+                    assert d.tobytes() == want[k][1].tobytes() and np.array_equal(c, want[k][0])
+                targets = full
+            else:
+                same(targets, topped if after == "draw" else want, after)
+            assert ctx.replay_count() == before + 1
+            if after != "destroy":
+                batch.run()
+                same(targets, want, "the run after")
+                assert ctx.replay_count() == before + 1
+                batch.close()
+
+
+def test_batch_of_many_wide_triangles_renders_every_time():
+    """More triangles of many tiles than a pass's list holds: which of them it
+    holds differs from run to run, and the images do not."""
+    from hana_amd.gpu import Batch, Context, build_uniforms
+    scene = soup_scene(594, 640, 480, 500, 900, 90)
+    with Context(0) as ctx:
+        u, mesh, tex = build_uniforms(scene), ctx.mesh(scene.mesh), (ctx.texture(scene.diffuse), ctx.texture(scene.normal))
+        single, t = ctx.target(640, 480), ctx.target(640, 480)
+        ctx.draw(mesh, scene.shader, u, single, *tex)
+        col, dep = ctx.read(single, 640, 480)
+        batch = Batch(ctx)
+        batch.add(ctx.frame_desc(mesh, scene.shader, False, u, t, None, *tex))
+        batch.finalize(use_graph=True)
+        junk = np.full((480, 640, 4), 0x5A, np.uint8), np.full((480, 640), 7, np.float32)
+        for k in range(200):
+            ctx.upload(t, *junk)
+            batch.run()
+            c, d = ctx.read(t, 640, 480)
+            assert d.tobytes() == dep.tobytes() and np.array_equal(c, col), k
+        batch.close()
