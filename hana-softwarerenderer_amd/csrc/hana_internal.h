@@ -136,8 +136,8 @@ constexpr size_t kMaxLoggedCalls = 1024;
 constexpr size_t kStagePiece = size_t(8) << 20;
 // chunk descriptors that a workspace grows to after an overflow (2 GB);
 // sequences that need more bin by counting, which takes a second set-up: 3 M faces
-// in random order on 1,000 of 32,400 tiles 550 us a frame with places for their
-// descriptors (2^27.1) and 905 by counting, 20 M on all of them 11.4 and 14.3 ms
+// in random order on 1,000 of 32,400 tiles 506 us a frame with places for their
+// descriptors (2^27.1) and 901 by counting, 20 M on all of them 10.9 and 14.1 ms
 constexpr uint64_t kGrownChunks = uint64_t(1) << 28;
 // streams (each with a workspace) that consecutive per-call draws rotate over
 #ifndef HANA_DRAW_SLOTS

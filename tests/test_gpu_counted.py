@@ -2,6 +2,7 @@
 by how they crowd: counted binning renders them, against the oracle (depth
 bit-exact, colour as in test_gpu_parity)."""
 import ctypes as C
+import dataclasses
 import time
 
 import numpy as np
@@ -165,28 +166,47 @@ def test_more_descriptors_than_a_workspace_grows_to(oracle):
         batch.close()
 
 
+def frame_time(ctx, scene, frames=6):
+    """The fastest of some frames, in seconds."""
+    from hana_amd.gpu import build_uniforms
+    args = (ctx.mesh(scene.mesh), scene.shader, build_uniforms(scene), ctx.target(scene.width, scene.height),
+            ctx.texture(scene.diffuse), ctx.texture(scene.normal))
+    best = 1e9
+    for _ in range(frames):
+        t0 = time.perf_counter()
+        ctx.clear(args[3])
+        ctx.draw(*args)
+        ctx.sync()
+        best = min(best, time.perf_counter() - t0)
+    return best
+
+
 def test_scattered_faces_take_no_longer_than_a_scan_of_their_entries():
     """Three million faces that crowd into a thousand tiles of a 4K target, in
     random order and row by row: a tile reads its own entries only, so the order
     costs a few times as much at most."""
-    from hana_amd.gpu import Context, build_uniforms
+    from hana_amd.gpu import Context
     scene = layered_scene(1, 1500, 1000, 3840, 2160, 14, fill=0.17, jitter=10.0)
     order = np.lexsort((np.arange(len(scene.mesh.idx)), scene.mesh.idx.min(1)))
     rows = sg.Mesh(scene.mesh.pos, scene.mesh.nrm, scene.mesh.uv, np.ascontiguousarray(scene.mesh.idx[order]))
-    took = []
+    ordered = dataclasses.replace(scene, mesh=rows)
     with Context(0) as ctx:
-        u, tex = build_uniforms(scene), (ctx.texture(scene.diffuse), ctx.texture(scene.normal))
-        t = ctx.target(3840, 2160)
-        for m in (ctx.mesh(rows), ctx.mesh(scene.mesh)):
-            best = 1e9
-            for k in range(6):
-                t0 = time.perf_counter()
-                ctx.clear(t)
-                ctx.draw(m, scene.shader, u, t, *tex)
-                ctx.sync()
-                best = min(best, time.perf_counter() - t0)
-            took.append(best)
+        took = [frame_time(ctx, s) for s in (ordered, scene)]
     assert took[1] < 8 * took[0], took
+
+
+def test_crowded_tile_takes_time_by_its_entries():
+    """Sixteen times the triangles on the same two tiles take at most sixteen times
+    as long (and a tenth for the clock): a list of a tile's entries begins where
+    the one before ended."""
+    from hana_amd.gpu import Context
+    with Context(0) as ctx:
+        took = []
+        for n in (400_000, 6_400_000):
+            scene = soup_scene(n, 1920, 1080, 500, 600, 15)
+            scene.mesh.pos[:, :2] *= np.float32(0.005)
+            took.append(frame_time(ctx, scene))
+    assert took[1] < 17.6 * took[0], took
 
 
 def test_counted_beside_an_overflow(oracle):
