@@ -1986,8 +1986,28 @@ static void tuning_out(const Tuning& t, double ms, hana_tuning* out) {
     out->tile_size = tile_edge(t.tile_shift);
     out->raster_wgs_per_cu = t.raster_wgs_per_cu;
     out->parts = t.parts;
-    out->raster_waves = t.raster_waves;
+    out->raster_waves = t.auto_waves ? 0 : t.raster_waves;
     out->ms = ms;
+}
+
+// A prepared batch's tuning as a caller can set it: the waves that were chosen
+// where its rasters all have the same, else 0, which chooses them again.
+static Tuning batch_tuning(const hana_batch* b) {
+    Tuning t = b->tuning;
+    int waves = 0;
+    bool same = true;
+    for (const hana_batch_part& part : b->parts)
+        for (int g = 0; g < 2; g++) {
+            if (part.plan.raster_wgs == 0 && !part.plan.group_count[g]) continue;
+            const int w = part.plan.raster_waves[part.plan.raster_wgs > 0 ? 0 : g];
+            same = same && (!waves || w == waves);
+            waves = w;
+        }
+    if (t.auto_waves && waves && same) {
+        t.raster_waves = waves;
+        t.auto_waves = false;
+    }
+    return t;
 }
 
 int hana_gpu_set_tuning(hana_ctx* c, const hana_tuning* t) {
@@ -2007,7 +2027,7 @@ int hana_batch_set_tuning(hana_ctx* c, hana_batch* b, const hana_tuning* t) {
 
 int hana_batch_get_tuning(hana_ctx* c, const hana_batch* b, hana_tuning* out) {
     if (!c || !b || !out) return HANA_E_INVALID;
-    tuning_out(b->tuning, b->tuned_ms, out);
+    tuning_out(batch_tuning(b), b->tuned_ms, out);
     return HANA_OK;
 }
 
@@ -2070,7 +2090,7 @@ int hana_batch_autotune(hana_ctx* c, hana_batch* b, int use_graph, int reps, han
     if ((r = batch_prepare(c, b, use_graph != 0))) return r;
     b->tuned_ms = best_ms;
     b->finalized = true;
-    if (chosen) tuning_out(best, best_ms, chosen);
+    if (chosen) tuning_out(batch_tuning(b), best_ms, chosen);
     return HANA_OK;
 }
 

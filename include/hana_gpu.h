@@ -257,6 +257,8 @@ int hana_batch_finalize(hana_ctx* ctx, hana_batch* b, int use_graph);
  * rendered by every run.  `chosen` (nullable) receives the choice and its
  * time. */
 int hana_batch_autotune(hana_ctx* ctx, hana_batch* b, int use_graph, int reps, hana_tuning* chosen);
+/* The batch's tuning as hana_batch_set_tuning takes it; raster_waves is 0 where
+ * it was chosen per raster and the rasters differ. */
 int hana_batch_get_tuning(hana_ctx* ctx, const hana_batch* b, hana_tuning* out);
 int hana_batch_run(hana_ctx* ctx, hana_batch* b);
 int hana_batch_destroy(hana_ctx* ctx, hana_batch* b);
