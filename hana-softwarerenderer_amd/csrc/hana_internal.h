@@ -3,6 +3,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <string>
 #include <utility>
 #include <vector>
@@ -139,6 +140,15 @@ constexpr size_t kStagePiece = size_t(8) << 20;
 // in random order on 1,000 of 32,400 tiles 506 us a frame with places for their
 // descriptors (2^27.1) and 901 by counting, 20 M on all of them 10.9 and 14.1 ms
 constexpr uint64_t kGrownChunks = uint64_t(1) << 28;
+// The places for chunk descriptors that a tile has at first: a tile has one chunk
+// per set-up workgroup whose faces touch it.  Meshes whose neighbouring faces
+// follow one another need a few dozen; eight per face over all tiles hold even
+// scattered ones, and beyond 512 a tile two per face do.
+inline uint64_t tile_places(uint64_t faces, uint64_t tiles) {
+    const uint64_t per_tile = faces / tiles + 1;
+    const uint64_t places = std::min<uint64_t>(8 * per_tile, std::max<uint64_t>(512, 2 * per_tile));
+    return std::max<uint64_t>(places, tiles > (1u << 20) ? 16 : 64) + CHUNK_SLACK;
+}
 // streams (each with a workspace) that consecutive per-call draws rotate over
 #ifndef HANA_DRAW_SLOTS
 #define HANA_DRAW_SLOTS 4

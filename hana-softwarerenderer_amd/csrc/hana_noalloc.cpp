@@ -228,9 +228,7 @@ extern "C" int hana_render_frame_noalloc(hana_ctx* c, const hana_frame_desc* f) 
     left = left > 256 ? left - 256 : 0;
     const size_t min_bins = std::max<size_t>(seg_region + tf + 64, std::min(WIDE_TILES * tris, nominal_bins));
     const size_t spare = left > min_bins ? left - min_bins : 0;
-    const size_t per_face = tf / ntiles + 1;
-    const size_t want_cap = std::max<size_t>(std::min<size_t>(8 * per_face, std::max<size_t>(512, 2 * per_face)), 64) + CHUNK_SLACK;
-    size_t cap = std::min(spare / 4 / ntiles, std::max(want_cap, spare / 8 / ntiles));
+    size_t cap = std::min<size_t>(spare / 4 / ntiles, std::max<size_t>(tile_places(tf, ntiles), spare / 8 / ntiles));
     if (cap >= 8) cap = 4 * (cap / 4 - 1 + (cap / 4 & 1));   // an odd number of 32-byte groups
     cap = std::max<size_t>(cap, 1);
     ws.chunks = cv.take<uint2>(cap * ntiles);

@@ -346,14 +346,9 @@ int bind_plan(hana_ctx* c, Plan& pl, Arena& A, uint32_t min_bins, uint32_t min_p
         if ((r = ensure(c, A.bins, sizeof(uint32_t) * want_bins))) return r;
         A.bin_cap = (uint32_t)want_bins;
     }
-    // chunk descriptors: a tile has one per set-up workgroup whose faces touch
-    // it.  Meshes whose neighbouring faces follow one another need a few
-    // dozen; eight per face over all tiles hold even scattered ones, and
-    // beyond 512 a tile two per face do
-    const uint64_t tiles = (uint64_t)std::max(pl.total_tiles, 1), per_face = pl.total_f / tiles + 1;
-    uint64_t want_cap = std::min<uint64_t>(8 * per_face, std::max<uint64_t>(512, 2 * per_face));
-    want_cap = std::max<uint64_t>(want_cap, tiles > (1u << 20) ? 16 : 64) + CHUNK_SLACK;
-    if (pl.counted) want_cap = 32;   // a tile's range of the bins
+    // chunk descriptors (by counting a tile's only chunk is its range of the bins)
+    const uint64_t tiles = (uint64_t)std::max(pl.total_tiles, 1);
+    const uint64_t want_cap = pl.counted ? 32 : tile_places(pl.total_f, tiles);
     uint64_t want_slots = tiles * want_cap;
     if (want_slots > A.chunk_slots) {
         if ((r = ensure(c, A.chunks, sizeof(uint2) * want_slots))) return r;
@@ -729,7 +724,7 @@ int check_status(hana_ctx* c) {
         }
         uint32_t cap = flags & FLAG_CAPACITY;
         if (cap)
-            for (int k = 0; k < c->nslots; k++)
+            for (int k = 0; k < (c->pipelined ? c->nslots : 1); k++)
                 if ((r = grow_arena(c, slot_arena(c, k), need))) {
                     forget();
                     return r;

@@ -89,13 +89,18 @@ namespace {
 
 // Device footprint charged to a request: its targets and the per-pass
 // workspace (per vertex: position, varyings, outcode; per face: bins, clip
-// queue and pool).
+// queue and pool; per tile: chunk descriptors and two sets of counters; the list
+// of wide triangles).
 int64_t request_bytes(const hana_request& r, int sw, int sh) {
     int64_t V = r.mesh->V, F = r.mesh->F;
     int passes = r.enable_shadow ? 2 : 1;
     int64_t b = px_bucket((int64_t)r.width * r.height) * 8;
     if (r.enable_shadow) b += px_bucket((int64_t)sw * sh) * 8;
     b += passes * (V * 56 + F * 84);
+    auto tiles_of = [](int w, int h) { return ((int64_t)(w + 15) / 16) * ((h + 15) / 16); };
+    int64_t tiles = tiles_of(r.width, r.height);
+    if (r.enable_shadow) tiles += tiles_of(sw, sh);
+    b += tiles * (8 * (int64_t)tile_places(passes * F, tiles) + 8) + passes * 8 * (int64_t)WIDE_MAX;
     return b;
 }
 

@@ -344,3 +344,23 @@ def test_batch_of_many_wide_triangles_renders_every_time():
             c, d = ctx.read(t, 640, 480)
             assert d.tobytes() == dep.tobytes() and np.array_equal(c, col), k
         batch.close()
+
+
+@pytest.mark.parametrize("wh,shadow_wh,faces", [((1920, 1080), None, 5000), ((640, 480), (1024, 1024), 200_000)])
+def test_server_budget_counts_the_workspace(wh, shadow_wh, faces):
+    """A request is charged for its targets, its vertices' and faces' arrays and
+    the tiles' chunk descriptors (8 bytes each)."""
+    from hana_amd.gpu import Context, Server
+    s = soup_scene(faces, *wh, 2, 30, 4)
+    maps = [wh] + ([shadow_wh] if shadow_wh else [])
+    tiles = sum(-(-w // 16) * -(-h // 16) for w, h in maps)
+    per_tile = max(min(8 * (len(maps) * faces // tiles + 1), 512), 64) + 16
+    least = sum(8 * w * h for w, h in maps) + len(maps) * (3 * faces * 49 + faces * 70) + tiles * 8 * per_tile
+    with Context(0) as ctx:
+        server = Server(ctx, lanes=1)
+        server.submit(ctx.mesh(s.mesh), s.shader, shadow_wh is not None, *wh, s.cam_pos, s.light_pos, ctx.texture(s.diffuse),
+                      ctx.texture(s.normal), shadow_wh=shadow_wh or (0, 0))
+        res = collect(server, 1)
+        st = server.stats()
+        server.close()
+    assert res[0][0] == 0 and least <= st["peak_inflight_bytes"] < 2 * least
