@@ -1063,9 +1063,10 @@ struct Counted {
 // Whether the chunked binning whose counters are given ran out of descriptors
 // or bins, and of nothing else.
 __device__ __forceinline__ bool chunks_ran_out(const uint32_t* seq, uint32_t region, const Workspace& ws) {
-    const uint64_t pairs = ((uint64_t)seq[SEQ_PAIRS] | ((uint64_t)seq[SEQ_PAIRS + 1] << 32)) + region;
+    const uint64_t shared = (uint64_t)seq[SEQ_PAIRS] | ((uint64_t)seq[SEQ_PAIRS + 1] << 32);
     const uint64_t wide = (uint64_t)seq[SEQ_WIDE_PAIRS] | ((uint64_t)seq[SEQ_WIDE_PAIRS + 1] << 32);
-    return !(seq[SEQ_FLAGS] & FLAG_NO_RASTER) && pairs + wide <= MAX_PAIRS && (pairs > ws.bin_cap || seq[SEQ_MAX_CHUNKS]);
+    const uint32_t f = sequence_flags(shared, region, wide, ws.bin_cap);
+    return !((seq[SEQ_FLAGS] & FLAG_NO_RASTER) || (f & FLAG_PAIR_LIMIT)) && (f || seq[SEQ_MAX_CHUNKS]);
 }
 __device__ __forceinline__ bool counted_runs(const Workspace& ws, const Counted& q) {
     if (q.place) return ws.seq[SEQ_COUNTED] != 0u;
@@ -1379,20 +1380,19 @@ __global__ __launch_bounds__(BLOCK) void k_front(FrontTables tables, PassDesc* _
 __device__ __forceinline__ bool sequence_fits(const Workspace& ws, bool publish) {
     typedef uint32_t u8_vec __attribute__((ext_vector_type(8)));
     u8_vec q = *(const HANA_CONST_AS u8_vec*)ws.seq;
-    uint64_t pairs = ((uint64_t)q[SEQ_PAIRS] | ((uint64_t)q[SEQ_PAIRS + 1] << 32)) + ws.seg_region;
-    uint64_t wide = (uint64_t)q[SEQ_WIDE_PAIRS] | ((uint64_t)q[SEQ_WIDE_PAIRS + 1] << 32);
-    uint32_t f = q[SEQ_FLAGS];
-    if (pairs + wide > MAX_PAIRS) {
-        f |= FLAG_PAIR_LIMIT;
-    } else {
-        if (pairs > ws.bin_cap) f |= FLAG_BIN_OVERFLOW;
-        if (q[SEQ_MAX_CHUNKS]) f |= FLAG_CHUNK_OVERFLOW;
-    }
+    const uint64_t shared = (uint64_t)q[SEQ_PAIRS] | ((uint64_t)q[SEQ_PAIRS + 1] << 32);
+    const uint64_t wide = (uint64_t)q[SEQ_WIDE_PAIRS] | ((uint64_t)q[SEQ_WIDE_PAIRS + 1] << 32);
+    const uint32_t limits = sequence_flags(shared, ws.seg_region, wide, ws.bin_cap);
+    uint32_t f = q[SEQ_FLAGS] | limits;
+    if (q[SEQ_MAX_CHUNKS] && !(f & FLAG_PAIR_LIMIT)) f |= FLAG_CHUNK_OVERFLOW;
     if (publish) {
         if (!(f & FLAG_PAIR_LIMIT)) {
-            atomicMax(&ws.status[STATUS_NEED_BINS], (uint32_t)pairs);
+            const uint64_t pairs = shared + ws.seg_region;
+            atomicMax(&ws.status[STATUS_NEED_BINS], pairs < MAX_PAIRS ? (uint32_t)pairs : MAX_PAIRS);
             if (f & FLAG_CHUNK_OVERFLOW) {
+                // (more than any workspace grows to where no number of them would do)
                 uint64_t slots = ((uint64_t)q[SEQ_MAX_CHUNKS] + CHUNK_SLACK) * ws.q_items >> 10;
+                if (limits & FLAG_CHUNK_OVERFLOW) slots = 0xFFFFFFFFu;
                 atomicMax(&ws.status[STATUS_NEED_CHUNKS], (uint32_t)(slots < 0xFFFFFFFFu ? slots + 1u : slots));
                 atomicMax(&ws.status[STATUS_OVER_FACES], ~ws.faces);
                 atomicMax(&ws.status[STATUS_OVER_TILES], ~ws.q_items);

@@ -227,6 +227,8 @@ int build_plan(hana_ctx* c, std::vector<PassSpec> specs, Plan& pl, const Tuning&
     }
     pl.vblocks = vb;
     pl.fblocks = fb;
+    // more faces than leave the set-up workgroups bin positions of their own
+    if (!pl.front && (uint64_t)fb * SEG_PAIRS * BLOCK * FPT + 4096 > MAX_PAIRS) pl.counted = true;
     pl.total_v = voff;
     pl.total_vs = vsoff;
     pl.total_f = fo;
@@ -340,7 +342,7 @@ int bind_plan(hana_ctx* c, Plan& pl, Arena& A, uint32_t min_bins, uint32_t min_p
     const uint64_t seg_region = pl.counted ? 0 : (uint64_t)pl.fblocks * SEG_PAIRS * BLOCK * (pl.front ? FRONT_FPT : FPT);
     uint64_t want_bins = std::max<uint64_t>({(uint64_t)min_bins, (uint64_t)4 * pl.total_f + 2 * nt, 1u << 22,
                                              seg_region + (uint64_t)pl.total_f + 4096});
-    if (seg_region + 4096 > MAX_PAIRS) return fail(c, HANA_E_NOMEM, "launch sequence too large (triangle list)");
+    if ((uint64_t)pl.fblocks * BLOCK * FPT + 4096 > MAX_PAIRS) return fail(c, HANA_E_NOMEM, "launch sequence too large (faces)");
     want_bins = std::min<uint64_t>(want_bins, MAX_PAIRS);
     if (want_bins > A.bin_cap) {
         if ((r = ensure(c, A.bins, sizeof(uint32_t) * want_bins))) return r;
@@ -608,7 +610,7 @@ static int grow_chunks(hana_ctx* c, Arena& A, const Needs& need) {
 static int grow_arena(hana_ctx* c, Arena& A, const Needs& need) {
     const uint32_t flags = need.w[STATUS_FLAGS], need_bins = need.w[STATUS_NEED_BINS],
                    need_polys = need.w[STATUS_NEED_POLYS];
-    if (flags & FLAG_BIN_OVERFLOW) {
+    if ((flags & FLAG_BIN_OVERFLOW) && (!(flags & FLAG_CHUNK_OVERFLOW) || chunks_grow(need))) {
         uint64_t want = std::max<uint64_t>((uint64_t)need_bins + need_bins / 4 + 1024, A.bin_cap);
         want = std::min<uint64_t>(want, MAX_PAIRS);
         int r = ensure(c, A.bins, sizeof(uint32_t) * want);
@@ -1754,14 +1756,19 @@ static int batch_size_part(hana_ctx* c, hana_batch* b, hana_batch_part& part) {
                                              "(triangle, tile) pairs; split the batch");
             return HANA_OK;   // a polygon over POLY_MAX vertices is dropped at every run, like a per-call draw
         }
-        min_bins = std::max(min_bins, st[STATUS_NEED_BINS] + st[STATUS_NEED_BINS] / 8 + 1024);
+        const uint64_t need_bins = (uint64_t)st[STATUS_NEED_BINS] + st[STATUS_NEED_BINS] / 8 + 1024;
+        min_bins = std::max(min_bins, (uint32_t)std::min<uint64_t>(need_bins, MAX_PAIRS));
         min_polys = st[STATUS_NEED_POLYS] + st[STATUS_NEED_POLYS] / 8 + 1024;
         Needs need;
         need.take(st);
         // as in check_status: by counting where the descriptors do not grow that
         // far, or when growing them was not enough
-        if (attempt >= 2 || ((st[STATUS_FLAGS] & FLAG_CHUNK_OVERFLOW) && !chunks_grow(need))) counted = true;
-        else if ((st[STATUS_FLAGS] & FLAG_CHUNK_OVERFLOW) && (r = grow_chunks(c, A, need))) return r;
+        if (!counted && (attempt >= 2 || ((st[STATUS_FLAGS] & FLAG_CHUNK_OVERFLOW) && !chunks_grow(need)))) {
+            counted = true;
+            min_bins = 0;   // its own run will tell
+        } else if ((st[STATUS_FLAGS] & FLAG_CHUNK_OVERFLOW) && (r = grow_chunks(c, A, need))) {
+            return r;
+        }
     }
     return fail(c, HANA_E_OVERFLOW, "hana_batch_finalize: capacity not reached");
 }

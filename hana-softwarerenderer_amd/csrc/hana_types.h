@@ -3,6 +3,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "hana_limits.h"
+
 namespace hana {
 
 enum {
@@ -217,16 +219,6 @@ enum { SEQ_POLYS = 0, SEQ_CLIPQ = 1, SEQ_FLAGS = 2, SEQ_MAX_CHUNKS = 3, SEQ_PAIR
 // descriptors.
 enum { STATUS_FLAGS = 0, STATUS_NEED_BINS = 1, STATUS_NEED_POLYS = 2, STATUS_NEED_CHUNKS = 3, STATUS_OVER_FACES = 4,
        STATUS_OVER_TILES = 5, STATUS_WORDS = 6 };
-enum { FLAG_BIN_OVERFLOW = 1, FLAG_POLY_OVERFLOW = 2, FLAG_POLY_TOO_LARGE = 4, FLAG_CLIPQ_OVERFLOW = 8,
-       FLAG_CHUNK_OVERFLOW = 16, FLAG_PAIR_LIMIT = 32, FLAG_QUEUE_STALL = 64 };
-// A workspace capacity ran out: the sequence is incomplete, its rasters write
-// nothing, and the host grows the workspace and renders it again.
-constexpr uint32_t FLAG_CAPACITY = FLAG_BIN_OVERFLOW | FLAG_POLY_OVERFLOW | FLAG_CLIPQ_OVERFLOW | FLAG_CHUNK_OVERFLOW;
-// Flags of a sequence whose rasters do nothing.
-constexpr uint32_t FLAG_NO_RASTER = FLAG_CAPACITY | FLAG_PAIR_LIMIT;
-// (triangle, tile) pairs one launch sequence may hold: bin positions are
-// 32-bit.  A sequence with more sets FLAG_PAIR_LIMIT and rasterises nothing.
-constexpr uint32_t MAX_PAIRS = 0xFFFFFFF0u;
 // vertex outcode bits
 constexpr uint32_t CODE_VISIBLE = 0x80u;
 constexpr uint32_t CODE_PLANES = 0x7Fu;
