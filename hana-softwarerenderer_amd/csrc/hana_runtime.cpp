@@ -1397,15 +1397,16 @@ static int read_planes(hana_ctx* c, hana_target* t, const ReadBack* b, int count
         const int bands = (int)((n + band - 1) / band);
         uint32_t* flags = reinterpret_cast<uint32_t*>(c->stage_host + c->stage_cap);
         uint32_t* flags_dev = reinterpret_cast<uint32_t*>(c->stage_dev + c->stage_cap);
-        // 16-byte aligned planes; a second one that this leaves no room for follows by itself
+        // 16-byte aligned planes: the staging is a power of two of at least 4096
+        // bytes, so that where two planes fit, so do two rounded up
         const size_t pitch = (4 * n + 15) & ~(size_t)15;
-        const int planes = pitch * count <= c->stage_cap ? count : 1;
-        for (int i = 0; i < planes; i++)
+        if (pitch * count > c->stage_cap) return fail(c, HANA_E_DEVICE, "internal error: planes larger than their staging");
+        for (int i = 0; i < count; i++)
             HIP_TRY(c, launch_read_back(static_cast<const uint32_t*>(b[i].src), reinterpret_cast<uint32_t*>(c->stage_dev + i * pitch),
                                         t->w, t->h, b[i].flip, band, c->stage_count.as<uint32_t>() + i * READ_BANDS,
                                         flags_dev + i * READ_BANDS, c->stage_epoch, c->stream));
         bool again = false;
-        for (int i = 0; i < planes && !again; i++)
+        for (int i = 0; i < count && !again; i++)
             for (int k = 0; k < bands; k++) {
                 if (bands == 1) {
                     if (i == 0) HIP_TRY(c, hipStreamSynchronize(c->stream));
@@ -1428,7 +1429,6 @@ static int read_planes(hana_ctx* c, hana_target* t, const ReadBack* b, int count
             continue;
         }
         HIP_TRY(c, hipStreamSynchronize(c->stream));
-        if (planes < count && (r = read_pieces(c, b[1].dst, b[1].src, 4 * n))) return r;
         return checked ? st : check_status(c);
     }
     for (int i = 0; i < count; i++) {
