@@ -223,14 +223,20 @@ TRAFFIC_FILES = {"c2": os.path.join(REPO, "profiles", "traffic_large_frame.json"
                  "c5": os.path.join(REPO, "profiles", "traffic_micro.json")}
 
 
-def measured(section, stage, field):
+TUNING_FIELDS = ("tile_size", "raster_wgs_per_cu", "parts", "raster_waves")
+
+
+def measured(section, stage, field, tuning=None):
     """A per-launch figure of a stage from the committed counter summary of
-    the workload (rocprofv3 --pmc), or None."""
+    the workload (rocprofv3 --pmc), or None; of a batch, only if it was counted
+    with the same tuning."""
     f = TRAFFIC_FILES.get(section)
     if not f or not os.path.exists(f):
         return None
-    per = json.load(open(f)).get("per_launch", {})
-    v = per.get(stage)
+    summary = json.load(open(f))
+    if tuning is not None and summary.get("tuning") != [tuning[k] for k in TUNING_FIELDS]:
+        return None
+    v = summary.get("per_launch", {}).get(stage)
     if not v:
         return None
     if field == "traffic":
@@ -238,15 +244,17 @@ def measured(section, stage, field):
     return int(v[field]) if field in v else None
 
 
-def roofline(section, stage_ms, launches, stage_bytes):
+def roofline(section, stage_ms, launches, stage_bytes, tuning=None):
     """The dominant stage against the HBM peak: algorithmic bytes per launch
-    over its mean launch time (HIP events on the stream it runs on)."""
+    over its mean launch time (HIP events on the stream it runs on).  Counted
+    traffic and instructions stand beside it where they were counted with the
+    same tuning."""
     stage = max(stage_ms, key=lambda k: stage_ms[k])
     n = max(launches.get(stage, 1), 1)
     per_launch_ms = stage_ms[stage] / n
     nbytes = stage_bytes.get(stage, 0) / n
     gbps = nbytes / (per_launch_ms * 1e-3) / 1e9 if per_launch_ms > 0 else 0.0
-    tr = measured(section, stage, "traffic")
+    tr = measured(section, stage, "traffic", tuning)
     out = {"bound": "hbm", "kernel": stage, "achieved": round(gbps, 2), "peak": HBM_PEAK_GBPS, "unit": "GB/s",
            "frac": round(gbps / HBM_PEAK_GBPS, 5), "bytes_per_launch": int(nbytes), "traffic": tr,
            "traffic_source": (os.path.relpath(TRAFFIC_FILES[section], REPO) + ": rocprofv3 --pmc FETCH_SIZE and "
@@ -254,7 +262,7 @@ def roofline(section, stage_ms, launches, stage_bytes):
            "launch_us": round(per_launch_ms * 1e3, 2), "launches_per_step": n,
            "time_source": "HIP events recorded around each launch on the library's stream (stage timing on: "
                           "launches not overlapped)"}
-    valu = measured(section, stage, "valu_instr")
+    valu = measured(section, stage, "valu_instr", tuning)
     if valu is not None and per_launch_ms > 0:
         rate = valu / (per_launch_ms * 1e-3)
         out["valu"] = {"wave_instr_per_launch": valu, "achieved": round(rate / 1e9, 2),
@@ -519,7 +527,7 @@ def bench_c3(ctx, args, scenes, cpu):
            "speedup_vs_per_call": round(t_call / t_batch, 2) if t_call else None,
            "stage_ms": {k: round(v, 5) for k, v in stage_ms.items()},
            "batch_alg_bytes": batch_bytes, "batch_achieved_GBps": round(batch_bytes / t_batch / 1e9, 2),
-           "roofline": roofline("c3", stage_ms, launches, stage_bytes), "parity": parity}
+           "roofline": roofline("c3", stage_ms, launches, stage_bytes, chosen), "parity": parity}
     if sweep:
         out["tuning_sweep"] = sweep
     if frags:
@@ -688,7 +696,7 @@ def _counters(d):
     return tot, disp
 
 
-def summarize_counters(workload, d, out_json):
+def summarize_counters(workload, d, out_json, tuning=None):
     """Per-launch HBM bytes (FETCH_SIZE, WRITE_SIZE scaled by a plain copy's
     readings) and SQ counters, by stage; writes OUT_JSON, prints markdown."""
     copy_bytes = 64 * 1024 * 1024 * 4
@@ -711,6 +719,8 @@ def summarize_counters(workload, d, out_json):
             for c, v in cs.items():
                 e[c] = v / n
     out = {"workload": workload, "fetch_scale": fs, "write_scale": ws_, "per_launch": {}}
+    if tuning:
+        out["tuning"] = [int(x) for x in tuning.split(",")]
     for st, e in per.items():
         o = {}
         if "FETCH_SIZE" in e:
@@ -799,9 +809,10 @@ def main():
     ap.add_argument("--no-fp32", action="store_true", help="skip the fp32 shadow-map variants of c2 and c5")
     ap.add_argument("--copy-calibration", action="store_true",
                     help="only run a plain 256 MiB device-to-device copy (scales rocprof FETCH/WRITE_SIZE)")
-    ap.add_argument("--summarize-counters", nargs=3, metavar=("WORKLOAD", "DIR", "OUT_JSON"),
+    ap.add_argument("--summarize-counters", nargs="+", metavar="WORKLOAD DIR OUT_JSON [TUNING]",
                     help="summarise rocprofv3 --pmc runs under DIR (subfolders pmc_* and the copy calibration "
-                         "cal_fetch, cal_write) into per-launch figures by stage; prints a markdown table")
+                         "cal_fetch, cal_write) into per-launch figures by stage, of a batch with the --tuning it "
+                         "ran with; prints a markdown table")
     ap.add_argument("--summarize-trace", nargs="+", metavar="DIR [LAST]",
                     help="print the rocprofv3 --stats kernel summary under DIR as a markdown table, and with LAST "
                          "each kernel's mean over its last LAST dispatches")
