@@ -163,8 +163,7 @@ constexpr size_t kHugeSequenceFaces = size_t(1) << 24;
 // launch sequences of at most this many faces run their geometry in one launch
 // (k_front).  Beyond, shading every vertex about six times costs more than the
 // launches: a 400,000-face frame with its shadow pass 81 us a frame in three
-// launches, 85 in one; a batch of 64 scenes, of whose four parts one is below
-// the limit, 424 us, 440 with the limit at 2^17
+// launches, 85 in one
 #ifndef HANA_FRONT_FACES
 #define HANA_FRONT_FACES (1 << 18)
 #endif

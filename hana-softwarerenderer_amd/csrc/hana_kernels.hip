@@ -135,7 +135,8 @@ constexpr uint32_t FACE_MASK = FACE_FAST - 1u;
 // A triangle of e x e px then scans about e^2 pixels instead of (e + 1)^2, and
 // one between two columns none: the shadow and main rasters of 20 M
 // micro-triangles at 3840x2160 went from 1495 and 756 us to 948 and 555, those
-// of a 1.3 M-triangle 1920x1080 frame from 60 and 46 us to 50 and 40.
+// of a 1.3 M-triangle 1920x1080 frame from 60 and 46 us to 50 and 40 (reading
+// bins of one range per tile; with chunks they take 1090 and 637, 59 and 48).
 // (Testing the coverage of the triangles with at most 1, 2 or 3 candidates
 // left in set-up and dropping the uncovered ones as well took as much time
 // there as it saved here.)
@@ -656,7 +657,7 @@ __device__ __forceinline__ void seg_sums(SegLds<BITS, THREADS, CAP>& L, SegSums&
 //    fits -- a workgroup's faces follow one another in the mesh and mostly lie
 //    close together --, else the distinct tiles by a hash, whose probes are a
 //    chain of LDS accesses.  There one workgroup's chain is the launch's time
-//    (thumbnail, 300x300 with 1,160 faces: 15.4 -> 13.3 us a frame).  Where
+//    (128x128 with 192 faces: 15.4 -> 13.3 us a frame).  Where
 //    workgroups fill the chip it is the instructions that count, and the plain
 //    loop is faster (460,800 faces at 1080p: set-up 28.7 us against 32.8).
 //  - The pairs go to the workgroup's own entries of the bins, [own, own_end),

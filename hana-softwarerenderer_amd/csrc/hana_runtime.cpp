@@ -136,7 +136,7 @@ int materialize_clear(hana_ctx* c, hana_target* t, hipStream_t s) {
 // raster group, and within the main group those that sample a shadow map
 // drawn by the first group come last: the persistent raster's queue holds the
 // tiles in pass order, so every shadow tile precedes the tiles that wait for
-// them.  Every per-pass slice is 1024-vertex aligned.
+// them.  Every per-pass slice is aligned to the vertices of a workgroup.
 int build_plan(hana_ctx* c, std::vector<PassSpec> specs, Plan& pl, const Tuning& tu, size_t front_faces, bool counted) {
     {
         std::vector<std::pair<int, size_t>> key(specs.size());
