@@ -324,6 +324,13 @@ static void counters_launched(Arena& A) {
     A.counters_next ^= 1;
 }
 
+// An arena's chunk descriptors; without memory for them it has none.
+static int ensure_chunks(hana_ctx* c, Arena& A, uint64_t slots) {
+    int r = ensure(c, A.chunks, sizeof(uint2) * slots);
+    A.chunk_slots = r ? A.chunks.cap / sizeof(uint2) : std::max(slots, A.chunk_slots);
+    return r;
+}
+
 // Allocates the arena for a plan and resolves the slice pointers.
 int bind_plan(hana_ctx* c, Plan& pl, Arena& A, uint32_t min_bins, uint32_t min_polys, bool with_stats,
               hipStream_t s) {
@@ -352,10 +359,7 @@ int bind_plan(hana_ctx* c, Plan& pl, Arena& A, uint32_t min_bins, uint32_t min_p
     const uint64_t tiles = (uint64_t)std::max(pl.total_tiles, 1);
     const uint64_t want_cap = pl.counted ? 32 : tile_places(pl.total_f, tiles);
     uint64_t want_slots = tiles * want_cap;
-    if (want_slots > A.chunk_slots) {
-        if ((r = ensure(c, A.chunks, sizeof(uint2) * want_slots))) return r;
-        A.chunk_slots = want_slots;
-    }
+    if (want_slots > A.chunk_slots && (r = ensure_chunks(c, A, want_slots))) return r;
     if ((r = ensure(c, A.wide, sizeof(uint2) * WIDE_MAX * std::max(n, 1)))) return r;
     uint64_t want_polys = std::max<uint64_t>({(uint64_t)min_polys, pl.total_f / 16 + 4096});
     want_polys = std::min<uint64_t>(want_polys, POOL_CAP_MAX);
@@ -599,10 +603,12 @@ struct Needs {
 static uint64_t full_places(const Needs& need) { return (uint64_t)need.w[STATUS_NEED_CHUNKS] * 1024 / 4 * 5; }
 static bool chunks_grow(const Needs& need) { return full_places(need) <= kGrownChunks; }
 static int grow_chunks(hana_ctx* c, Arena& A, const Needs& need) {
-    const uint64_t want = std::max(full_places(need), A.chunk_slots);
-    int r = ensure(c, A.chunks, sizeof(uint2) * want);
-    if (!r) A.chunk_slots = want;
-    return r;
+    return ensure_chunks(c, A, std::max(full_places(need), A.chunk_slots));
+}
+// Sequences of the size of those that ran out of descriptors bin by counting from now on.
+static void count_such(hana_ctx* c, const Needs& need) {
+    c->counted_faces = std::min<size_t>(c->counted_faces, ~need.w[STATUS_OVER_FACES]);
+    c->counted_tiles = std::min<size_t>(c->counted_tiles, ~need.w[STATUS_OVER_TILES]);
 }
 
 // Grows an arena's bins, chunk descriptors and clip pool to the needs reported
@@ -617,9 +623,11 @@ static int grow_arena(hana_ctx* c, Arena& A, const Needs& need) {
         if (r) return r;
         A.bin_cap = (uint32_t)want;
     }
-    if ((flags & FLAG_CHUNK_OVERFLOW) && chunks_grow(need)) {
-        int r = grow_chunks(c, A, need);
-        if (r) return r;
+    if (flags & FLAG_CHUNK_OVERFLOW) {
+        // without memory for the places, too
+        int r = chunks_grow(need) ? grow_chunks(c, A, need) : HANA_E_NOMEM;
+        if (r == HANA_E_NOMEM) count_such(c, need);
+        else if (r) return r;
     }
     if (flags & FLAG_POLY_OVERFLOW) {
         uint64_t want = std::max<uint64_t>((uint64_t)need_polys + need_polys / 4 + 1024, A.poly_cap);
@@ -749,10 +757,6 @@ int check_status(hana_ctx* c) {
             return fail(c, HANA_E_OVERFLOW,
                         "a batch outgrew its workspace and left targets as they were, and a no-alloc frame followed it; "
                         "the workspace was grown, render both again");
-        }
-        if ((cap & FLAG_CHUNK_OVERFLOW) && !chunks_grow(need)) {
-            c->counted_faces = std::min<size_t>(c->counted_faces, ~need.w[STATUS_OVER_FACES]);
-            c->counted_tiles = std::min<size_t>(c->counted_tiles, ~need.w[STATUS_OVER_TILES]);
         }
         if ((rerun || (cap && c->replay_overflow)) && attempt < 4) {
             c->replays++;
@@ -1697,10 +1701,10 @@ static int batch_leave_room(hana_ctx* c, hana_batch_part& part, uint32_t* min_bi
             *counted = true;
             return HANA_OK;
         }
-        int r = ensure(c, A.chunks, sizeof(uint2) * slots);
-        if (r) return r;
-        A.chunk_slots = slots;
-        *grown = true;
+        const int r = ensure_chunks(c, A, slots);
+        if (r && r != HANA_E_NOMEM) return r;
+        *(r ? counted : grown) = true;
+        if (r) return HANA_OK;
     }
     if (pl.ws.seg_region + shared > pl.ws.bin_cap) {
         if (pl.ws.seg_region + shared > MAX_PAIRS) *counted = true;
@@ -1762,12 +1766,14 @@ static int batch_size_part(hana_ctx* c, hana_batch* b, hana_batch_part& part) {
         Needs need;
         need.take(st);
         // as in check_status: by counting where the descriptors do not grow that
-        // far, or when growing them was not enough
-        if (!counted && (attempt >= 2 || ((st[STATUS_FLAGS] & FLAG_CHUNK_OVERFLOW) && !chunks_grow(need)))) {
-            counted = true;
-            min_bins = 0;   // its own run will tell
-        } else if ((st[STATUS_FLAGS] & FLAG_CHUNK_OVERFLOW) && (r = grow_chunks(c, A, need))) {
-            return r;
+        // far or have no memory to, or when growing them was not enough
+        if (!counted && (attempt >= 2 || (st[STATUS_FLAGS] & FLAG_CHUNK_OVERFLOW))) {
+            r = attempt < 2 && chunks_grow(need) ? grow_chunks(c, A, need) : HANA_E_NOMEM;
+            if (r && r != HANA_E_NOMEM) return r;
+            if (r) {
+                counted = true;
+                min_bins = 0;   // its own run will tell
+            }
         }
     }
     return fail(c, HANA_E_OVERFLOW, "hana_batch_finalize: capacity not reached");

@@ -364,3 +364,32 @@ def test_server_budget_counts_the_workspace(wh, shadow_wh, faces):
         st = server.stats()
         server.close()
     assert res[0][0] == 0 and least <= st["peak_inflight_bytes"] < 2 * least
+
+
+def test_noalloc_frame_behind_a_batch_that_is_to_be_run_again():
+    """A frame without allocation cannot be drawn again behind the batch: the wait
+    says so, and the next run is right."""
+    from hana_amd.gpu import HANA_E_OVERFLOW, Batch, Context, HanaError, build_uniforms
+    scene = soup_scene(60_000, 2048, 1024, 2, 8, 91)
+    crowded = scene.mesh.pos.copy()
+    crowded[:, :2] *= np.float32(0.03)
+    with Context(0) as ctx:
+        u, tex = build_uniforms(scene), (ctx.texture(scene.diffuse), ctx.texture(scene.normal))
+        mesh, t, other = ctx.mesh(scene.mesh), ctx.target(2048, 1024), ctx.target(2048, 1024)
+        batch = Batch(ctx)
+        batch.add(ctx.frame_desc(mesh, scene.shader, False, u, t, None, *tex))
+        batch.finalize(use_graph=True)
+        move_vertices(ctx, mesh, crowded)
+        batch.run()
+        d = ctx.frame_desc(mesh, scene.shader, False, u, other, None, *tex)
+        ctx.check(ctx.lib.hana_render_frame_noalloc(ctx.h, C.byref(d)), "noalloc")
+        with pytest.raises(HanaError) as err:
+            ctx.sync()
+        assert err.value.code == HANA_E_OVERFLOW and "no-alloc" in str(err.value)
+        ctx.clear(other)
+        ctx.draw(mesh, scene.shader, u, other, *tex)
+        want = ctx.read(other, 2048, 1024)
+        batch.run()
+        got = ctx.read(t, 2048, 1024)
+        assert got[1].tobytes() == want[1].tobytes() and np.array_equal(got[0], want[0])
+        batch.close()
